@@ -110,16 +110,19 @@ int qcs_apply_gate(qcs_register* r, uint32_t k, uint32_t traits,
 int qcs_apply_dense(qcs_register* r, uint32_t k, const uint32_t* qubits,
                     const double* mat);
 
-/* A batch of gates in order; fuse_width 0/1 applies them one by one, 2..5
- * runs the fusion pass first (blocks of at most fuse_width qubits), and
- * QCS_FUSE_AUTO picks the width (0 or 2..5) whose blocks cost least under
- * the fusion cost table (qcs_autotune_fusion, measured on first use for
- * this precision and qubit count). No counterpart in the reference, which
- * applies gates one by one (QubitRegister.h:488-492). */
+/* A batch of gates in order, run in passes of many gates over the state
+ * whatever the width. fuse_width 0/1 takes the gates as they come (a refused
+ * gate ends the batch after those before it); with 2..5 a list that the
+ * fusion pass (qcs_fuse) refuses at that width is refused whole, and
+ * QCS_FUSE_AUTO also reports the width (0 or 2..5) whose blocks would cost
+ * least under the fusion cost table (qcs_autotune_fusion, measured on first
+ * use for this precision and qubit count). No counterpart in the reference,
+ * which applies gates one by one (QubitRegister.h:488-492). */
 #define QCS_FUSE_AUTO 0xFFFFFFFFu
 int qcs_apply_circuit(qcs_register* r, const qcs_gate* gates, uint32_t n,
                       uint32_t fuse_width);
-/* The width the last qcs_apply_circuit on r used (0: unfused). */
+/* The width of the last qcs_apply_circuit on r (0: none; QCS_FUSE_AUTO's
+ * choice). */
 uint32_t qcs_last_fuse_width(const qcs_register* r);
 
 /* The fusion pass alone (host only, no device): rewrites `gates` into at
@@ -132,11 +135,12 @@ int qcs_fuse(const qcs_gate* gates, uint32_t n, uint32_t width,
 
 /* Recorded-gate replay as one graph launch: replaces the gate-by-gate loops
    of QubitRegister::Compute / Uncompute (QubitRegister.h:553-590). A
-   program is compiled for one register: the sequence is fused to blocks of
-   <= fuse_width qubits (0: no fusion, else 2..5); with adjoint != 0 it is
-   the inverse sequence (gates reversed, matrices conjugate-transposed, as
-   Uncompute applies them); its matrices are uploaded once into memory the
-   program owns and its launches are captured into a hipGraph. qcs_program_run
+   program is compiled for one register: the sequence is cut into passes of
+   many gates as by qcs_apply_circuit (fuse_width 0, 2..5 or QCS_FUSE_AUTO);
+   with adjoint != 0 it is the inverse sequence (gates reversed, matrices
+   conjugate-transposed, as Uncompute applies them); its operations and
+   matrices are uploaded once into memory the program owns and its launches
+   are captured into a hipGraph. qcs_program_run
    replays the graph on the register's stream. */
 typedef struct qcs_program qcs_program;
 int qcs_program_create(qcs_register* r, const qcs_gate* gates, uint32_t n,

@@ -282,6 +282,12 @@ int rising(qcs_register* r, uint32_t ne, const uint32_t* ei, const uint32_t* ej,
 // qft.hip
 int qft(qcs_register* r, uint32_t sq, uint32_t eq, int do_swap, int inverse);
 
+// circuit.hip: a gate list in passes of many gates; the first gate its entry
+// point refuses ends it with that error.
+int run_gates(qcs_register* r, const qcs_gate* gates, uint32_t n);
+// Upper bound of the parameter bytes run_gates stages for one gate.
+size_t gates_param_bound(const qcs_register* r, const qcs_gate& g);
+
 // autotune.hip: the fused sequence of the cheapest fusion width
 int pick_fusion(qcs_register* r, const qcs_gate* gates, uint32_t n, std::vector<qcs_gate>& out, uint32_t* width);
 

@@ -26,7 +26,6 @@
 #include <algorithm>
 #include <complex>
 #include <cstring>
-#include <functional>
 #include <vector>
 
 #include "qcsim_amd.h"
@@ -218,11 +217,9 @@ static qcs_gate block_gate(const qcs_gate* gates, const Pending& P, const std::v
     return fg;
 }
 
-int fuse_stream(const qcs_gate* gates, uint32_t n, uint32_t width, const std::function<int(const qcs_gate&)>& emit) {
+// What the fusion pass asks of a gate list.
+int fuse_check(const qcs_gate* gates, uint32_t n, uint32_t width) {
     if (width < 1 || width > 5) return set_error(QCS_EINVAL, "fusion width must be 1..5");
-    Pending P;
-    P.mask.resize(n);
-    P.next.resize(n);
     for (uint32_t i = 0; i < n; ++i) {
         const qcs_gate& g = gates[i];
         if (g.k < 1 || g.k > 5) return set_error(QCS_EINVAL, "gate %u: arity must be 1..5", i);
@@ -232,7 +229,19 @@ int fuse_stream(const qcs_gate* gates, uint32_t n, uint32_t width, const std::fu
             gm |= 1ull << g.qubits[j];
         }
         if (popc(gm) != int(g.k)) return set_error(QCS_EINVAL, "gate %u: qubits must be different", i);
-        P.mask[i] = gm;
+    }
+    return QCS_OK;
+}
+
+int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate>& out) {
+    out.clear();
+    if (const int e = fuse_check(gates, n, width)) return e;
+    Pending P;
+    P.mask.resize(n);
+    P.next.resize(n);
+    for (uint32_t i = 0; i < n; ++i) {
+        P.mask[i] = 0;
+        for (uint32_t j = 0; j < gates[i].k; ++j) P.mask[i] |= 1ull << gates[i].qubits[j];
         P.next[i] = i + 1 < n ? int(i + 1) : -1;
     }
     P.head = n ? 0 : -1;
@@ -320,18 +329,9 @@ int fuse_stream(const qcs_gate* gates, uint32_t n, uint32_t width, const std::fu
                 prev = i;
             }
         }
-        // the block leaves (ascending indices) as one gate, at once
-        if (const int e = emit(block_gate(gates, P, take))) return e;
+        out.push_back(block_gate(gates, P, take));
     }
     return QCS_OK;
-}
-
-int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate>& out) {
-    out.clear();
-    return fuse_stream(gates, n, width, [&](const qcs_gate& g) {
-        out.push_back(g);
-        return QCS_OK;
-    });
 }
 
 }  // namespace qcs

@@ -3,14 +3,15 @@
 // The reference records gates between ComputeStart and ComputeEnd and
 // replays them with Compute, or in reverse with adjoint matrices with
 // Uncompute (QubitRegister.h:536-590). A program is such a sequence
-// compiled once for one register: optionally fused, its dense matrices
-// uploaded into memory the program owns, and its launches captured from
-// the register's stream into a hipGraph. Running it is one graph launch on
-// the same stream, so a sequence of small-state gates costs one launch
-// instead of one per gate. Programs hold only gate launches (no
-// reductions, measurements or host work) and no memset nodes; a program
-// whose register has since exchanged its state buffer (qcs_swap_state) is
-// captured again before it runs.
+// compiled once for one register: cut into passes of many gates
+// (circuit.hip), the passes' operations uploaded into memory the program
+// owns, and its launches captured from the register's stream into a
+// hipGraph. Running it is one graph launch on the same stream, so a sequence
+// of small-state gates costs a launch for some tens of gates instead of one
+// for each (600 gates on 16 qubits: 409 us against 1439). Programs hold only
+// gate launches (no reductions, measurements or host work) and no memset
+// nodes; a program whose register has since exchanged its state buffer
+// (qcs_swap_state) is captured again before it runs.
 #include <algorithm>
 #include <complex>
 #include <cstring>
@@ -19,8 +20,7 @@
 #include "common.h"
 
 namespace qcs {
-int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate>& out);
-int kdense(qcs_register* r, uint32_t k, const uint32_t* qubits, const double* mat_host);
+int fuse_check(const qcs_gate* gates, uint32_t n, uint32_t width);
 
 // The inverse of a gate: conjugate transpose of its matrix; the phase of
 // the iSWAP kernels flips (their matrix is implied by the trait).
@@ -38,24 +38,13 @@ static qcs_gate adjoint_gate(const qcs_gate& g) {
     if (isd) a.traits |= QCS_TRAIT_ISWAP;
     return a;
 }
-// Upper bound of the parameter bytes one block's launch stages (each
-// staging is rounded up to 256 B): a dense block takes at most one staging
-// slot; a generic 2- or 3-qubit gate may run k_nq_split, which stages its
-// matrix as D*D real parts then D*D imaginary parts; every other launch
-// passes its parameters as kernel arguments.
-static size_t param_bound(const qcs_register* r, const qcs_gate& g) {
-    if ((g.flags & QCS_GATE_DENSE) || g.k > 3) return (r->mat_bytes + 255) & ~size_t(255);
-    if (g.k < 2) return 0;
-    const size_t D = size_t(1) << g.k;
-    return (2 * D * D * sizeof(double) + 255) & ~size_t(255);
-}
 }  // namespace qcs
 
 using namespace qcs;
 
 struct qcs_program {
     qcs_register* r = nullptr;
-    std::vector<qcs_gate> blocks;  // the (fused) sequence, kept for re-capture
+    std::vector<qcs_gate> gates;  // the sequence, kept for re-capture
     size_t param_bytes = 0;        // upper bound of what the launches stage
     void* psi = nullptr;  // state buffer the graph was captured for
     hipGraph_t graph = nullptr;
@@ -64,8 +53,8 @@ struct qcs_program {
     uint32_t launches = 0;
 };
 
-// Captures p->blocks on p->r's stream into a new graph (dropping any older
-// one) and uploads the dense matrices the launches read.
+// Captures p->gates on p->r's stream into a new graph (dropping any older
+// one) and uploads the operations and matrices the launches read.
 static int capture(qcs_program* p) {
     qcs_register* r = p->r;
     if (p->exec) (void)hipGraphExecDestroy(p->exec);
@@ -86,13 +75,7 @@ static int capture(qcs_program* p) {
         return set_error(QCS_EDEVICE, "stream capture failed");
     r->sink = &sink;
     const uint64_t l0 = r->launches;
-    int e = QCS_OK;
-    for (size_t i = 0; i < p->blocks.size() && !e; ++i) {
-        const qcs_gate& g = p->blocks[i];
-        e = (g.flags & QCS_GATE_DENSE) || g.k > 3
-                ? kdense(r, g.k, g.qubits, g.mat)
-                : qcs_apply_gate(r, g.k, g.traits, g.qubits[0], g.qubits[1], g.qubits[2], g.mat);
-    }
+    const int e = run_gates(r, p->gates.data(), uint32_t(p->gates.size()));
     r->sink = nullptr;
     p->launches = uint32_t(r->launches - l0);
     r->launches = l0;
@@ -139,17 +122,17 @@ int qcs_program_create(qcs_register* r, const qcs_gate* gates, uint32_t n, uint3
     auto* p = new qcs_program;
     p->r = r;
     if (fuse_width >= 2) {
-        uint32_t picked = fuse_width;
-        const int e = fuse_width == QCS_FUSE_AUTO ? pick_fusion(r, seq.data(), uint32_t(seq.size()), p->blocks, &picked)
-                                                  : fuse(seq.data(), uint32_t(seq.size()), fuse_width, p->blocks);
+        std::vector<qcs_gate> fused;
+        uint32_t picked = 0;
+        const int e = fuse_width == QCS_FUSE_AUTO ? pick_fusion(r, seq.data(), uint32_t(seq.size()), fused, &picked)
+                                                  : fuse_check(seq.data(), uint32_t(seq.size()), fuse_width);
         if (e) {
             delete p;
             return e;
         }
-    } else {
-        p->blocks.swap(seq);
     }
-    for (const auto& g : p->blocks) p->param_bytes += param_bound(r, g);
+    p->gates.swap(seq);
+    for (const auto& g : p->gates) p->param_bytes += gates_param_bound(r, g);
     if (const int e = capture(p)) {
         qcs_program_destroy(p);
         return e;
