@@ -136,7 +136,7 @@ int qcs_create(uint32_t nqubits, int precision, qcs_register** out) {
         (void)hipGetLastError();
         return fail(QCS_ENOMEM, "hipMalloc of scratch failed");
     }
-    if (hipHostMalloc(reinterpret_cast<void**>(&r->hpin), sizeof(double) * 64) != hipSuccess ||
+    if (hipHostMalloc(reinterpret_cast<void**>(&r->hpin), sizeof(double) * kPauliResults) != hipSuccess ||
         hipHostMalloc(&r->hmat, r->mat_bytes * qcs_register::kMatSlots) != hipSuccess)
         return fail(QCS_ENOMEM, "hipHostMalloc failed");
     if (hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking) != hipSuccess ||

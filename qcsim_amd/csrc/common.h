@@ -199,14 +199,18 @@ namespace qcs {
 constexpr uint64_t kMaxBlocks = 1ull << 22;
 constexpr int kRedBlocks = 4096;     // fixed grid of reductions (deterministic)
 constexpr int kRedThreads = 256;
-// Pauli-string expectations: at most kPauliTerms terms per pass, partials
-// of at most kPauliBlocks blocks.
+// Pauli-string expectations: at most kPauliTerms terms of a wide x mask per
+// pass, with partials of at most kPauliBlocks blocks; of the terms of tile
+// passes at most kPauliResults at a time, with partials of 256 blocks.
 constexpr int kPauliTerms = 16;
 constexpr int kPauliBlocks = 2048;
+constexpr int kPauliResults = 128;
 // reduction scratch per register: kRedBlocks * 3 partials, or the Pauli
-// partials, then 64 result slots
-constexpr int kRedDoubles = (kRedBlocks * 3 > kPauliTerms * kPauliBlocks ? kRedBlocks * 3 : kPauliTerms * kPauliBlocks) + 64;
-constexpr int kRedResult = kRedDoubles - 64;  // first result slot
+// partials, then the result slots
+constexpr int kRedDoubles =
+    (kRedBlocks * 3 > kPauliTerms * kPauliBlocks ? kRedBlocks * 3 : kPauliTerms * kPauliBlocks) + kPauliResults;
+static_assert(kPauliResults * 256 <= kRedDoubles - kPauliResults, "partials of a batch of Pauli terms");
+constexpr int kRedResult = kRedDoubles - kPauliResults;  // first result slot
 constexpr size_t kXferBytes = size_t(64) << 20;
 constexpr uint32_t kChunkLog = 11;   // CDF chunk = 2048 amplitudes
 constexpr int kScanThreads = 256;

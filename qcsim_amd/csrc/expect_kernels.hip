@@ -8,15 +8,17 @@
 // The reference measures such a string after a basis change and averages
 // 10000 sampled parities (VQE.h:116-142, with the change of basis at
 // :33-44); it leaves this exact form as a TODO (QubitRegister.h:649). Here
-// the terms that share one x mask are evaluated in one read-only pass:
+// they are evaluated in read-only passes over the state:
 //   x = 0:  <P> = sum_s |psi_s|^2 sigma(s), sigma(s) = (-1)^{popcount(s & z)}
-//   x != 0: the pair (s, t = s ^ x) with bit h = msb(x) of s clear adds
-//           sigma(s) (kappa a + conj a), a = conj(psi_s) psi_t and
-//           kappa = (-1)^{ny}, since sigma(t) = kappa sigma(s); so each term
-//           sums sigma(s) Re a (ny even) or sigma(s) Im a (ny odd), and
-//           <P> = 2 (-1)^{ny/2} S (even) or 2 (-1)^{(ny-1)/2} S (odd).
-// Each amplitude is read once per x mask; all sums are FP64 with a fixed
-// grid and a fixed combination order.
+//   x != 0: a pair (s, t = s ^ x) adds sigma(s) (kappa a + conj a),
+//           a = conj(psi_s) psi_t and kappa = (-1)^{ny}, since
+//           sigma(t) = kappa sigma(s); so each term sums sigma(s) Re a (ny
+//           even) or sigma(s) Im a (ny odd) over the pairs, whichever of the
+//           two stands for s, and <P> = 2 (-1)^{ny/2} S (even) or
+//           2 (-1)^{(ny-1)/2} S (odd).
+// A pass takes every term whose x mask lies in its tile (k_pauli_tile); a
+// mask too wide for a tile has one of its own (k_pauli). All sums are FP64
+// with a fixed grid and a fixed combination order.
 #include <algorithm>
 #include <map>
 #include <vector>
@@ -40,48 +42,34 @@ struct PauliFlip {
     uint64_t z[kPauliTerms];
 };
 
-// One pass for the terms j < nt that share x (PAIR: x != 0, whose highest
-// bit is hbit). The grid stride is a power of two, so an index splits into
-// disjoint bit sets: s = s_thread | s_iter, s_thread from the work-item's
-// index and s_iter from the iteration alone (insert_run maps disjoint bit
-// sets to disjoint bit sets). Hence sigma_j(s) = sigma_j(s_thread)
-// sigma_j(s_iter): the second factor is the same for the whole wave, kept as
-// the high word of a double +-1.0 on the scalar unit and updated with one XOR
-// per term and iteration along the Gray walk; the vector unit adds v (+-) per
-// term with FP64 FMAs (x = 0: |psi_s|^2; x != 0: conj(psi_s) psi_{s^x}, real
-// and imaginary parts, of which the host keeps the one its term needs); the
-// first factor is applied once per work-item at the end.
-// Product term of one iteration: |psi_s|^2 (x = 0), or conj(psi_s) psi_{s^x}
-// as (re, im).
-template <typename T, bool PAIR>
+// One pass for the terms j < nt that share x (highest bit hbit), the pair
+// taken at the index with that bit clear. The grid stride is a power of two,
+// so an index splits into disjoint bit sets: s = s_thread | s_iter, s_thread
+// from the work-item's index and s_iter from the iteration alone (insert_run
+// maps disjoint bit sets to disjoint bit sets). Hence sigma_j(s) =
+// sigma_j(s_thread) sigma_j(s_iter): the second factor is the same for the
+// whole wave, kept as the high word of a double +-1.0 on the scalar unit and
+// updated with one XOR per term and iteration along the Gray walk; the vector
+// unit adds conj(psi_s) psi_{s^x} (+-) per term with FP64 FMAs, both parts,
+// of which the term needs one; the first factor is applied once per work-item
+// at the end.
+template <typename T>
 __device__ __forceinline__ void pauli_product(const cv<T>* __restrict__ psi, uint64_t s, uint64_t x, double& re,
                                               double& im) {
-    if constexpr (PAIR) {
-        const cv<T> u = ldamp<T, true>(psi + s);
-        const cv<T> w = ldamp<T, true>(psi + (s ^ x));
-        re = double(u.x) * double(w.x) + double(u.y) * double(w.y);
-        im = double(u.x) * double(w.y) - double(u.y) * double(w.x);
-    } else {
-        const cv<T> v = ldamp<T, true>(psi + s);
-        re = double(v.x) * double(v.x) + double(v.y) * double(v.y);
-        im = 0;
-    }
+    const cv<T> u = ldamp<T, true>(psi + s);
+    const cv<T> w = ldamp<T, true>(psi + (s ^ x));
+    re = double(u.x) * double(w.x) + double(u.y) * double(w.y);
+    im = double(u.x) * double(w.y) - double(u.y) * double(w.x);
 }
 
-template <typename T, int G, bool PAIR>
+template <typename T, int G>
 __global__ __launch_bounds__(kExThreads) void k_pauli(const cv<T>* __restrict__ psi, uint64_t npairs, uint64_t x,
                                                       uint32_t hbit, uint32_t nt, uint32_t niter, uint32_t odd_mask,
                                                       PauliFlip F, double* __restrict__ partial) {
-    // iterations per loop trip, their loads issued together: 4 single loads
-    // (x = 0) or 2 pairs
-    constexpr uint32_t U = PAIR ? 2 : 4;
     __shared__ double lds[4][G];
-    double ar[G], ai[PAIR ? G : 1];
+    double ar[G], ai[G];
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
-        ar[j] = 0;
-        if constexpr (PAIR) ai[j] = 0;
-    }
+    for (int j = 0; j < G; ++j) ar[j] = ai[j] = 0;
     uint64_t sg[G];  // the per-iteration signs (+-1.0) as bit patterns
 #pragma unroll
     for (int j = 0; j < G; ++j) sg[j] = 0x3FF0000000000000ull;
@@ -90,70 +78,45 @@ __global__ __launch_bounds__(kExThreads) void k_pauli(const cv<T>* __restrict__ 
     // adds nothing
     const bool live = t < npairs;
     const double wt = live ? 1.0 : 0.0;
-    const uint64_t st = live ? (PAIR ? insert_run(t, hbit, 1) : t) : 0;
+    const uint64_t st = live ? insert_run(t, hbit, 1) : 0;
     auto acc = [&](double re, double im, int j) {
         const double sgn = __longlong_as_double(static_cast<long long>(sg[j]));
         ar[j] = fma(re, sgn, ar[j]);
-        if constexpr (PAIR) ai[j] = fma(im, sgn, ai[j]);
+        ai[j] = fma(im, sgn, ai[j]);
     };
     uint64_t sk = 0;
-    if (niter >= U) {
-        for (uint32_t k = 0; k < niter; k += U) {
-            if (k) {  // Gray step k flips iteration bit ctz(k) >= log2(U)
+    if (niter >= 2) {
+        // two pairs a trip, their loads issued together
+        for (uint32_t k = 0; k < niter; k += 2) {
+            if (k) {  // Gray step k flips iteration bit ctz(k) >= 1
                 const uint32_t b = __builtin_ctz(k);
                 sk ^= F.bit[b];
 #pragma unroll
                 for (int j = 0; j < G; ++j) sg[j] ^= uint64_t(F.w[b][j]) << 32;
             }
-            // steps k+1 .. k+U-1 flip bits 0 / 1 0 1 / 0
-            uint64_t s[U];
-            s[0] = st | sk;
-            s[1] = s[0] ^ F.bit[0];
-            if constexpr (U == 4) {
-                s[2] = s[1] ^ F.bit[1];
-                s[3] = s[2] ^ F.bit[0];
-            }
-            double re[U], im[U];
-#pragma unroll
-            for (uint32_t u = 0; u < U; ++u) pauli_product<T, PAIR>(psi, s[u], x, re[u], im[u]);
+            const uint64_t s0 = st | sk, s1 = s0 ^ F.bit[0];  // step k+1 flips bit 0
+            double re[2], im[2];
+            pauli_product<T>(psi, s0, x, re[0], im[0]);
+            pauli_product<T>(psi, s1, x, re[1], im[1]);
 #pragma unroll
             for (int j = 0; j < G; ++j) {
                 acc(re[0], im[0], j);
                 sg[j] ^= uint64_t(F.w[0][j]) << 32;
                 acc(re[1], im[1], j);
-                if constexpr (U == 4) {
-                    sg[j] ^= uint64_t(F.w[1][j]) << 32;
-                    acc(re[2], im[2], j);
-                    sg[j] ^= uint64_t(F.w[0][j]) << 32;
-                    acc(re[3], im[3], j);
-                }
             }
-            // sk and sg of the trip's last step, k + U - 1 (from step k:
-            // bit 1 for U = 4, the two flips of bit 0 cancelling; bit 0 for
-            // U = 2)
-            sk ^= U == 4 ? F.bit[1] : F.bit[0];
+            sk ^= F.bit[0];
         }
-    } else {
-        for (uint32_t k = 0; k < niter; ++k) {
-            if (k) {
-                const uint32_t b = __builtin_ctz(k);
-                sk ^= F.bit[b];
+    } else if (niter) {
+        double re, im;
+        pauli_product<T>(psi, st, x, re, im);
 #pragma unroll
-                for (int j = 0; j < G; ++j) sg[j] ^= uint64_t(F.w[b][j]) << 32;
-            }
-            double re, im;
-            pauli_product<T, PAIR>(psi, st | sk, x, re, im);
-#pragma unroll
-            for (int j = 0; j < G; ++j) acc(re, im, j);
-        }
+        for (int j = 0; j < G; ++j) acc(re, im, j);
     }
     // per term: the part the host needs, the work-item's sign, the wave's sum
     const uint32_t w = threadIdx.x >> 6;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-        double v = ar[j];
-        if constexpr (PAIR)
-            if ((odd_mask >> j) & 1) v = ai[j];
+        double v = (odd_mask >> j) & 1 ? ai[j] : ar[j];
         v *= wt;
         if (__popcll(st & F.z[j]) & 1) v = -v;
         v = wave_sum(v);
@@ -161,20 +124,194 @@ __global__ __launch_bounds__(kExThreads) void k_pauli(const cv<T>* __restrict__ 
     }
     __syncthreads();
     if (threadIdx.x < nt)
-        partial[uint64_t(blockIdx.x) * nt + threadIdx.x] =
+        partial[threadIdx.x * gridDim.x + blockIdx.x] =
             ((lds[0][threadIdx.x] + lds[1][threadIdx.x]) + lds[2][threadIdx.x]) + lds[3][threadIdx.x];
 }
 
-// sum over blocks of the per-block partials of each term, fixed order
-__global__ __launch_bounds__(kExThreads) void k_pauli_final(const double* __restrict__ partial, uint32_t nb,
-                                                            uint32_t nt, double* __restrict__ out) {
-    __shared__ double lds[4];
-    for (uint32_t j = 0; j < nt; ++j) {
-        double acc = 0;
-        for (uint32_t b = threadIdx.x; b < nb; b += kExThreads) acc += partial[uint64_t(b) * nt + j];
-        const double t = block_sum256(acc, lds);
-        if (threadIdx.x == 0) out[j] = t;
+// The terms of a pass that a tile covers. A tile is the 2^t amplitudes that
+// differ in the t tile qubits; a term belongs to the pass if its x mask lies
+// in them. A block walks over tiles, each thread with the four amplitudes of
+// the top two tile qubits in registers and, if the pass has terms with x != 0,
+// the tile in LDS, from where it reads the partners of its pairs.
+//
+// A sum over tiles is kept per thread and register index, so the signs of a z
+// mask inside the tile come in only at the end: any number of such terms
+// costs the products of their x masks. A slot is two such sums: of the two
+// pairs of one x mask, real or imaginary part, or, in passes without pairs,
+// of two terms with x = 0 whose z mask leaves the tile. z bits outside the
+// tile flip the sign of a sum from tile to tile.
+//
+// 26 qubits complex128, a Heisenberg chain in a field (101 terms, 25 x masks):
+// 5.8 ms in a pass for each x mask and each 16 diagonal terms, 0.71 ms in
+// three tile passes. They read the 1 GiB in 190 to 294 us, the more the more
+// slots (11 in the slowest), 190 being the rate of a copy's reads: a slot
+// costs each wave a trip to LDS. One block of 1024 threads a CU holds two
+// tiles in LDS (one barrier a tile) and prefetches the next into registers.
+// 27 terms on 27 qubits complex64: 0.51 ms in two passes, now 0.26 ms in one.
+constexpr int kPtMax = 12;       // tile qubits
+constexpr int kPtThreads = 1024;  // of a full tile
+constexpr int kPtSlots = 12;
+constexpr int kPtTerms = 64;     // terms of a pass
+constexpr int kPtBlocks = 256;
+
+struct PauliTile {  // words throughout: the scalar unit loads nothing smaller
+    uint32_t t, ns, nt;
+    uint32_t im;                   // slots of imaginary parts
+    uint32_t pos[kPtMax];          // tile qubits, ascending
+    uint64_t tile_bits, step;      // the tile qubits; the grid's size on the qubits outside
+    uint32_t x[kPtSlots];          // x mask within the tile
+    uint32_t zt[2 * kPtSlots];     // z bits on the tile index; without pairs: from bit 30 on those on the register
+                                   // qubits. With pairs one word a slot
+    uint32_t first[kPtSlots + 1];  // terms first[j]..first[j+1] are slot j's, from first[ns] on those of x = 0
+    uint32_t z[kPtTerms];          // z mask within the tile; without pairs: bit 15 for the slot's second sum
+};
+
+template <typename T, bool PAIRS>
+__global__ __launch_bounds__(kPtThreads) void k_pauli_tile(const cv<T>* __restrict__ psi, uint64_t amps, uint32_t ntiles,
+                                                           PauliTile P, double* __restrict__ partial) {
+    __shared__ cv<T> s[2][PAIRS ? 1 << kPtMax : 1];
+    __shared__ double red[kPtThreads / 64][kPtTerms];
+    const uint32_t tid = threadIdx.x, t = P.t, top = t - 2;
+    const bool active = tid < 1u << top;
+    uint64_t off = 0, hi[4];
+    for (uint32_t i = 0; i < top; ++i) off |= active ? uint64_t(tid >> i & 1) << P.pos[i] : 0;
+    // a register of one qubit has two of the four amplitudes; the others'
+    // sums stay out of the results
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        hi[k] = uint64_t(k & 1) << P.pos[top] | uint64_t(k >> 1) << P.pos[top + 1];
+        if (hi[k] >= amps) hi[k] = 0;
     }
+    const bool half = amps < 4;
+    uint64_t base = blockIdx.x;
+    for (uint32_t i = 0; i < t; ++i) {
+        const uint64_t low = (1ull << P.pos[i]) - 1;
+        base = ((base & ~low) << 1) | (base & low);
+    }
+    auto load = [&](cv<T> (&a)[4]) {
+        const cv<T>* p = psi + base;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a[k] = ldamp<T, true>(p + hi[k] + off);
+    };
+    double own[4] = {0, 0, 0, 0}, sum[2 * kPtSlots];
+#pragma unroll
+    for (int i = 0; i < 2 * kPtSlots; ++i) sum[i] = 0;
+    uint32_t neg = 0;  // sums held with the opposite sign
+    cv<T> a[4], b[4];
+    uint32_t tile = blockIdx.x, buf = 0;
+    load(a);
+    for (; tile < ntiles; tile += gridDim.x, buf ^= 1) {
+        if (PAIRS && active)
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) s[buf][tid | k << top] = a[k];
+        if (tile + gridDim.x < ntiles) base = ((base | P.tile_bits) + P.step) & ~P.tile_bits;  // carries pass the tile's bits
+        load(b);
+        if (PAIRS) __syncthreads();
+        // held over the loop, the slots' LDS addresses cost 24 vector registers,
+        // their conditions 48 scalar ones, and both spill
+        uint32_t l = tid, ns = P.ns, im = P.im;
+        asm volatile("" : "+v"(l), "+s"(ns), "+s"(im));
+        double w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            w[k] = double(a[k].x) * double(a[k].x) + double(a[k].y) * double(a[k].y);
+            own[k] += w[k];
+        }
+        const double p01 = w[0] + w[1], m01 = w[0] - w[1], p23 = w[2] + w[3], m23 = w[2] - w[3];
+#pragma unroll
+        for (int j = 0; j < kPtSlots; ++j)
+            if (j < int(ns)) {
+                if constexpr (!PAIRS) {
+#pragma unroll
+                    for (int i = 2 * j; i < 2 * j + 2; ++i) {
+                        if ((__popc(tile & P.zt[i]) ^ neg >> i) & 1) {
+                            neg ^= 1u << i;
+                            sum[i] = -sum[i];
+                        }
+                        const uint32_t c = P.zt[i] >> 30;
+                        if (c == 0)
+                            sum[i] += p01 + p23;
+                        else if (c == 1)
+                            sum[i] += m01 + m23;
+                        else if (c == 2)
+                            sum[i] += p01 - p23;
+                        else
+                            sum[i] += m01 - m23;
+                    }
+                } else {
+                    if ((__popc(tile & P.zt[j]) ^ neg >> j) & 1) {
+                        neg ^= 1u << j;
+                        sum[2 * j] = -sum[2 * j];
+                        sum[2 * j + 1] = -sum[2 * j + 1];
+                    }
+                    // the pairs of thread l and thread l ^ x: l takes those of its
+                    // register indices 0 and 1, l ^ x of 2 and 3, by the highest
+                    // bit of x; a mask on the register qubits leaves each thread
+                    // two pairs of its own
+                    const uint32_t x = P.x[j], xr = x >> top, xl = x & ((1u << top) - 1);
+                    const bool up = xr == 0 && (l >> (31 - __clz(int(xl | 1))) & 1);
+                    const bool odd = up || xr == 1;
+                    const cv<T> u0 = up ? a[2] : a[0], u1 = odd ? a[3] : a[1];
+                    const cv<T> v0 = s[buf][(l | (up ? 2u << top : 0)) ^ x];
+                    const cv<T> v1 = s[buf][(l | (odd ? 3u : 1u) << top) ^ x];
+                    if (!(im >> j & 1)) {
+                        sum[2 * j] = fma(double(u0.x), double(v0.x), fma(double(u0.y), double(v0.y), sum[2 * j]));
+                        sum[2 * j + 1] = fma(double(u1.x), double(v1.x), fma(double(u1.y), double(v1.y), sum[2 * j + 1]));
+                    } else {
+                        sum[2 * j] = fma(double(u0.x), double(v0.y), fma(-double(u0.y), double(v0.x), sum[2 * j]));
+                        sum[2 * j + 1] = fma(double(u1.x), double(v1.y), fma(-double(u1.y), double(v1.x), sum[2 * j + 1]));
+                    }
+                }
+            }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a[k] = b[k];
+    }
+    // per term: the signs of the thread's indices, the wave's sum
+    const uint32_t wave = tid >> 6, lane = tid & 63;
+    auto put = [&](uint32_t e, double v) {
+        v = wave_sum(active ? v : 0.0);
+        if (lane == 0) red[wave][e] = v;
+    };
+    auto sgn = [](uint32_t z, uint32_t i, double v) { return __popc(z & i) & 1 ? -v : v; };
+#pragma unroll
+    for (int j = 0; j < kPtSlots; ++j)
+        if (j < int(P.ns)) {
+            const double s0 = neg >> (PAIRS ? j : 2 * j) & 1 ? -sum[2 * j] : sum[2 * j];
+            const double s1 = PAIRS && half ? 0 : neg >> (PAIRS ? j : 2 * j + 1) & 1 ? -sum[2 * j + 1] : sum[2 * j + 1];
+            const uint32_t x = P.x[j], xr = x >> top, xl = x & ((1u << top) - 1);
+            const bool up = xr == 0 && (tid >> (31 - __clz(int(xl | 1))) & 1);
+            const uint32_t i0 = tid | (up ? 2u << top : 0), i1 = tid | (up || xr == 1 ? 3u : 1u) << top;
+            for (uint32_t e = P.first[j]; e < P.first[j + 1]; ++e) {
+                const uint32_t z = P.z[e];
+                if (!PAIRS)
+                    put(e, sgn(z & ((1u << top) - 1), tid, z >> 15 ? s1 : s0));
+                else
+                    put(e, sgn(z, i0, s0) + sgn(z, i1, s1));
+            }
+        }
+    if (half) own[2] = own[3] = 0;
+    for (uint32_t e = P.first[P.ns]; e < P.nt; ++e) {
+        const uint32_t z = P.z[e];
+        put(e, (sgn(z, tid, own[0]) + sgn(z, tid | 1u << top, own[1])) +
+                   (sgn(z, tid | 2u << top, own[2]) + sgn(z, tid | 3u << top, own[3])));
+    }
+    __syncthreads();
+    if (tid < P.nt) {
+        double v = red[0][tid];
+        for (uint32_t i = 1; i < blockDim.x / 64; ++i) v += red[i][tid];
+        partial[tid * gridDim.x + blockIdx.x] = v;
+    }
+}
+
+// out[j] = sum of the nb partials of term j = blockIdx.x, in a fixed order
+__global__ __launch_bounds__(kExThreads) void k_pauli_final(const double* __restrict__ partial, uint32_t nb,
+                                                            double* __restrict__ out) {
+    __shared__ double lds[4];
+    const double* p = partial + size_t(blockIdx.x) * nb;
+    double acc = 0;
+    for (uint32_t b = threadIdx.x; b < nb; b += kExThreads) acc += p[b];
+    const double t = block_sum256(acc, lds);
+    if (threadIdx.x == 0) out[blockIdx.x] = t;
 }
 
 // <psi[0..len) | v[0..len)> partial sums (conj(psi) v), FP64.
@@ -288,84 +425,216 @@ static uint64_t xfer_amps(const qcs_register* r) {
 
 static uint32_t grid256(uint64_t n) { return uint32_t((n + 255) / 256); }
 
+// <P> from the sum S of a term's pass.
+static double pauli_scale(uint64_t x, uint64_t z) {
+    if (!x) return 1;
+    const uint32_t ny = uint32_t(__builtin_popcountll(x & z));
+    return ny / 2 & 1 ? -2.0 : 2.0;
+}
+
+// Terms of one x mask too wide for a tile, kPauliTerms at a time.
+template <typename T>
+static int pauli_wide(qcs_register* r, const std::vector<uint32_t>& terms, uint64_t x, const uint64_t* zmask,
+                      double* out) {
+    const uint64_t npairs = r->A / 2;
+    const uint32_t hbit = uint32_t(63 - __builtin_clzll(x));
+    double* res = r->red + kRedResult;
+    for (size_t t0 = 0; t0 < terms.size(); t0 += kPauliTerms) {
+        const uint32_t nt = uint32_t(std::min<size_t>(kPauliTerms, terms.size() - t0));
+        uint32_t odd = 0;
+        // a power-of-two grid (the sign split needs a power-of-two stride)
+        uint64_t nb = 1;
+        while (nb < uint64_t(kPauliBlocks) && nb * kExThreads * 8 < npairs) nb <<= 1;
+        const uint64_t stride = nb * kExThreads;
+        const uint32_t lstride = uint32_t(__builtin_ctzll(stride));
+        const uint64_t niter = npairs > stride ? npairs / stride : 1;
+        const uint32_t ibits = uint32_t(__builtin_ctzll(niter));
+        if (ibits > kFlipBits) return set_error(QCS_EINVAL, "state too large for the Pauli pass");
+        PauliFlip F{};
+        for (uint32_t j = 0; j < nt; ++j) {
+            const uint64_t z = zmask[terms[t0 + j]];
+            F.z[j] = z;
+            if (__builtin_popcountll(x & z) & 1) odd |= 1u << j;
+        }
+        for (uint32_t b = 0; b < ibits; ++b) {
+            const uint32_t kb = lstride + b, pos = kb >= hbit ? kb + 1 : kb;
+            F.bit[b] = 1ull << pos;
+            for (uint32_t j = 0; j < nt; ++j) F.w[b][j] = uint32_t((F.z[j] >> pos) & 1) << 31;
+        }
+        const cv<T>* psi = static_cast<const cv<T>*>(r->psi);
+        const dim3 grid{unsigned(nb)}, block{unsigned(kExThreads)};
+        if (nt <= 8)
+            hipLaunchKernelGGL((k_pauli<T, 8>), grid, block, 0, r->stream, psi, npairs, x, hbit, nt, uint32_t(niter), odd,
+                               F, r->red);
+        else
+            hipLaunchKernelGGL((k_pauli<T, kPauliTerms>), grid, block, 0, r->stream, psi, npairs, x, hbit, nt,
+                               uint32_t(niter), odd, F, r->red);
+        if (const int e = check_launch(r, "k_pauli")) return e;
+        hipLaunchKernelGGL(k_pauli_final, dim3(nt), dim3(kExThreads), 0, r->stream, r->red, uint32_t(nb), res);
+        if (const int e = check_launch(r, "k_pauli_final")) return e;
+        double sums[kPauliTerms];
+        if (const int e = fetch(r, res, int(nt), sums)) return e;
+        for (uint32_t j = 0; j < nt; ++j) out[terms[t0 + j]] = pauli_scale(x, zmask[terms[t0 + j]]) * sums[j];
+    }
+    return QCS_OK;
+}
+
+// The qubits of the next tile: the lowest ones, for whole memory lines, then
+// the x masks that need the fewest more, in order of first appearance.
+static uint64_t pauli_tile_qubits(const std::vector<uint64_t>& xs, uint64_t low, uint32_t n, uint32_t t) {
+    uint64_t S = low;
+    for (;;) {
+        uint64_t best = 0;
+        int need = 64;
+        for (const uint64_t x : xs) {
+            const int more = __builtin_popcountll(x & ~S);
+            if (more && more < need && more + __builtin_popcountll(S) <= int(t)) {
+                need = more;
+                best = x;
+            }
+        }
+        if (!best) break;
+        S |= best;
+    }
+    for (uint32_t q = 0; q < n && __builtin_popcountll(S) < int(t); ++q) S |= 1ull << q;
+    return S;
+}
+
+// bits of m at the set bits of S, packed
+static uint32_t pack_bits(uint64_t m, uint64_t S) {
+    uint32_t v = 0, i = 0;
+    for (; S; S &= S - 1, ++i) v |= uint32_t(m >> __builtin_ctzll(S) & 1) << i;
+    return v;
+}
+
 template <typename T>
 static int pauli_t(qcs_register* r, uint32_t nterms, const uint64_t* xmask, const uint64_t* zmask, double* out) {
     const uint64_t full = r->A - 1;
-    // terms grouped by x mask, in order of first appearance
-    std::vector<uint64_t> xs;
-    std::map<uint64_t, std::vector<uint32_t>> groups;
-    for (uint32_t t = 0; t < nterms; ++t) {
+    for (uint32_t t = 0; t < nterms; ++t)
         if ((xmask[t] | zmask[t]) & ~full) return set_error(QCS_EINVAL, "term %u: mask beyond the register", t);
-        auto it = groups.find(xmask[t]);
-        if (it == groups.end()) {
-            xs.push_back(xmask[t]);
-            groups[xmask[t]] = {t};
+    const uint32_t n = r->n, t = std::max<uint32_t>(2, std::min<uint32_t>(n, kPtMax));
+    const uint64_t low = (1ull << std::min<uint32_t>(n, sizeof(T) == 8 ? 3 : 4)) - 1;
+    const uint32_t ntiles = n > t ? 1u << (n - t) : 1, nb = std::min<uint32_t>(ntiles, kPtBlocks);
+    std::vector<uint32_t> rest;
+    std::vector<uint64_t> wide, xs;
+    std::map<uint64_t, std::vector<uint32_t>> wides;
+    for (uint32_t i = 0; i < nterms; ++i) {
+        const uint64_t x = xmask[i];
+        if (__builtin_popcountll(x | low) <= int(t)) {
+            rest.push_back(i);
         } else {
-            it->second.push_back(t);
+            if (!wides.count(x)) wide.push_back(x);
+            wides[x].push_back(i);
         }
     }
+    // the terms whose sums are on their way
+    std::vector<uint32_t> batch;
     double* res = r->red + kRedResult;
-    for (const uint64_t x : xs) {
-        const std::vector<uint32_t>& terms = groups[x];
-        const uint64_t npairs = x ? r->A / 2 : r->A;
-        const uint32_t hbit = x ? uint32_t(63 - __builtin_clzll(x)) : 0;
-        for (size_t t0 = 0; t0 < terms.size(); t0 += kPauliTerms) {
-            const uint32_t nt = uint32_t(std::min<size_t>(kPauliTerms, terms.size() - t0));
-            uint32_t odd = 0;
-            // a power-of-two grid (the sign split needs a power-of-two stride)
-            uint64_t nb = 1;
-            while (nb < uint64_t(kPauliBlocks) && nb * kExThreads * 8 < npairs) nb <<= 1;
-            const uint64_t stride = nb * kExThreads;
-            const uint32_t lstride = uint32_t(__builtin_ctzll(stride));
-            const uint64_t niter = npairs > stride ? npairs / stride : 1;
-            const uint32_t ibits = uint32_t(__builtin_ctzll(niter));
-            if (ibits > kFlipBits) return set_error(QCS_EINVAL, "state too large for the Pauli pass");
-            PauliFlip F{};
-            for (uint32_t j = 0; j < nt; ++j) {
-                const uint64_t z = zmask[terms[t0 + j]];
-                F.z[j] = z;
-                if (__builtin_popcountll(x & z) & 1) odd |= 1u << j;
-            }
-            for (uint32_t b = 0; b < ibits; ++b) {
-                const uint32_t kb = lstride + b, pos = (x && kb >= hbit) ? kb + 1 : kb;
-                F.bit[b] = 1ull << pos;
-                for (uint32_t j = 0; j < nt; ++j) F.w[b][j] = uint32_t((F.z[j] >> pos) & 1) << 31;
-            }
-            const cv<T>* psi = static_cast<const cv<T>*>(r->psi);
-            const dim3 grid{unsigned(nb)}, block{unsigned(kExThreads)};
-            const uint32_t ni = uint32_t(niter);
-            if (x == 0) {
-                if (nt <= 8)
-                    hipLaunchKernelGGL((k_pauli<T, 8, false>), grid, block, 0, r->stream, psi, npairs, x, hbit, nt, ni,
-                                       odd, F, r->red);
-                else
-                    hipLaunchKernelGGL((k_pauli<T, kPauliTerms, false>), grid, block, 0, r->stream, psi, npairs, x,
-                                       hbit, nt, ni, odd, F, r->red);
-            } else {
-                if (nt <= 8)
-                    hipLaunchKernelGGL((k_pauli<T, 8, true>), grid, block, 0, r->stream, psi, npairs, x, hbit, nt, ni,
-                                       odd, F, r->red);
-                else
-                    hipLaunchKernelGGL((k_pauli<T, kPauliTerms, true>), grid, block, 0, r->stream, psi, npairs, x,
-                                       hbit, nt, ni, odd, F, r->red);
-            }
-            if (const int e = check_launch(r, "k_pauli")) return e;
-            hipLaunchKernelGGL(k_pauli_final, dim3(1), dim3(kExThreads), 0, r->stream, r->red, uint32_t(nb), nt, res);
-            if (const int e = check_launch(r, "k_pauli_final")) return e;
-            double sums[kPauliTerms];
-            if (const int e = fetch(r, res, int(nt), sums)) return e;
-            for (uint32_t j = 0; j < nt; ++j) {
-                const uint32_t t = terms[t0 + j];
-                const uint32_t ny = uint32_t(__builtin_popcountll(x & zmask[t]));
-                if (x == 0) {
-                    out[t] = sums[j];
-                } else {
-                    const uint32_t k = (ny & 1) ? (ny - 1) / 2 : ny / 2;
-                    out[t] = (k & 1 ? -2.0 : 2.0) * sums[j];
+    auto flush = [&]() -> int {
+        if (batch.empty()) return QCS_OK;
+        hipLaunchKernelGGL(k_pauli_final, dim3(unsigned(batch.size())), dim3(kExThreads), 0, r->stream, r->red, nb, res);
+        if (const int e = check_launch(r, "k_pauli_final")) return e;
+        double sums[kPauliResults];
+        if (const int e = fetch(r, res, int(batch.size()), sums)) return e;
+        for (size_t j = 0; j < batch.size(); ++j) out[batch[j]] = pauli_scale(xmask[batch[j]], zmask[batch[j]]) * sums[j];
+        batch.clear();
+        return QCS_OK;
+    };
+    while (!rest.empty()) {
+        xs.clear();
+        for (const uint32_t i : rest)
+            if (xmask[i] && std::find(xs.begin(), xs.end(), xmask[i]) == xs.end()) xs.push_back(xmask[i]);
+        const uint64_t S = n < t ? 3 : pauli_tile_qubits(xs, low, n, t);
+        PauliTile P{};
+        P.t = t;
+        P.tile_bits = S;
+        P.step = nb;
+        for (uint64_t m = S, i = 0; m; m &= m - 1) P.pos[i++] = uint32_t(__builtin_ctzll(m));
+        for (uint32_t i = 0; i < t; ++i) {
+            const uint64_t below = (1ull << P.pos[i]) - 1;
+            P.step = ((P.step & ~below) << 1) | (P.step & below);
+        }
+        struct Slot {
+            uint64_t x;
+            bool im;
+            uint32_t zt, halves;
+            std::vector<uint32_t> terms;
+            std::vector<uint32_t> z;
+        };
+        std::vector<Slot> slots;
+        std::vector<uint32_t> inner, left;
+        const uint32_t top = t - 2;
+        uint32_t taken = 0;
+        const uint32_t most = std::min<uint32_t>(kPtTerms, kPauliResults - uint32_t(batch.size()));
+        for (const uint32_t i : rest) {
+            const uint64_t x = xmask[i], z = zmask[i];
+            const uint32_t zt = pack_bits(z, full & ~S), zl = pack_bits(z, S);
+            bool ok = taken < most && !(x & ~S);
+            if (ok && x) {
+                const bool im = __builtin_popcountll(x & z) & 1;
+                size_t j = 0;
+                while (j < slots.size() && !(slots[j].x == x && slots[j].im == im && slots[j].zt == zt)) ++j;
+                ok = j < slots.size() || j < kPtSlots;
+                if (ok) {
+                    if (j == slots.size()) {
+                        slots.push_back(Slot{x, im, zt, 2, {}, {}});
+                        P.zt[j] = zt;
+                    }
+                    slots[j].terms.push_back(i);
+                    slots[j].z.push_back(zl);
+                }
+            } else if (ok && !zt) {
+                inner.push_back(i);
+            } else if (ok) {
+                // with a later x mask's tile around it it costs nothing
+                size_t j = slots.size();
+                const bool half = j && slots[j - 1].halves == 1;
+                ok = xs.empty() && (half || j < kPtSlots);
+                if (ok) {
+                    if (!half) slots.push_back(Slot{0, false, 0, 0, {}, {}});
+                    j = slots.size() - 1;
+                    const uint32_t h = slots[j].halves++;
+                    P.zt[2 * j + h] = zt | (zl >> top) << 30;
+                    slots[j].terms.push_back(i);
+                    slots[j].z.push_back(zl | h << 15);
                 }
             }
+            if (ok)
+                ++taken;
+            else
+                left.push_back(i);
         }
+        if (!taken) {  // no result slot free
+            if (const int e = flush()) return e;
+            continue;
+        }
+        bool pairs = false;
+        P.ns = uint32_t(slots.size());
+        for (size_t j = 0; j < slots.size(); ++j) {
+            P.im |= uint32_t(slots[j].im) << j;
+            P.x[j] = pack_bits(slots[j].x, S);
+            pairs = pairs || slots[j].x;
+            P.first[j] = P.nt;
+            for (size_t k = 0; k < slots[j].terms.size(); ++k) P.z[P.nt++] = slots[j].z[k];
+        }
+        P.first[P.ns] = P.nt;
+        for (const uint32_t i : inner) P.z[P.nt++] = pack_bits(zmask[i], S);
+        const unsigned threads = std::max(64u, 1u << top);
+        double* partial = r->red + batch.size() * nb;
+        if (pairs)
+            hipLaunchKernelGGL((k_pauli_tile<T, true>), dim3(nb), dim3(threads), 0, r->stream,
+                               static_cast<const cv<T>*>(r->psi), r->A, ntiles, P, partial);
+        else
+            hipLaunchKernelGGL((k_pauli_tile<T, false>), dim3(nb), dim3(threads), 0, r->stream,
+                               static_cast<const cv<T>*>(r->psi), r->A, ntiles, P, partial);
+        if (const int e = check_launch(r, "k_pauli_tile")) return e;
+        for (const Slot& sl : slots) batch.insert(batch.end(), sl.terms.begin(), sl.terms.end());
+        batch.insert(batch.end(), inner.begin(), inner.end());
+        rest.swap(left);
     }
+    if (const int e = flush()) return e;
+    for (const uint64_t x : wide)
+        if (const int e = pauli_wide<T>(r, wides[x], x, zmask, out)) return e;
     return QCS_OK;
 }
 
