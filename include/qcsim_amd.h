@@ -290,8 +290,8 @@ int qcs_qaoa_plan(uint32_t n, uint32_t tile_bits, uint32_t group, uint32_t p, ui
  * Pauli-string Hamiltonian, the value VariationalQuantumEigensolver::
  * EstimateEnergy (VQE.h:204-212) estimates from sampled parities. Instance
  * i has nqubits[i] qubits and nterms[i] terms (x masks, z masks and
- * coefficients concatenated; masks as in qcs_pauli_expectation). One launch
- * per size class (<= 8, <= 10, <= 12 qubits), complex128 state in LDS. */
+ * coefficients concatenated; masks as in qcs_pauli_expectation). One launch,
+ * complex128 state in LDS. */
 typedef struct qcs_vqe qcs_vqe;
 int qcs_vqe_create(uint32_t ninst, const uint32_t* nqubits, const uint32_t* nterms,
                    const uint64_t* xmask, const uint64_t* zmask, const double* coef,

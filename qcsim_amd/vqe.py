@@ -5,7 +5,7 @@ hardware-efficient ansatz (VQE::PauliStringVQE::Ansatz, VQE.h:78-114) and
 scored with the exact FP64 energy sum_t c_t <psi|P_t|psi> of a Pauli-string
 Hamiltonian: the value that VariationalQuantumEigensolver::EstimateEnergy
 (VQE.h:204-212) estimates from 10000 samples per term. Instances of uneven
-size and parameter count run together, one launch per size class.
+size and parameter count run together in one launch.
 
 ``ansatz_gates`` gives the same ansatz as a gate list, for a single register
 (QubitRegister.ApplyGate) of any size.
