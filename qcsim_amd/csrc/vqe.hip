@@ -32,6 +32,7 @@
 // one a term).
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "common.h"
@@ -329,12 +330,13 @@ struct qcs_vqe {
     std::vector<VInst> hinst;
     uint32_t nunits = 0;
     size_t lds = 0;                   // of a block
-    VInst* dinst = nullptr;
     VUnit* dunits = nullptr;
     uint64_t* dxm = nullptr;
     uint64_t* dzm = nullptr;
     double* dcoef = nullptr;
-    double* dparams = nullptr;
+    // what an evaluation sends, in one copy: the instances, then the parameters
+    std::vector<char> stage;
+    char* dstage = nullptr;
     size_t params_cap = 0;
     double2* arena = nullptr;
     double* denergy = nullptr;
@@ -348,8 +350,8 @@ extern "C" {
 int qcs_vqe_destroy(qcs_vqe* v) {
     if (!v) return QCS_OK;
     if (v->stream) (void)hipStreamSynchronize(v->stream);
-    for (void* p : {static_cast<void*>(v->dinst), static_cast<void*>(v->dunits), static_cast<void*>(v->dxm),
-                    static_cast<void*>(v->dzm), static_cast<void*>(v->dcoef), static_cast<void*>(v->dparams),
+    for (void* p : {static_cast<void*>(v->dunits), static_cast<void*>(v->dxm),
+                    static_cast<void*>(v->dzm), static_cast<void*>(v->dcoef), static_cast<void*>(v->dstage),
                     static_cast<void*>(v->arena), static_cast<void*>(v->denergy)})
         if (p) (void)hipFree(p);
     if (v->ev0) (void)hipEventDestroy(v->ev0);
@@ -418,8 +420,7 @@ int qcs_vqe_create(uint32_t ninst, const uint32_t* nqubits, const uint32_t* nter
         qcs_vqe_destroy(v);
         return set_error(QCS_EDEVICE, "stream creation failed");
     }
-    if (hipMalloc(reinterpret_cast<void**>(&v->dinst), sizeof(VInst) * ninst) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void**>(&v->dunits), sizeof(VUnit) * units.size()) != hipSuccess ||
+    if (hipMalloc(reinterpret_cast<void**>(&v->dunits), sizeof(VUnit) * units.size()) != hipSuccess ||
         hipMalloc(reinterpret_cast<void**>(&v->dxm), sizeof(uint64_t) * nt) != hipSuccess ||
         hipMalloc(reinterpret_cast<void**>(&v->dzm), sizeof(uint64_t) * nt) != hipSuccess ||
         hipMalloc(reinterpret_cast<void**>(&v->dcoef), sizeof(double) * nt) != hipSuccess ||
@@ -450,25 +451,28 @@ int qcs_vqe_evaluate(qcs_vqe* v, const uint32_t* nparams, const double* params, 
         if (poff > 0xffffffffull) return set_error(QCS_EINVAL, "too many parameters");
     }
     if (poff && !params) return set_error(QCS_EINVAL, "null parameters");
-    if (poff > v->params_cap) {
+    const size_t ibytes = sizeof(VInst) * v->ninst, pbytes = sizeof(double) * poff;
+    if (!v->dstage || poff > v->params_cap) {
         if (hipStreamSynchronize(v->stream) != hipSuccess) return set_error(QCS_EDEVICE, "sync failed");
-        if (v->dparams) (void)hipFree(v->dparams);
-        v->dparams = nullptr;
+        if (v->dstage) (void)hipFree(v->dstage);
+        v->dstage = nullptr;
         v->params_cap = 0;
-        if (hipMalloc(reinterpret_cast<void**>(&v->dparams), sizeof(double) * poff) != hipSuccess) {
+        if (hipMalloc(reinterpret_cast<void**>(&v->dstage), ibytes + pbytes) != hipSuccess) {
             (void)hipGetLastError();
+            v->dstage = nullptr;
             return set_error(QCS_ENOMEM, "parameter buffer");
         }
         v->params_cap = poff;
+        v->stage.resize(ibytes + pbytes);
     }
-    if ((poff && hipMemcpyAsync(v->dparams, params, sizeof(double) * poff, hipMemcpyHostToDevice, v->stream) !=
-                     hipSuccess) ||
-        hipMemcpyAsync(v->dinst, v->hinst.data(), sizeof(VInst) * v->ninst, hipMemcpyHostToDevice, v->stream) !=
-            hipSuccess ||
+    std::memcpy(v->stage.data(), v->hinst.data(), ibytes);
+    if (poff) std::memcpy(v->stage.data() + ibytes, params, pbytes);
+    if (hipMemcpyAsync(v->dstage, v->stage.data(), ibytes + pbytes, hipMemcpyHostToDevice, v->stream) != hipSuccess ||
         hipEventRecord(v->ev0, v->stream) != hipSuccess)
         return set_error(QCS_EDEVICE, "batched VQE upload failed");
-    hipLaunchKernelGGL(k_vqe, dim3(v->nunits), dim3(256), v->lds, v->stream, v->dinst, v->dunits, v->dparams, v->dxm,
-                       v->dzm, v->dcoef, v->arena, v->denergy);
+    hipLaunchKernelGGL(k_vqe, dim3(v->nunits), dim3(256), v->lds, v->stream,
+                       reinterpret_cast<const VInst*>(v->dstage), v->dunits,
+                       reinterpret_cast<const double*>(v->dstage + ibytes), v->dxm, v->dzm, v->dcoef, v->arena, v->denergy);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(QCS_EDEVICE, "k_vqe launch failed: %s", hipGetErrorString(e));
     if (hipEventRecord(v->ev1, v->stream) != hipSuccess ||

@@ -26,6 +26,7 @@ T_ISWAP = 0x20
 T_ISWAPDAG = 0x40
 
 _S2 = 1.0 / math.sqrt(2.0)
+_QUBITS = {2: 1, 4: 2, 8: 3}
 
 
 class QuantumGateWithOp:
@@ -42,7 +43,8 @@ class QuantumGateWithOp:
         return self._m
 
     def getQubitsNumber(self) -> int:
-        return int(round(math.log2(self._m.shape[0])))
+        n = self._m.shape[0]
+        return _QUBITS.get(n) or int(round(math.log2(n)))
 
     def setOperator(self, m):
         self._m = np.array(m, dtype=np.complex128)

@@ -108,10 +108,15 @@ class VqeBatch:
     def evaluate(self, params) -> np.ndarray:
         """params: one sequence of ansatz parameters per instance (lengths may
         differ). Returns the energies."""
-        counts = np.array([len(p) for p in params], dtype=np.uint32)
+        counts = np.fromiter(map(len, params), dtype=np.uint32)
         assert counts.shape[0] == len(self.instances)
-        flat = np.ascontiguousarray(np.concatenate([np.asarray(p, dtype=np.float64) for p in params])
-                                    if counts.sum() else np.zeros(1))
+        if not counts.any():
+            flat = np.zeros(1)
+        else:
+            try:
+                flat = np.ascontiguousarray(np.concatenate(params, dtype=np.float64))
+            except TypeError:  # values that numpy converts one by one only
+                flat = np.concatenate([np.asarray(p, dtype=np.float64) for p in params])
         out = np.zeros(len(self.instances))
         check(lib().qcs_vqe_evaluate(self._h, counts.ctypes.data_as(_PU32), flat.ctypes.data_as(_PD),
                                      out.ctypes.data_as(_PD)))
