@@ -62,7 +62,7 @@ struct QUnit {
     uint32_t layer;
     uint32_t qlo;    // first qubit of the mixer group
     uint32_t slot;   // energy partial slot (mixer with energy)
-    uint32_t ntile;  // consecutive tiles from idx (tile launches)
+    uint32_t ntile;  // consecutive tiles, or 256-orbit chunks, from idx
     uint32_t flags;  // tile launches: kTileRxOnly
 };
 
@@ -86,6 +86,13 @@ __host__ __device__ __forceinline__ uint64_t arena_xor(uint64_t i) {
 constexpr uint32_t kMixChunks = 8;  // 256-orbit chunks per mixer unit
 constexpr uint32_t kTileRun = 8;    // tiles per tile unit (one instance) with the cost diagonal
 constexpr uint32_t kTileRunRx = 64; // tiles per Rx-only tile unit (no per-tile terms to stage)
+// Those are the longest runs: a launch that they would cut into fewer units
+// than there are CUs takes shorter ones, for about two units a CU. At depth 4,
+// us with the longest runs and with shorter ones: one instance of 22 qubits
+// 921 and 296, eight of 20 qubits 929 and 417, one of 14 qubits 191 and 131;
+// above the line shorter runs pay their units' setup without a gain (sixteen
+// instances of 22 qubits 2000 and 2101, 256 of 14 qubits 277 and 284).
+constexpr uint32_t kUnitsFew = 256, kUnits = 512;
 
 // Instance parameters staged in LDS by every unit.
 struct IsingLds {
@@ -777,7 +784,7 @@ __global__ __launch_bounds__(256, 4) void k_qaoa_tile_rx(float2* __restrict__ ar
 // index at hand, can run in any pass that sees each amplitude once.
 enum : int { MIX_PLAIN = 0, MIX_ENERGY = 1, MIX_MERGE = 2 };
 
-// Mixer units: kMixChunks chunks of 256 orbits of the qubits qlo ..
+// Mixer units: runs of chunks of 256 orbits of the qubits qlo ..
 // qlo+g-1, in the unit's mode.
 template <int g, int MODE>
 __global__ __launch_bounds__(256) void k_qaoa_mix(float2* __restrict__ arena, const QInst* __restrict__ insts,
@@ -844,7 +851,7 @@ __global__ __launch_bounds__(256) void k_qaoa_mix(float2* __restrict__ arena, co
         double hz = 0, jzz = 0;
         uint64_t prev = 0;
 #pragma unroll 1
-        for (uint32_t r = 0; r < kMixChunks; ++r) {
+        for (uint32_t r = 0; r < U.ntile; ++r) {
             const uint64_t o = (uint64_t(U.idx) + r) * 256 + threadIdx.x;
             if (o >= norb) break;
             const uint64_t base = insert_run(o, U.qlo, g);
@@ -1170,42 +1177,49 @@ static int build_plan(qcs_qaoa* q) {
     for (uint32_t i : large) {
         passes.push_back(instance_passes(q->nq[i], Tm, G, q->p));
         nstep = std::max(nstep, passes.back().size());
-        // energy slots: one per unit of the instance's last pass
-        QInst& I = q->inst_h[i];
-        const uint64_t chunks = (((1ull << q->nq[i]) >> passes.back().back().g) + 255) / 256;
-        I.tbits = Tm;
-        I.pslot0 = pslot;
-        I.npslots = uint32_t((chunks + kMixChunks - 1) / kMixChunks);
-        pslot += I.npslots;
+        q->inst_h[i].tbits = Tm;
     }
     // step s: pass s of every instance that has one, one launch per
     // (kind, width, mode) present
     for (size_t s = 0; s < nstep; ++s) {
         const size_t first = pend.size();
-        for (size_t k = 0; k < large.size(); ++k) {
-            if (s >= passes[k].size()) continue;
-            const PassSpec& S = passes[k][s];
-            const uint32_t i = large[k], n = q->nq[i];
-            const bool tile = S.kind == qcs_qaoa::L_TILE;
-            // Rx-only tile passes run on their own kernel
-            const uint8_t kind = tile && (S.mode & kTileRxOnly) ? uint8_t(qcs_qaoa::L_TILE_RX) : S.kind;
-            const uint8_t g = tile ? 0 : S.g, md = tile ? 0 : S.mode;
-            size_t j = first;
-            while (j < pend.size() && !(pend[j].kind == kind && pend[j].g == g && pend[j].mode == md)) ++j;
-            if (j == pend.size()) pend.push_back(Pending{kind, g, md, {}});
-            auto& P = pend[j];
-            if (tile) {
-                const uint32_t run = (S.mode & kTileRxOnly) ? kTileRunRx : kTileRun;
-                for (uint32_t t = 0, nt = 1u << (n - Tm); t < nt; t += run)
-                    P.units.push_back(QUnit{i, t, S.layer, 0, 0, std::min(run, nt - t), S.mode});
-            } else {
-                const bool en = S.mode == MIX_ENERGY;
-                const uint64_t chunks = (((1ull << n) >> S.g) + 255) / 256;
-                uint32_t slot = q->inst_h[i].pslot0;
-                for (uint64_t c = 0; c < chunks; c += kMixChunks)
-                    P.units.push_back(QUnit{i, uint32_t(c), S.layer, S.qlo, en ? slot++ : 0u, 0, 0});
+        std::vector<uint64_t> work, units;  // of each launch: tiles or chunks, and units of the longest runs
+        // first what each launch does, then its units, in runs by that
+        for (int emit = 0; emit < 2; ++emit)
+            for (size_t k = 0; k < large.size(); ++k) {
+                if (s >= passes[k].size()) continue;
+                const PassSpec& S = passes[k][s];
+                const uint32_t i = large[k], n = q->nq[i];
+                const bool tile = S.kind == qcs_qaoa::L_TILE, rx = tile && (S.mode & kTileRxOnly);
+                // Rx-only tile passes run on their own kernel
+                const uint8_t kind = rx ? uint8_t(qcs_qaoa::L_TILE_RX) : S.kind;
+                const uint8_t g = tile ? 0 : S.g, md = tile ? 0 : S.mode;
+                const uint64_t count = tile ? 1ull << (n - Tm) : (((1ull << n) >> S.g) + 255) / 256;
+                const uint32_t longest = rx ? kTileRunRx : tile ? kTileRun : kMixChunks;
+                size_t j = first;
+                while (j < pend.size() && !(pend[j].kind == kind && pend[j].g == g && pend[j].mode == md)) ++j;
+                if (!emit) {
+                    if (j == pend.size()) {
+                        pend.push_back(Pending{kind, g, md, {}});
+                        work.push_back(0);
+                        units.push_back(0);
+                    }
+                    work[j - first] += count;
+                    units[j - first] += (count + longest - 1) / longest;
+                    continue;
+                }
+                const uint32_t run = units[j - first] >= kUnitsFew
+                                         ? longest
+                                         : uint32_t(std::clamp<uint64_t>(work[j - first] / kUnits, 1, longest));
+                // energy slots: one per unit of the instance's last pass
+                const bool en = !tile && S.mode == MIX_ENERGY;
+                if (en) q->inst_h[i].pslot0 = pslot;
+                for (uint64_t t = 0; t < count; t += run)
+                    pend[j].units.push_back(QUnit{i, uint32_t(t), S.layer, S.qlo, en ? pslot++ : 0u,
+                                                  uint32_t(std::min<uint64_t>(run, count - t)),
+                                                  tile ? uint32_t(S.mode) : 0u});
+                if (en) q->inst_h[i].npslots = pslot - q->inst_h[i].pslot0;
             }
-        }
     }
     q->nstages = uint32_t(pend.size());
     if (hipMemcpy(q->d_inst, q->inst_h.data(), sizeof(QInst) * q->ninst, hipMemcpyHostToDevice) != hipSuccess)

@@ -173,3 +173,27 @@ def test_large_uneven_batch_sample_matches_oracle():
         assert abs(E[i] - e_ref) < 2e-5 * scale, (i, inst.n, E[i], e_ref)
         assert err < 3e-6, (i, inst.n, err)
     batch.close()
+
+
+@pytest.mark.parametrize("n,copies", [(14, 1), (14, 3), (14, 200), (18, 20), (20, 1)])
+def test_unit_runs_do_not_change_an_instance(n, copies):
+    """Few instances are cut into short units, many into the longest ones: the
+    state of an instance is the same in either, its energy but for the order
+    of the FP64 partial sums; alone it equals the oracle's."""
+    p = 3
+    inst = make_batch_instances(31 * n, [n])[0]
+    rng = np.random.default_rng(n)
+    G, B = rng.uniform(0, np.pi, (1, p)), rng.uniform(0, np.pi, (1, p))
+    alone = QaoaBatch([inst], p)
+    many = QaoaBatch([inst] * copies, p)
+    e1 = alone.evaluate(G, B)
+    em = many.evaluate(np.repeat(G, copies, axis=0), np.repeat(B, copies, axis=0))
+    s1 = alone.state(0)
+    assert np.array_equal(s1, many.state(copies - 1))
+    scale = 1 + np.sum(np.abs(inst.J)) + np.sum(np.abs(inst.h))
+    assert np.max(np.abs(em - e1[0])) < 1e-12 * scale
+    e_ref, psi_ref = oracle_eval(inst, G[0], B[0])
+    assert abs(e1[0] - e_ref) < 2e-5 * scale
+    assert np.max(np.abs(s1 - psi_ref)) < 3e-6
+    alone.close()
+    many.close()
