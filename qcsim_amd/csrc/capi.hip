@@ -146,8 +146,7 @@ int qcs_create(uint32_t nqubits, int precision, qcs_register** out) {
         if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess ||
             hipEventRecord(ev, r->stream) != hipSuccess)
             return fail(QCS_EDEVICE, "staging event creation failed");
-    int e = kfill(r, 0, 0);
-    if (!e) e = kset_one(r, 0, 1, 0);
+    int e = kbasis(r, 0);
     if (!e && hipStreamSynchronize(r->stream) != hipSuccess) e = set_error(QCS_EDEVICE, "init sync failed");
     if (e) {
         qcs_destroy(r);
@@ -256,8 +255,7 @@ int qcs_set_amplitude(qcs_register* r, uint64_t idx, double re, double im) {
 int qcs_set_basis_state(qcs_register* r, uint64_t idx) {
     QCS_REQUIRE(r, "null register");
     if (idx >= r->A) return QCS_OK;  // silent no-op (:76)
-    int e = kfill(r, 0, 0);
-    return e ? e : kset_one(r, idx, 1, 0);
+    return kbasis(r, idx);
 }
 
 int qcs_fill(qcs_register* r, double re, double im) {
@@ -429,14 +427,11 @@ static inline uint64_t range_mask(uint32_t first, uint32_t second) {
 }  // extern "C"
 
 namespace qcs {
-int measure_no_collapse_impl(qcs_register* r, int all, uint32_t first, uint32_t second, double u,
-                             uint64_t* outcome, const ShotDev* dev) {
+static int measure_no_collapse(qcs_register* r, int all, uint32_t first, uint32_t second, double u, uint64_t* outcome) {
     QCS_REQUIRE(r && outcome, "null argument");
     if (!all) QCS_REQUIRE(first <= second && second < r->n, "measured qubit range out of bounds");
-    // prob = 1 - u (QubitRegister.h:621), formed on the device
     uint64_t st = 0;
-    const int e = cdf_search(r, 1, &u, 1, 0, 0, &st, 1, dev);
-    if (e) return e;
+    if (const int e = cdf_one(r, 1. - u, 0, &st)) return e;  // prob = 1 - u (QubitRegister.h:621)
     *outcome = all ? st : (st & range_mask(first, second)) >> first;
     return QCS_OK;
 }
@@ -451,7 +446,7 @@ int sample_impl(qcs_register* r, int all, uint32_t first, uint32_t second, uint6
     if (nshots == 1) {
         // single-shot shortcut (QubitRegister.h:233-238, 335-340)
         uint64_t m = 0;
-        const int e = measure_no_collapse_impl(r, all, first, second, u[0], &m, dev);
+        const int e = measure_no_collapse(r, all, first, second, u[0], &m);
         if (e) return e;
         outcomes[0] = all ? m : (m & mask) >> shift;
         return QCS_OK;
@@ -459,12 +454,9 @@ int sample_impl(qcs_register* r, int all, uint32_t first, uint32_t second, uint6
     // truncation point: first i with cdf(i) > 1 - DBL_EPSILON (QubitRegister.h:250-253)
     const double thr = 1.0 - DBL_EPSILON;
     uint64_t t = 0;
-    int e = cdf_search(r, 1, &thr, 0, 1, r->A, &t, 1, dev);
-    if (e) return e;
-    const uint64_t len = t >= r->A ? r->A : t + 1;
     // prob = 1 - u per shot (QubitRegister.h:262), formed on the device
-    e = cdf_search(r, nshots, u, 1, 0, r->A, outcomes, 0, dev);  // the CDF just built
-    if (e) return e;
+    if (const int e = cdf_shots(r, nshots, u, thr, outcomes, &t, dev)) return e;
+    const uint64_t len = t >= r->A ? r->A : t + 1;
     for (uint64_t s = 0; s < nshots; ++s) {
         const uint64_t v = outcomes[s] < len ? outcomes[s] : len;  // lower_bound on [0, len)
         outcomes[s] = all ? v : (v & mask) >> shift;
@@ -479,12 +471,9 @@ int qcs_measure_all(qcs_register* r, double u, uint64_t* outcome) {
     QCS_REQUIRE(r && outcome, "null argument");
     const double prob = 1. - u;  // QubitRegister.h:171
     uint64_t st = 0;
-    int e = cdf_search(r, 1, &prob, 0, 0, r->A - 1, &st, 1);
-    if (e) return e;
-    e = kfill(r, 0, 0);
-    if (!e) e = kset_one(r, st, 1, 0);
+    if (const int e = cdf_one(r, prob, r->A - 1, &st)) return e;
     *outcome = st;
-    return e;
+    return kbasis(r, st);
 }
 
 int qcs_measure(qcs_register* r, uint32_t first, uint32_t second, double u, uint64_t* outcome) {
@@ -492,21 +481,14 @@ int qcs_measure(qcs_register* r, uint32_t first, uint32_t second, double u, uint
     QCS_REQUIRE(first <= second && second < r->n, "measured qubit range out of bounds");
     const double prob = 1. - u;  // QubitRegister.h:210
     uint64_t pstate = 0;
-    int e = cdf_search(r, 1, &prob, 0, 0, 0, &pstate, 1);
-    if (e) return e;
-    const uint64_t mask = range_mask(first, second);
-    const uint64_t meas = pstate & mask;
-    double accum = 0;
-    e = rsum_sq(r, first, second - first + 1, meas, &accum);
-    if (e) return e;
-    e = kcollapse(r, mask, meas, 1. / std::sqrt(accum));
-    *outcome = meas >> first;
-    return e;
+    if (const int e = rmeasure(r, first, second - first + 1, prob, &pstate)) return e;
+    *outcome = (pstate & range_mask(first, second)) >> first;
+    return QCS_OK;
 }
 
 int qcs_measure_no_collapse(qcs_register* r, int all, uint32_t first, uint32_t second, double u,
                             uint64_t* outcome) {
-    return measure_no_collapse_impl(r, all, first, second, u, outcome, nullptr);
+    return measure_no_collapse(r, all, first, second, u, outcome);
 }
 
 int qcs_sample(qcs_register* r, int all, uint32_t first, uint32_t second, uint64_t nshots, const double* u,

@@ -251,6 +251,7 @@ int kdiag_full(qcs_register* r, const double* diag_dev);
 int kfill(qcs_register* r, double re, double im);
 int kscale(qcs_register* r, double re, double im);
 int kset_one(qcs_register* r, uint64_t idx, double re, double im);
+int kbasis(qcs_register* r, uint64_t idx);
 
 // dense_kernels.hip: dense k-qubit blocks (k <= 5) on arbitrary qubits
 int kdense(qcs_register* r, uint32_t k, const uint32_t* qubits, const double* mat_host);
@@ -258,28 +259,27 @@ int kdense(qcs_register* r, uint32_t k, const uint32_t* qubits, const double* ma
 // reduce_kernels.hip (results in FP64)
 int rsum_sq(qcs_register* r, uint32_t first, uint32_t len, uint64_t val, double* out);
 int rinner(qcs_register* a, qcs_register* b, double* re_im, double* max_abs);
-// Device buffers for the shots of a CDF search: `cap` values in, `cap`
-// outcomes out. A search without them allocates its own, stream-ordered.
+// Device buffers for the shots of a sampling: `cap` values in, `cap` outcomes
+// out. Without them a few shots use the register's scratch, many their own
+// stream-ordered allocation.
 struct ShotDev {
     double* in = nullptr;
     uint64_t* out = nullptr;
     uint64_t cap = 0;
 };
-// CDF search: out[s] = first index whose cumulative probability reaches
-// prob_s (exceeds it with `strict`), or `dflt`, where prob_s = vals_host[s],
-// or 1 - vals_host[s] (computed on the device) with `one_minus`. build_cdf = 0
-// reuses the chunk CDF built by the previous search on this register, which
-// is only valid if the state has not changed since (the norms and rsum_sq
-// also use that buffer). `dev` (may be null) supplies the shot buffers.
-int cdf_search(qcs_register* r, uint64_t nshots, const double* vals_host, int one_minus, int strict,
-               uint64_t dflt, uint64_t* out_host, int build_cdf, const ShotDev* dev = nullptr);
-// qcs_measure_no_collapse / qcs_sample with the shot buffers of `dev`
-// (null: allocated per call)
-int measure_no_collapse_impl(qcs_register* r, int all, uint32_t first, uint32_t second, double u,
-                             uint64_t* outcome, const ShotDev* dev);
+// The first index whose cumulative probability reaches prob, or dflt.
+int cdf_one(qcs_register* r, double prob, uint64_t dflt, uint64_t* out_host);
+// The same for 1 - u[s] (formed on the device), dflt 2^n, and in trunc the
+// first index whose cumulative probability exceeds thr. `dev` (may be null)
+// supplies the shot buffers.
+int cdf_shots(qcs_register* r, uint64_t nshots, const double* u, double thr, uint64_t* out_host, uint64_t* trunc,
+              const ShotDev* dev);
+// The state that prob selects (0 if none), and the register collapsed onto
+// its bits first .. first + len - 1.
+int rmeasure(qcs_register* r, uint32_t first, uint32_t len, double prob, uint64_t* state);
+// qcs_sample with the shot buffers of `dev` (may be null)
 int sample_impl(qcs_register* r, int all, uint32_t first, uint32_t second, uint64_t nshots, const double* u,
                 uint64_t* outcomes, const ShotDev* dev);
-int kcollapse(qcs_register* r, uint64_t mask, uint64_t val, double scale);
 int rising(qcs_register* r, uint32_t ne, const uint32_t* ei, const uint32_t* ej,
            const double* J, const double* h, double* energy);
 

@@ -373,6 +373,12 @@ __global__ __launch_bounds__(kThreads) void k_fill(cv<T>* __restrict__ psi, uint
 }
 
 template <typename T>
+__global__ __launch_bounds__(kThreads) void k_basis(cv<T>* __restrict__ psi, uint64_t A, uint64_t idx, uint64_t boff) {
+    const uint64_t i = (uint64_t(blockIdx.x) + boff) * kThreads + threadIdx.x;
+    if (i < A) stamp<T, true>(psi + i, cv<T>{i == idx ? T(1) : T(0), T(0)});
+}
+
+template <typename T>
 __global__ __launch_bounds__(kThreads) void k_scale(cv<T>* __restrict__ psi, uint64_t A, T re, T im, uint64_t boff) {
     const uint64_t i = (uint64_t(blockIdx.x) + boff) * kThreads + threadIdx.x;
     if (i >= A) return;
@@ -739,6 +745,19 @@ int kfill(qcs_register* r, double re, double im) {
                                static_cast<float2*>(r->psi), r->A, float(re), float(im), boff);
     })
     return check_launch(r, "k_fill");
+}
+
+// Basis state idx, in one launch.
+int kbasis(qcs_register* r, uint64_t idx) {
+    QCS_CHUNKED(grid_for(r->A, kThreads), {
+        if (r->prec == QCS_COMPLEX128)
+            hipLaunchKernelGGL((k_basis<double>), dim3(g), dim3(kThreads), 0, r->stream,
+                               static_cast<double2*>(r->psi), r->A, idx, boff);
+        else
+            hipLaunchKernelGGL((k_basis<float>), dim3(g), dim3(kThreads), 0, r->stream,
+                               static_cast<float2*>(r->psi), r->A, idx, boff);
+    })
+    return check_launch(r, "k_basis");
 }
 
 int kscale(qcs_register* r, double re, double im) {

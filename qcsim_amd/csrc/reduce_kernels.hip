@@ -15,17 +15,24 @@
 #include <vector>
 
 #include <algorithm>
+#include <cstring>
 
 #include "common.h"
 
 namespace qcs {
 
-// Sum of |psi_s|^2 over s = insert_run(o, first, len) | val.
+// Sum of |psi_s|^2 over s = insert_run(o, first, len) | val. With st, val is
+// *st & val: an outcome still on the device.
+__device__ __forceinline__ uint64_t sum_val(uint64_t val, const uint64_t* __restrict__ st) {
+    return st ? *st & val : val;
+}
+
 template <typename T>
 __global__ __launch_bounds__(kRedThreads) void k_sum_sq(const cv<T>* __restrict__ psi, uint64_t norb,
-                                                        uint32_t first, uint32_t len, uint64_t val,
-                                                        double* __restrict__ partial) {
+                                                        uint32_t first, uint32_t len, uint64_t val0,
+                                                        const uint64_t* __restrict__ st, double* __restrict__ partial) {
     __shared__ double lds[4];
+    const uint64_t val = sum_val(val0, st);
     double acc = 0;
     const uint64_t stride = uint64_t(gridDim.x) * kRedThreads;
 #pragma unroll 4
@@ -43,9 +50,11 @@ constexpr uint32_t kSumBlock = 2048;
 
 template <typename T>
 __global__ __launch_bounds__(kRedThreads) void k_sum_sq_blocks(const cv<T>* __restrict__ psi, uint64_t norb,
-                                                               uint32_t first, uint32_t len, uint64_t val,
+                                                               uint32_t first, uint32_t len, uint64_t val0,
+                                                               const uint64_t* __restrict__ st,
                                                                double* __restrict__ partial, uint64_t b0) {
     __shared__ double lds[4];
+    const uint64_t val = sum_val(val0, st);
     const uint64_t blk = b0 + blockIdx.x;
     const uint64_t o0 = blk * kSumBlock + threadIdx.x;
     double acc = 0;
@@ -259,41 +268,13 @@ __global__ __launch_bounds__(1024) void k_scan_chunks(double* __restrict__ chunk
     }
 }
 
-// One block per shot. out[s] = first index i with prob <= cdf(i) (strict:
-// prob < cdf(i)), or `dflt` when the total stays below prob.
+// The first element of chunk c whose CDF value reaches prob (strict: exceeds
+// it), in every thread; `before` is the CDF up to the chunk. If rounding
+// leaves the chunk's last value short of it, the last element.
 template <typename T>
-__global__ __launch_bounds__(kScanThreads) void k_search(const cv<T>* __restrict__ psi, ChunkGeom g,
-                                                         const double* __restrict__ chunk, uint64_t nchunks,
-                                                         const double* __restrict__ probs, int one_minus,
-                                                         int strict, uint64_t dflt, uint64_t* __restrict__ out) {
-    __shared__ double lds[4];
-    __shared__ double nrm[kNrmLds];
-    __shared__ uint64_t sc;
-    __shared__ unsigned long long found;
-    const double prob = one_minus ? 1.0 - probs[blockIdx.x] : probs[blockIdx.x];
-    if (threadIdx.x == 0) {
-        // first c with chunk[c] >= prob (strict: > prob)
-        uint64_t lo = 0, hi = nchunks;
-        while (lo < hi) {
-            const uint64_t mid = (lo + hi) >> 1;
-            const double v = chunk[mid];
-            const bool ok = strict ? (v > prob) : (v >= prob);
-            if (ok) hi = mid;
-            else lo = mid + 1;
-        }
-        sc = lo;
-        found = ~0ull;
-    }
-    __syncthreads();
-    const uint64_t c = sc;
-    if (c >= nchunks) {
-        if (threadIdx.x == 0) out[blockIdx.x] = dflt;
-        return;
-    }
-    double total;
-    const uint64_t cbase = c * g.clen;
-    const double pre = chunk_thread_prefix<T>(psi, cbase, g, lds, nrm, &total);
-    double acc = (c > 0 ? chunk[c - 1] : 0.0) + pre;
+__device__ __forceinline__ uint64_t chunk_find(const double* nrm, uint64_t cbase, ChunkGeom g, double before, double pre,
+                                               double prob, int strict, unsigned long long* found) {
+    const double acc = before + pre;
     const uint64_t beg = uint64_t(threadIdx.x) * g.per;
     double run = 0;
     for (uint32_t i = 0; i < g.per; ++i) {
@@ -303,25 +284,78 @@ __global__ __launch_bounds__(kScanThreads) void k_search(const cv<T>* __restrict
         const double v = acc + run;
         const bool ok = strict ? (v > prob) : (v >= prob);
         if (ok) {
-            atomicMin(&found, (unsigned long long)(cbase + e));
+            atomicMin(found, (unsigned long long)(cbase + e));
             break;
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned long long f = found;
-        out[blockIdx.x] = (f == ~0ull) ? (cbase + g.clen - 1) : uint64_t(f);
-    }
+    const unsigned long long f = *found;
+    return f == ~0ull ? cbase + g.clen - 1 : uint64_t(f);
 }
 
+// One block per shot. out[s] = first index i with prob <= cdf(i) (strict:
+// prob < cdf(i)), or `dflt` when the total stays below prob; the probabilities
+// are probs[s] (one_minus: 1 - probs[s]), or without probs prob1. With tout
+// the last block looks for prob1 strictly and writes there. Without chunk the
+// state is one chunk, whose total the block adds up itself.
+template <typename T>
+__global__ __launch_bounds__(kScanThreads) void k_search(const cv<T>* __restrict__ psi, ChunkGeom g,
+                                                         const double* __restrict__ chunk, uint64_t nchunks,
+                                                         const double* __restrict__ probs, double prob1, int one_minus,
+                                                         int strict, uint64_t dflt, uint64_t* __restrict__ out,
+                                                         uint64_t* __restrict__ tout) {
+    __shared__ double lds[4];
+    __shared__ double nrm[kNrmLds];
+    __shared__ uint64_t sc;
+    __shared__ unsigned long long found;
+    double prob = prob1;
+    uint64_t* o = out + blockIdx.x;
+    if (tout && blockIdx.x == gridDim.x - 1) {
+        strict = 1;
+        o = tout;
+    } else if (probs) {
+        prob = one_minus ? 1.0 - probs[blockIdx.x] : probs[blockIdx.x];
+    }
+    auto reaches = [&](double v) { return strict ? v > prob : v >= prob; };
+    if (threadIdx.x == 0) {
+        // first c with chunk[c] >= prob (strict: > prob)
+        uint64_t lo = 0, hi = chunk ? nchunks : 0;
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi) >> 1;
+            if (reaches(chunk[mid])) hi = mid;
+            else lo = mid + 1;
+        }
+        sc = lo;
+        found = ~0ull;
+    }
+    __syncthreads();
+    const uint64_t c = sc;
+    if (c >= nchunks) {
+        if (threadIdx.x == 0) *o = dflt;
+        return;
+    }
+    double total;
+    const uint64_t cbase = c * g.clen;
+    const double pre = chunk_thread_prefix<T>(psi, cbase, g, lds, nrm, &total);
+    if (!chunk && !reaches(total)) {
+        if (threadIdx.x == 0) *o = dflt;
+        return;
+    }
+    const uint64_t f = chunk_find<T>(nrm, cbase, g, c > 0 ? chunk[c - 1] : 0.0, pre, prob, strict, &found);
+    if (threadIdx.x == 0) *o = f;
+}
+
+// psi[s] times 1 / sqrt(*sum) where (s & mask) == (*st & mask), else 0
 template <typename T>
 __global__ __launch_bounds__(kRedThreads) void k_collapse(cv<T>* __restrict__ psi, uint64_t A, uint64_t mask,
-                                                          uint64_t val, T scale, uint64_t boff) {
+                                                          const uint64_t* __restrict__ st,
+                                                          const double* __restrict__ sum, uint64_t boff) {
     // one amplitude per lane, one pass (no grid-stride loop)
     const uint64_t s = (uint64_t(blockIdx.x) + boff) * kRedThreads + threadIdx.x;
     if (s >= A) return;
+    const T scale = T(1. / sqrt(*sum));
     cv<T> v;
-    if ((s & mask) == val) {
+    if ((s & mask) == (*st & mask)) {
         v = ldamp<T, true>(psi + s);
         v.x *= scale;
         v.y *= scale;
@@ -330,6 +364,35 @@ __global__ __launch_bounds__(kRedThreads) void k_collapse(cv<T>* __restrict__ ps
         v.y = 0;
     }
     stamp<T, true>(psi + s, v);
+}
+
+// A measurement of a state of one chunk by one block: search, sum and
+// collapse as the separate kernels do them, in their order. What a small
+// register's measurement costs is launches and waits: 86 us in six launches
+// and three waits, 20 us in this one.
+template <typename T>
+__global__ __launch_bounds__(kScanThreads) void k_measure_one(cv<T>* __restrict__ psi, ChunkGeom g, double prob,
+                                                              uint64_t dflt, uint32_t first, uint32_t len,
+                                                              uint64_t* __restrict__ st) {
+    static_assert(kScanThreads == kRedThreads, "the sum's order is that of k_sum_sq");
+    __shared__ double lds[4];
+    __shared__ double nrm[kNrmLds];
+    __shared__ unsigned long long found;
+    if (threadIdx.x == 0) found = ~0ull;
+    double total;
+    const double pre = chunk_thread_prefix<T>(psi, 0, g, lds, nrm, &total);
+    const uint64_t f = total >= prob ? chunk_find<T>(nrm, 0, g, 0.0, pre, prob, 0, &found) : dflt;
+    const uint64_t mask = ((1ull << len) - 1) << first, val = f & mask;
+    double acc = 0;
+    for (uint64_t o = threadIdx.x; o < g.clen >> len; o += kScanThreads) acc += nrm[nrm_slot(insert_run(o, first, len) | val)];
+    (void)block_sum256(acc, lds);  // of which every thread needs the result
+    const T scale = T(1. / sqrt(((lds[0] + lds[1]) + lds[2]) + lds[3]));
+    for (uint64_t s = threadIdx.x; s < g.clen; s += kScanThreads) {
+        const cv<T> v = psi[s];
+        const bool in = (s & mask) == val;
+        psi[s] = cv<T>{in ? v.x * scale : T(0), in ? v.y * scale : T(0)};
+    }
+    if (threadIdx.x == 0) *st = f;
 }
 
 // Exact Ising energy sum_s |psi_s|^2 E(s), E(s) = -(sum h z + sum J z z).
@@ -387,8 +450,9 @@ int fetch(qcs_register* r, const double* dev, int n, double* host) {
     return QCS_OK;
 }
 
+// The sum, left in the first result slot.
 template <typename T>
-static int rsum_sq_t(qcs_register* r, uint32_t first, uint32_t len, uint64_t val, double* out) {
+static int rsum_sq_dev(qcs_register* r, uint32_t first, uint32_t len, uint64_t val, const uint64_t* st) {
     const uint64_t norb = r->A >> len;
     int nb = 0, e = 0;
     if (norb >= (uint64_t(1) << 20)) {
@@ -398,7 +462,7 @@ static int rsum_sq_t(qcs_register* r, uint32_t first, uint32_t len, uint64_t val
         for (uint64_t b0 = 0; b0 < nblk; b0 += (1ull << 22)) {
             const unsigned g = unsigned(std::min<uint64_t>(1ull << 22, nblk - b0));
             hipLaunchKernelGGL((k_sum_sq_blocks<T>), dim3(g), dim3(kRedThreads), 0, r->stream,
-                               static_cast<const cv<T>*>(r->psi), norb, first, len, val, r->chunk, b0);
+                               static_cast<const cv<T>*>(r->psi), norb, first, len, val, st, r->chunk, b0);
             if ((e = check_launch(r, "k_sum_sq_blocks"))) return e;
         }
         nb = red_blocks(nblk);
@@ -407,19 +471,18 @@ static int rsum_sq_t(qcs_register* r, uint32_t first, uint32_t len, uint64_t val
     } else {
         nb = red_blocks(norb);
         hipLaunchKernelGGL((k_sum_sq<T>), dim3(nb), dim3(kRedThreads), 0, r->stream,
-                           static_cast<const cv<T>*>(r->psi), norb, first, len, val, r->red);
+                           static_cast<const cv<T>*>(r->psi), norb, first, len, val, st, r->red);
         if ((e = check_launch(r, "k_sum_sq"))) return e;
     }
     double* res = r->red + kRedResult;
     hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kRedThreads), 0, r->stream, r->red, nb, 1, res);
-    e = check_launch(r, "k_final_sum");
-    if (e) return e;
-    return fetch(r, res, 1, out);
+    return check_launch(r, "k_final_sum");
 }
 
 int rsum_sq(qcs_register* r, uint32_t first, uint32_t len, uint64_t val, double* out) {
-    return r->prec == QCS_COMPLEX128 ? rsum_sq_t<double>(r, first, len, val, out)
-                                     : rsum_sq_t<float>(r, first, len, val, out);
+    const int e = r->prec == QCS_COMPLEX128 ? rsum_sq_dev<double>(r, first, len, val, nullptr)
+                                            : rsum_sq_dev<float>(r, first, len, val, nullptr);
+    return e ? e : fetch(r, r->red + kRedResult, 1, out);
 }
 
 template <typename Ta, typename Tb>
@@ -461,95 +524,149 @@ static ChunkGeom chunk_geom(const qcs_register* r) {
     return g;
 }
 
+// The CDF at the chunks' ends; nothing to do for a state of one chunk.
 template <typename T>
-static int cdf_search_t(qcs_register* r, uint64_t nshots, const double* vals_host, int one_minus, int strict,
-                        uint64_t dflt, uint64_t* out_host, bool build, const ShotDev* dev) {
-    const ChunkGeom g = chunk_geom(r);
+static int cdf_build(qcs_register* r, const ChunkGeom& g) {
     const uint64_t nchunks = r->A / g.clen;
-    const auto* psi = static_cast<const cv<T>*>(r->psi);
+    if (nchunks == 1) return QCS_OK;
     // at most 2^22 chunks (2^30 work-items) per launch: a grid's size in
     // work-items must stay below 2^32
     int e = 0;
-    for (uint64_t c0 = 0; build && c0 < nchunks; c0 += (1ull << 22)) {
+    for (uint64_t c0 = 0; c0 < nchunks; c0 += (1ull << 22)) {
         const uint64_t cnt = std::min<uint64_t>(1ull << 22, nchunks - c0);
-        hipLaunchKernelGGL((k_chunk_sums<T>), dim3(unsigned(cnt)), dim3(kScanThreads), 0, r->stream, psi, g,
-                           r->chunk, c0);
-        e = check_launch(r, "k_chunk_sums");
-        if (e) return e;
+        hipLaunchKernelGGL((k_chunk_sums<T>), dim3(unsigned(cnt)), dim3(kScanThreads), 0, r->stream,
+                           static_cast<const cv<T>*>(r->psi), g, r->chunk, c0);
+        if ((e = check_launch(r, "k_chunk_sums"))) return e;
     }
     // group totals live after the chunk totals (the buffer holds both)
     const uint64_t ngroups = (nchunks + kScanGroup - 1) / kScanGroup;
     double* grp = r->chunk + nchunks;
-    if (build) {
-        hipLaunchKernelGGL(k_scan_group, dim3(unsigned(ngroups)), dim3(kScanThreads), 0, r->stream, r->chunk,
-                           nchunks, grp);
-        e = check_launch(r, "k_scan_group");
-        if (e) return e;
-    }
-    if (build && ngroups > 1) {
+    hipLaunchKernelGGL(k_scan_group, dim3(unsigned(ngroups)), dim3(kScanThreads), 0, r->stream, r->chunk, nchunks, grp);
+    if ((e = check_launch(r, "k_scan_group"))) return e;
+    if (ngroups > 1) {
         hipLaunchKernelGGL(k_scan_chunks, dim3(1), dim3(1024), 0, r->stream, grp, ngroups);
-        e = check_launch(r, "k_scan_chunks");
-        if (e) return e;
+        if ((e = check_launch(r, "k_scan_chunks"))) return e;
         const uint64_t nadd = nchunks - kScanGroup;
         hipLaunchKernelGGL(k_add_group_offsets, dim3(unsigned((nadd + kScanThreads - 1) / kScanThreads)),
                            dim3(kScanThreads), 0, r->stream, r->chunk, nchunks, grp);
-        e = check_launch(r, "k_add_group_offsets");
-        if (e) return e;
+        if ((e = check_launch(r, "k_add_group_offsets"))) return e;
     }
-    // per-shot buffers: the caller's, or stream-ordered allocations
-    double* dvals = nullptr;
+    return QCS_OK;
+}
+
+template <typename T>
+static int search_launch(qcs_register* r, const ChunkGeom& g, uint64_t cnt, const double* probs, double prob1,
+                         uint64_t dflt, uint64_t* out, uint64_t* tout) {
+    const uint64_t nchunks = r->A / g.clen;
+    hipLaunchKernelGGL((k_search<T>), dim3(unsigned(cnt + (tout ? 1 : 0))), dim3(kScanThreads), 0, r->stream,
+                       static_cast<const cv<T>*>(r->psi), g, nchunks > 1 ? r->chunk : nullptr, nchunks, probs, prob1, 1, 0,
+                       dflt, out, tout);
+    return check_launch(r, "k_search");
+}
+
+template <typename T>
+static int cdf_one_t(qcs_register* r, double prob, uint64_t dflt, uint64_t* out_host) {
+    const ChunkGeom g = chunk_geom(r);
+    int e = cdf_build<T>(r, g);
+    if (!e) e = search_launch<T>(r, g, 1, nullptr, prob, dflt, r->dout, nullptr);
+    if (e) return e;
+    if (hipMemcpyAsync(r->hpin, r->dout, sizeof(uint64_t), hipMemcpyDeviceToHost, r->stream) != hipSuccess ||
+        hipStreamSynchronize(r->stream) != hipSuccess)
+        return set_error(QCS_EDEVICE, "cdf search sync failed");
+    std::memcpy(out_host, r->hpin, sizeof(uint64_t));
+    return QCS_OK;
+}
+
+int cdf_one(qcs_register* r, double prob, uint64_t dflt, uint64_t* out_host) {
+    return r->prec == QCS_COMPLEX128 ? cdf_one_t<double>(r, prob, dflt, out_host)
+                                     : cdf_one_t<float>(r, prob, dflt, out_host);
+}
+
+template <typename T>
+static int cdf_shots_t(qcs_register* r, uint64_t nshots, const double* u, double thr, uint64_t* out_host,
+                       uint64_t* trunc, const ShotDev* dev) {
+    const ChunkGeom g = chunk_geom(r);
+    if (const int e = cdf_build<T>(r, g)) return e;
+    // per-shot buffers: the caller's; for few shots the staging ring and the
+    // reduction scratch, free during a search; else stream-ordered allocations
+    int e = 0;
+    const size_t bytes = sizeof(double) * nshots;
+    const double* dvals = nullptr;
     uint64_t* douts = nullptr;
+    double* own = nullptr;
     if (dev) {
         if (nshots > dev->cap) return set_error(QCS_EINVAL, "%llu shots exceed the buffer of %llu",
                                                 (unsigned long long)nshots, (unsigned long long)dev->cap);
         dvals = dev->in;
         douts = dev->out;
-    } else if (hipMallocAsync(reinterpret_cast<void**>(&dvals), sizeof(double) * nshots, r->stream) != hipSuccess ||
-               hipMallocAsync(reinterpret_cast<void**>(&douts), sizeof(uint64_t) * nshots, r->stream) != hipSuccess) {
-        return set_error(QCS_ENOMEM, "shot buffers");
+    } else if (bytes <= r->mat_bytes) {
+        static_assert(sizeof(uint64_t) == sizeof(double), "outcomes in the reduction scratch");
+        const void* p = nullptr;
+        if ((e = stage_upload(r, u, bytes, &p))) return e;
+        dvals = static_cast<const double*>(p);
+        douts = reinterpret_cast<uint64_t*>(r->red);
+    } else {
+        if (hipMallocAsync(reinterpret_cast<void**>(&own), 2 * bytes, r->stream) != hipSuccess)
+            return set_error(QCS_ENOMEM, "shot buffers");
+        dvals = own;
+        douts = reinterpret_cast<uint64_t*>(own + nshots);
     }
-    if (hipMemcpyAsync(dvals, vals_host, sizeof(double) * nshots, hipMemcpyHostToDevice, r->stream) != hipSuccess)
+    if ((dev || own) && hipMemcpyAsync(const_cast<double*>(dvals), u, bytes, hipMemcpyHostToDevice, r->stream) != hipSuccess)
         e = set_error(QCS_EDEVICE, "shot upload failed");
     for (uint64_t s0 = 0; s0 < nshots && !e; s0 += 65535) {
         const uint64_t cnt = nshots - s0 < 65535 ? nshots - s0 : 65535;
-        hipLaunchKernelGGL((k_search<T>), dim3(unsigned(cnt)), dim3(kScanThreads), 0, r->stream, psi, g, r->chunk,
-                           nchunks, dvals + s0, one_minus, strict, dflt, douts + s0);
-        e = check_launch(r, "k_search");
+        e = search_launch<T>(r, g, cnt, dvals + s0, thr, r->A, douts + s0, s0 ? nullptr : r->dout);
     }
-    if (!e && hipMemcpyAsync(out_host, douts, sizeof(uint64_t) * nshots, hipMemcpyDeviceToHost, r->stream) !=
-                  hipSuccess)
+    if (!e && (hipMemcpyAsync(out_host, douts, sizeof(uint64_t) * nshots, hipMemcpyDeviceToHost, r->stream) !=
+                   hipSuccess ||
+               hipMemcpyAsync(r->hpin, r->dout, sizeof(uint64_t), hipMemcpyDeviceToHost, r->stream) != hipSuccess))
         e = set_error(QCS_EDEVICE, "shot download failed");
-    if (!dev) {
-        (void)hipFreeAsync(dvals, r->stream);
-        (void)hipFreeAsync(douts, r->stream);
-    }
+    if (own) (void)hipFreeAsync(own, r->stream);
     if (hipStreamSynchronize(r->stream) != hipSuccess && !e) e = set_error(QCS_EDEVICE, "cdf search sync failed");
+    std::memcpy(trunc, r->hpin, sizeof(uint64_t));
     return e;
 }
 
-int cdf_search(qcs_register* r, uint64_t nshots, const double* vals_host, int one_minus, int strict, uint64_t dflt,
-               uint64_t* out_host, int build_cdf, const ShotDev* dev) {
-    if (nshots == 0) return QCS_OK;
-    return r->prec == QCS_COMPLEX128
-               ? cdf_search_t<double>(r, nshots, vals_host, one_minus, strict, dflt, out_host, build_cdf, dev)
-               : cdf_search_t<float>(r, nshots, vals_host, one_minus, strict, dflt, out_host, build_cdf, dev);
+int cdf_shots(qcs_register* r, uint64_t nshots, const double* u, double thr, uint64_t* out_host, uint64_t* trunc,
+              const ShotDev* dev) {
+    return r->prec == QCS_COMPLEX128 ? cdf_shots_t<double>(r, nshots, u, thr, out_host, trunc, dev)
+                                     : cdf_shots_t<float>(r, nshots, u, thr, out_host, trunc, dev);
 }
 
-int kcollapse(qcs_register* r, uint64_t mask, uint64_t val, double scale) {
-    // at most 2^22 blocks (2^30 work-items) per launch: a grid's size in
-    // work-items must stay below 2^32
-    const uint64_t nblk = (r->A + kRedThreads - 1) / kRedThreads;
-    for (uint64_t boff = 0; boff < nblk; boff += (1ull << 22)) {
-        const unsigned g = unsigned(std::min<uint64_t>(1ull << 22, nblk - boff));
-        if (r->prec == QCS_COMPLEX128)
-            hipLaunchKernelGGL((k_collapse<double>), dim3(g), dim3(kRedThreads), 0, r->stream,
-                               static_cast<double2*>(r->psi), r->A, mask, val, scale, boff);
-        else
-            hipLaunchKernelGGL((k_collapse<float>), dim3(g), dim3(kRedThreads), 0, r->stream,
-                               static_cast<float2*>(r->psi), r->A, mask, val, float(scale), boff);
-        if (const int e = check_launch(r, "k_collapse")) return e;
+template <typename T>
+static int measure_t(qcs_register* r, uint32_t first, uint32_t len, double prob, uint64_t* state) {
+    const ChunkGeom g = chunk_geom(r);
+    const uint64_t mask = (len < 64 ? (1ull << len) - 1 : ~0ull) << first;
+    int e = 0;
+    if (g.clen == r->A) {
+        hipLaunchKernelGGL((k_measure_one<T>), dim3(1), dim3(kScanThreads), 0, r->stream, static_cast<cv<T>*>(r->psi), g,
+                           prob, uint64_t(0), first, len, r->dout);
+        e = check_launch(r, "k_measure_one");
+    } else {
+        e = cdf_build<T>(r, g);
+        if (!e) e = search_launch<T>(r, g, 1, nullptr, prob, 0, r->dout, nullptr);
+        if (!e) e = rsum_sq_dev<T>(r, first, len, mask, r->dout);
+        // at most 2^22 blocks (2^30 work-items) per launch: a grid's size in
+        // work-items must stay below 2^32
+        const uint64_t nblk = (r->A + kRedThreads - 1) / kRedThreads;
+        for (uint64_t boff = 0; boff < nblk && !e; boff += (1ull << 22)) {
+            const unsigned gr = unsigned(std::min<uint64_t>(1ull << 22, nblk - boff));
+            hipLaunchKernelGGL((k_collapse<T>), dim3(gr), dim3(kRedThreads), 0, r->stream, static_cast<cv<T>*>(r->psi),
+                               r->A, mask, r->dout, r->red + kRedResult, boff);
+            e = check_launch(r, "k_collapse");
+        }
     }
+    if (e) return e;
+    if (hipMemcpyAsync(r->hpin, r->dout, sizeof(uint64_t), hipMemcpyDeviceToHost, r->stream) != hipSuccess ||
+        hipStreamSynchronize(r->stream) != hipSuccess)
+        return set_error(QCS_EDEVICE, "measurement sync failed");
+    std::memcpy(state, r->hpin, sizeof(uint64_t));
     return QCS_OK;
+}
+
+int rmeasure(qcs_register* r, uint32_t first, uint32_t len, double prob, uint64_t* state) {
+    return r->prec == QCS_COMPLEX128 ? measure_t<double>(r, first, len, prob, state)
+                                     : measure_t<float>(r, first, len, prob, state);
 }
 
 template <typename T>
