@@ -3,7 +3,7 @@
 // The reference builds QFT/IQFT from Hadamards, controlled phase shifts and a
 // SWAP network (QuantumFourierTransform.h:35-87, QubitsSwapper.h:23-33): at
 // n = 30 that is 480 full passes over the state. Here the same operator is
-// applied in about (n - 12)/6 + 2 passes (5 at n = 30):
+// applied in about (n - 12)/9 + 2 passes (4 at n = 22 to 30):
 //
 //   The controlled phase shifts between target `cur` and every control below
 //   it (phase pi/2, pi/4, ... for distance 1, 2, ...) multiply to one
@@ -12,11 +12,12 @@
 //   H(eq), D_eq, H(eq-1), D_(eq-1), ..., D_(sq+1), H(sq) and the inverse is
 //   H(sq), D*_(sq+1), H(sq+1), ..., D*_eq, H(eq) (after the swaps).
 //
-//   k_qft_group applies that sequence for up to 4 consecutive targets at once
-//   with the 2^4 amplitudes of each orbit in registers, k_qft_gpair for 5 or
-//   6 with each orbit split over a lane pair; k_qft_lds applies it for all
-//   targets below 12 inside 4096-amplitude chunks staged in LDS, in rounds
-//   of up to 3 targets held in registers; the
+//   k_qft_lds applies that sequence for all targets below 12 inside
+//   4096-amplitude chunks staged in LDS, and for up to 9 higher ones in tiles
+//   of as many amplitudes, in rounds of up to 3 targets held in registers;
+//   k_qft_group for up to 4 targets with the 2^4 amplitudes of each orbit in
+//   registers, k_qft_gpair for 5 or 6 with each orbit split over a lane pair
+//   (where they are no slower, and for a capped group width); the
 //   SWAP network is one bit-reversal pass (k_bitrev_tile, LDS-tiled, or
 //   k_bitrev_pairs when runs of >= 8 amplitudes stay contiguous).
 //
@@ -478,65 +479,90 @@ __device__ __forceinline__ void round_orbit(cv<T>* x, uint64_t base, const QftAr
     }
 }
 
-template <typename T, int G, bool INV>
-__device__ void lds_round(cv<T>* s, uint64_t cbase, uint32_t clog, const QftArgs& a, const double2* __restrict__ tw,
-                          const QftRoots& R) {
+// A tile of 2^clog amplitudes: the lowest `low` qubits and the ones from `at`
+// on; or a contiguous chunk (low = at = clog).
+struct QftTile {
+    uint32_t clog, low, at;
+};
+
+// global index of tile element i, but for the bits outside the tile
+template <bool CHUNK>
+__device__ __forceinline__ uint64_t tile_index(uint32_t i, const QftTile& t) {
+    if constexpr (CHUNK) return i;
+    return (i & ((1u << t.low) - 1)) | uint64_t(i >> t.low) << t.at;
+}
+
+// The round on targets a.lo .. a.lo+G-1, at tile bits l .. l+G-1.
+template <typename T, int G, bool INV, bool CHUNK>
+__device__ void lds_round(cv<T>* s, uint64_t base, const QftTile& t, uint32_t l, const QftArgs& a,
+                          const double2* __restrict__ tw, const QftRoots& R) {
     constexpr int D = 1 << G;
-    const uint32_t norb = 1u << (clog - G);
+    const uint32_t norb = 1u << (t.clog - G);
     for (uint32_t o = threadIdx.x; o < norb; o += kLdsThreads) {
-        const uint32_t lb = uint32_t(insert_run(o, a.lo, G));
+        const uint32_t lb = uint32_t(insert_run(o, l, G));
         cv<T> x[D];
 #pragma unroll
-        for (int c = 0; c < D; ++c) x[c] = s[swz(lb + (uint32_t(c) << a.lo))];
-        round_orbit<T, G, INV>(x, cbase | lb, a, tw, R);
+        for (int c = 0; c < D; ++c) x[c] = s[swz(lb + (uint32_t(c) << l))];
+        round_orbit<T, G, INV>(x, base | tile_index<CHUNK>(lb, t), a, tw, R);
 #pragma unroll
-        for (int c = 0; c < D; ++c) s[swz(lb + (uint32_t(c) << a.lo))] = x[c];
+        for (int c = 0; c < D; ++c) s[swz(lb + (uint32_t(c) << l))] = x[c];
     }
 }
 
-template <typename T, bool INV>
-__device__ void lds_round_g(cv<T>* s, uint64_t cbase, uint32_t clog, const QftArgs& a, const double2* tw,
+template <typename T, bool INV, bool CHUNK>
+__device__ void lds_round_g(cv<T>* s, uint64_t base, const QftTile& t, uint32_t l, const QftArgs& a, const double2* tw,
                             const QftRoots& R) {
     static_assert(kLdsRound <= 3, "rounds of at most 3 targets");
     switch (a.g) {
-        case 1: lds_round<T, 1, INV>(s, cbase, clog, a, tw, R); break;
-        case 2: lds_round<T, 2, INV>(s, cbase, clog, a, tw, R); break;
-        default: lds_round<T, 3, INV>(s, cbase, clog, a, tw, R); break;
+        case 1: lds_round<T, 1, INV, CHUNK>(s, base, t, l, a, tw, R); break;
+        case 2: lds_round<T, 2, INV, CHUNK>(s, base, t, l, a, tw, R); break;
+        default: lds_round<T, 3, INV, CHUNK>(s, base, t, l, a, tw, R); break;
     }
 }
 
-// Targets sq..hi (hi < clog <= kLdsLog) inside contiguous chunks of 2^clog
-// amplitudes staged in LDS, in rounds of up to kLdsRound consecutive targets
-// (from the top down for the QFT, from sq up for its inverse); one LDS round
-// trip per round instead of one per target. One chunk per block (one-shot
-// grid, in launches of at most kMaxBlocks blocks from chunk boff).
-template <typename T, bool INV>
-__global__ __launch_bounds__(kLdsThreads) void k_qft_lds(cv<T>* __restrict__ psi, uint32_t clog, uint64_t boff, QftArgs a,
-                                                 uint32_t hi, const double2* __restrict__ tw, const QftRoots R) {
+// Targets a.lo .. a.lo+a.g-1, which are tile bits, on tiles staged in LDS, in
+// rounds of up to kLdsRound consecutive targets (from the top down for the
+// QFT, from the lowest up for its inverse); one LDS round trip per round
+// instead of one per target. One tile per block (one-shot grid, in launches
+// of at most kMaxBlocks blocks from tile boff).
+//
+// The lowest targets come in contiguous chunks of 2^12 amplitudes, the others
+// five to nine a tile (complex64: to eight) with the lowest qubits, whole
+// memory lines. Two such passes took the place of three in registers at 25 to
+// 29 qubits: a transform of 29 qubits complex128 16.9 ms, now 13.8 ms, of 20
+// qubits (one for two) 49 us, now 35 us. A pass is bound by HBM: 3.3 ms for
+// the 16 GiB it moves at 29 qubits, a copy's rate.
+template <typename T, bool INV, bool CHUNK>
+__global__ __launch_bounds__(kLdsThreads) void k_qft_lds(cv<T>* __restrict__ psi, QftTile t, uint64_t boff, QftArgs a,
+                                                 const double2* __restrict__ tw, const QftRoots R) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     cv<T>* s = reinterpret_cast<cv<T>*>(smem_raw);
-    constexpr int EPT = (1 << kLdsLog) / kLdsThreads;  // chunk elements per thread
-    const uint32_t C = 1u << clog;
-    const uint64_t cbase = (boff + blockIdx.x) << clog;
-    // Forward, full chunk, the top round on the chunk's top 3 bits: a
-    // thread's 8 loaded elements tid + 512 k are one orbit of those bits, so
-    // that round runs in registers before the tile goes to LDS (one LDS round
-    // trip fewer).
+    constexpr int EPT = (1 << kLdsLog) / kLdsThreads;  // tile elements per thread
+    const uint32_t C = 1u << t.clog, off = CHUNK ? 0 : t.at - t.low;  // a target q is tile bit q - off
+    const uint64_t blk = boff + blockIdx.x;
+    const uint64_t base =
+        CHUNK ? blk << t.clog : (blk & ((1ull << off) - 1)) << t.low | blk >> off << (t.clog + off);
+    const uint32_t l0 = a.lo - off, l1 = l0 + a.g - 1;  // first and last target's tile bits
+    // Forward, full tile, the top round on the tile's top 3 bits: a thread's
+    // 8 loaded elements tid + 512 k are one orbit of those bits, so that round
+    // runs in registers before the tile goes to LDS (one LDS round trip
+    // fewer).
     static_assert(EPT == 8 && kLdsRound == 3, "the loaded elements are one 3-target orbit");
-    const bool reg_top = !INV && clog == uint32_t(kLdsLog) && hi == clog - 1 && hi >= a.sq + 2;
+    const bool reg_top = !INV && t.clog == uint32_t(kLdsLog) && l1 == t.clog - 1 && a.g >= kLdsRound;
+    auto round = [&](uint32_t lo, uint32_t g) {
+        QftArgs r = a;
+        r.lo = a.lo + (lo - l0);
+        r.g = g;
+        return r;
+    };
     {
         cv<T> v[EPT];
 #pragma unroll
         for (int k = 0; k < EPT; ++k) {
             const uint32_t i = threadIdx.x + uint32_t(kLdsThreads) * k;
-            if (i < C) v[k] = ldamp<T, kStagedNtLoads>(psi + cbase + i);
+            if (i < C) v[k] = ldamp<T, kStagedNtLoads>(psi + (base | tile_index<CHUNK>(i, t)));
         }
-        if (reg_top) {
-            QftArgs r = a;
-            r.lo = hi - 2;
-            r.g = 3;
-            round_orbit<T, 3, false>(v, cbase | threadIdx.x, r, tw, R);
-        }
+        if (reg_top) round_orbit<T, 3, false>(v, base | tile_index<CHUNK>(threadIdx.x, t), round(l1 - 2, 3), tw, R);
 #pragma unroll
         for (int k = 0; k < EPT; ++k) {
             const uint32_t i = threadIdx.x + uint32_t(kLdsThreads) * k;
@@ -545,24 +571,21 @@ __global__ __launch_bounds__(kLdsThreads) void k_qft_lds(cv<T>* __restrict__ psi
         __syncthreads();
     }
     if (!INV) {
-        for (int top = int(hi) - (reg_top ? kLdsRound : 0); top >= int(a.sq); top -= kLdsRound) {
-            QftArgs r = a;
-            r.lo = uint32_t(top - (kLdsRound - 1) > int(a.sq) ? top - (kLdsRound - 1) : int(a.sq));
-            r.g = uint32_t(top) - r.lo + 1;
-            lds_round_g<T, false>(s, cbase, clog, r, tw, R);
+        for (int top = int(l1) - (reg_top ? kLdsRound : 0); top >= int(l0); top -= kLdsRound) {
+            const uint32_t lo = uint32_t(top - (kLdsRound - 1) > int(l0) ? top - (kLdsRound - 1) : int(l0));
+            lds_round_g<T, false, CHUNK>(s, base, t, lo, round(lo, uint32_t(top) - lo + 1), tw, R);
             __syncthreads();
         }
     } else {
-        for (uint32_t lo = a.sq; lo <= hi; lo += kLdsRound) {
-            QftArgs r = a;
-            r.lo = lo;
-            r.g = hi - lo + 1 < uint32_t(kLdsRound) ? hi - lo + 1 : uint32_t(kLdsRound);
-            lds_round_g<T, true>(s, cbase, clog, r, tw, R);
+        for (uint32_t lo = l0; lo <= l1; lo += kLdsRound) {
+            const uint32_t g = l1 - lo + 1 < uint32_t(kLdsRound) ? l1 - lo + 1 : uint32_t(kLdsRound);
+            lds_round_g<T, true, CHUNK>(s, base, t, lo, round(lo, g), tw, R);
             __syncthreads();
         }
     }
-    const T hs = hscale<T>(hi - a.sq + 1);
-    for (uint32_t i = threadIdx.x; i < C; i += kLdsThreads) stamp<T, true>(psi + cbase + i, scaled<T>(s[swz(i)], hs));
+    const T hs = hscale<T>(a.g);
+    for (uint32_t i = threadIdx.x; i < C; i += kLdsThreads)
+        stamp<T, true>(psi + (base | tile_index<CHUNK>(i, t)), scaled<T>(s[swz(i)], hs));
 }
 
 // ---- bit reversal of the range [sq, eq] ---------------------------------------
@@ -728,22 +751,25 @@ static int launch_group(qcs_register* r, const double2* tw, uint32_t sq, uint32_
     return check_launch(r, "k_qft_group");
 }
 
+// Targets lo .. lo+g-1 of the range in tiles.
 template <typename T>
-static int launch_lds(qcs_register* r, const double2* tw, uint32_t sq, uint32_t eq, uint32_t hi, uint32_t clog,
-                      bool inv) {
-    const QftArgs a{sq, eq, sq, hi - sq + 1};
-    const uint64_t nchunks = r->A >> clog;
-    const size_t shm = sizeof(cv<T>) << clog;
+static int launch_lds(qcs_register* r, const double2* tw, const QftTile& t, const QftArgs& a, bool inv) {
+    const uint64_t tiles = r->A >> t.clog;
+    const size_t shm = sizeof(cv<T>) << t.clog;
     auto* psi = static_cast<cv<T>*>(r->psi);
     static const QftRoots roots = group_roots();
-    for (uint64_t boff = 0; boff < nchunks; boff += kMaxBlocks) {
-        const unsigned g = unsigned(std::min<uint64_t>(kMaxBlocks, nchunks - boff));
-        if (inv)
-            hipLaunchKernelGGL((k_qft_lds<T, true>), dim3(g), dim3(kLdsThreads), shm, r->stream, psi, clog, boff, a, hi, tw,
-                               roots);
-        else
-            hipLaunchKernelGGL((k_qft_lds<T, false>), dim3(g), dim3(kLdsThreads), shm, r->stream, psi, clog, boff, a, hi, tw,
-                               roots);
+    for (uint64_t boff = 0; boff < tiles; boff += kMaxBlocks) {
+        const unsigned g = unsigned(std::min<uint64_t>(kMaxBlocks, tiles - boff));
+#define QCS_LDS(II, CC) \
+    hipLaunchKernelGGL((k_qft_lds<T, II, CC>), dim3(g), dim3(kLdsThreads), shm, r->stream, psi, t, boff, a, tw, roots)
+        if (t.low == t.at) {
+            if (inv) QCS_LDS(true, true);
+            else QCS_LDS(false, true);
+        } else {
+            if (inv) QCS_LDS(true, false);
+            else QCS_LDS(false, false);
+        }
+#undef QCS_LDS
     }
     return check_launch(r, "k_qft_lds");
 }
@@ -789,31 +815,59 @@ static int qft_fused(qcs_register* r, uint32_t sq, uint32_t eq, int do_swap, int
     const uint32_t clog = r->n < uint32_t(kLdsLog) ? r->n : uint32_t(kLdsLog);
     const bool use_lds = sq < clog && (eq - sq + 1) >= 2;
     const uint32_t lds_hi = use_lds ? (eq < clog - 1 ? eq : clog - 1) : sq - 1;
-    // register groups over (lds_hi, eq], in blocks of <= gmax from the top
-    // (QCS_QFT_GROUP overrides the widest group, 1..6)
+    // The targets above, in as few passes as nine (complex64: eight) targets a
+    // tile allow, the narrower passes on top: at 29 qubits complex128 eight
+    // targets from 21 on and nine from 12 on take 3.6 and 3.5 ms, but nine from
+    // 20 on, 512 runs of 128 B 16 MiB apart, 5.7 ms. Register groups remain
+    // where they are no slower: up to four targets (16 qubits: 18.5 us against
+    // 18.8) and ten or eleven, in two passes either way (23 qubits: 212 us
+    // against 221). QCS_QFT_GROUP (1..6) has groups of at most that width
+    // throughout.
     static const int gmax = [] {
         const char* v = std::getenv("QCS_QFT_GROUP");
-        const int g = v ? std::atoi(v) : kGroupMax;
-        return g >= 1 && g <= kGroupMax ? g : kGroupMax;
+        const int g = v ? std::atoi(v) : 0;
+        return g >= 1 && g <= kGroupMax ? g : 0;
     }();
-    std::vector<std::pair<uint32_t, uint32_t>> groups;  // (lo, g)
+    constexpr uint32_t kTileTargets = sizeof(T) == 8 ? 9 : 8, kRegTargets = 4;
+    struct Group {
+        uint32_t lo, g;
+        bool tiled;
+    };
+    std::vector<Group> groups;  // from the top
     const uint32_t first = use_lds ? lds_hi + 1 : sq;
+    const bool tiles = !gmax && first >= uint32_t(kLdsLog);
     for (int64_t hi = eq; hi >= int64_t(first);) {
-        const uint32_t g = uint32_t(std::min<int64_t>(gmax, hi - int64_t(first) + 1));
-        groups.push_back({uint32_t(hi) - g + 1, g});
+        const uint32_t rest = uint32_t(hi - int64_t(first) + 1);
+        uint32_t g = std::min<uint32_t>(rest, uint32_t(gmax ? gmax : kGroupMax));
+        bool tiled = false;
+        if (tiles && rest > kRegTargets && rest != 10 && rest != 11) {
+            const uint32_t passes = (rest + kTileTargets - 1) / kTileTargets;
+            g = rest / passes;
+            tiled = true;
+        }
+        groups.push_back({uint32_t(hi) - g + 1, g, tiled});
         hi -= g;
     }
+    auto chunks = [&](bool inv) {
+        return launch_lds<T>(r, tw, QftTile{clog, clog, clog}, QftArgs{sq, eq, sq, lds_hi - sq + 1}, inv);
+    };
+    auto group = [&](const Group& G, bool inv) {
+        if (G.tiled)
+            return launch_lds<T>(r, tw, QftTile{uint32_t(kLdsLog), uint32_t(kLdsLog) - G.g, G.lo},
+                                 QftArgs{sq, eq, G.lo, G.g}, inv);
+        return launch_group<T>(r, tw, sq, eq, G.lo, G.g, inv);
+    };
     int e = QCS_OK;
     if (!inverse) {
         for (const auto& gr : groups)
-            if ((e = launch_group<T>(r, tw, sq, eq, gr.first, gr.second, false))) return e;
-        if (use_lds && (e = launch_lds<T>(r, tw, sq, eq, lds_hi, clog, false))) return e;
+            if ((e = group(gr, false))) return e;
+        if (use_lds && (e = chunks(false))) return e;
         if (do_swap && (e = bitrev<T>(r, sq, eq))) return e;
     } else {
         if (do_swap && (e = bitrev<T>(r, sq, eq))) return e;
-        if (use_lds && (e = launch_lds<T>(r, tw, sq, eq, lds_hi, clog, true))) return e;
+        if (use_lds && (e = chunks(true))) return e;
         for (auto it = groups.rbegin(); it != groups.rend(); ++it)
-            if ((e = launch_group<T>(r, tw, sq, eq, it->first, it->second, true))) return e;
+            if ((e = group(*it, true))) return e;
     }
     return QCS_OK;
 }
