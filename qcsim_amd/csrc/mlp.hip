@@ -20,7 +20,7 @@
 // loss and the whole backward pass with the activations in LDS; k_mlp_dw
 // then sums every layer's weight and bias gradients over the batch and
 // applies Adam in its epilogue. Measured on MI355X (17 -> 256 x 3 -> 1,
-// batch 4096): 86 us a step, against 5.4 ms for GEMMs and column sums that put
+// batch 4096): 70 us a step, against 5.4 ms for GEMMs and column sums that put
 // one block of 256 threads, or 16 blocks, on a sum over the batch.
 #include <algorithm>
 #include <cmath>
@@ -405,16 +405,12 @@ __global__ __launch_bounds__(64 * NW) void k_mlp_rows(MlpRows a) {
     }
 }
 
-// Adam on one FP32 master weight; returns the new value.
-__device__ __forceinline__ float adam_step(float* w, float* m, float* v, size_t i, float gi, float lr, float b1,
-                                           float b2, float eps, float c1, float c2) {
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    w[i] = wi;
-    return wi;
+// Adam on one FP32 master weight and its moments.
+__device__ __forceinline__ void adam_step(float& w, float& m, float& v, float gi, float lr, float b1, float b2,
+                                          float eps, float c1, float c2) {
+    m = b1 * m + (1.f - b1) * gi;
+    v = b2 * v + (1.f - b2) * gi * gi;
+    w = w - lr * (m / c1) / (sqrtf(v / c2) + eps);
 }
 
 struct DwLayer {
@@ -444,26 +440,32 @@ struct DwArgs {
 // that row the bias gradient. A block owns 32 x 32 outputs, a wave one 16 x
 // 16 tile: one FMA chain per output over the whole batch is what the order
 // asks for, so the time is the chain (18 ns per 4 rows, 19 us for 4096) and
-// one tile per wave spreads the layers over the most CUs. Slabs of 256 rows
-// are staged in LDS while the slab before them is multiplied. The last block
-// adds the loss terms. Measured (17 -> 256 x 3 -> 1, 4096 rows): 46 us; with
-// operands read from LDS one matrix instruction ahead and branches around the
-// loads 75 us.
-__global__ __launch_bounds__(256) void k_mlp_dw(DwArgs a) {
-    constexpr int KS = 256, LA = 32, LZ = 48;  // strides that put the four k of an operand in different banks
-    __shared__ __attribute__((aligned(16))) float Zs[KS * LZ];
-    __shared__ __attribute__((aligned(16))) bf16 As[KS * LA];
-    const int tid = threadIdx.x;
+// one tile per wave spreads the layers over the most CUs. Four waves multiply;
+// four others bring slabs of 192 rows to LDS meanwhile, three ahead, one
+// barrier a slab. Each matrix instruction keeps the next one of the chain
+// waiting, and in that time one of the reads and conversions for later ones is
+// issued. The last block adds the loss terms. Measured (17 -> 256 x 3 -> 1,
+// 4096 rows): 29 us; with the reads of eight matrix instructions ahead of
+// them 36 us; with the multiplying waves bringing the slabs themselves between
+// two barriers each 46 us; with branches around the loads 75 us.
+__global__ __launch_bounds__(512) void k_mlp_dw(DwArgs a) {
+    constexpr int KS = 192, NG = KS / 32, L = 32, NB = 4;  // rows of a slab, in groups of 32; columns; slabs in LDS
+    __shared__ __attribute__((aligned(16))) float Zs[NB][KS * L];
+    __shared__ __attribute__((aligned(16))) bf16 As[NB][KS * L];
+    const int tid = threadIdx.x & 255;
+    const bool stager = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // the same in a whole wave
     if (blockIdx.x == a.blocks) {
         float s = 0.f;
-        for (int i = tid; i < a.B; i += 256) s += a.lossv[i];
-        Zs[tid] = s;
+        if (!stager) {
+            for (int i = tid; i < a.B; i += 256) s += a.lossv[i];
+            Zs[0][tid] = s;
+        }
         __syncthreads();
         for (int o = 128; o > 0; o >>= 1) {
-            if (tid < o) Zs[tid] += Zs[tid + o];
+            if (!stager && tid < o) Zs[0][tid] += Zs[0][tid + o];
             __syncthreads();
         }
-        if (tid == 0) a.loss[0] = Zs[0];
+        if (threadIdx.x == 0) a.loss[0] = Zs[0][0];
         return;
     }
     int li = 0;
@@ -471,101 +473,155 @@ __global__ __launch_bounds__(256) void k_mlp_dw(DwArgs a) {
     const DwLayer& y = a.layer[li];
     const int M = y.M, N = y.N, lda = y.lda, ldz = y.ldz;
     const int m0 = int((blockIdx.x - y.block0) / y.nblk) * 32, n0 = int((blockIdx.x - y.block0) % y.nblk) * 32;
-    const int lane = tid & 63, wave = tid >> 6, c = lane & 15, kk = lane >> 4, wm = (wave & 1) * 16, wn = (wave >> 1) * 16;
-    const int ach = tid & 3, ar = tid >> 2;  // A: 8 columns of row ar + 64 i
-    const int zch = tid & 7, zr = tid >> 3;  // Z: 4 columns of row zr + 32 i
-    // loads without branches: a row past the batch or a column past the
-    // matrix reads one that is there, and rows past the batch are zeroed on
-    // the way to LDS (outputs of other columns are not stored)
-    uint4 ra[2][4];
-    float4 rz[2][8];
-    const bf16* Ap = y.A + (m0 + ach * 8 < lda ? m0 + ach * 8 : 0);
-    const float* Zp = y.Z + (n0 + zch * 4 < ldz ? n0 + zch * 4 : 0);
-    const int last = a.B - 1;
-    auto load = [&](int set, int k0) {
+    const int slabs = (a.B + KS - 1) / KS;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Both kinds of waves pass slabs + 1 barriers. After the first the first two
+    // slabs are there, after each later one a slab is used up and one more there.
+    if (stager) {
+        // Every instruction these waves issue delays the matrix instructions of
+        // the others on their SIMD: slabs go from memory to LDS directly, 1 KiB
+        // an instruction, at fixed offsets of the thread from a scalar base.
+        // Rows past the batch read as zeros through the descriptor's length
+        // (which does not see a scalar offset beside it, hence none). A column
+        // past the matrix reads one that is there; outputs of other columns are
+        // not stored. The 16-byte pieces of a row of Z change
+        // places by bit 1 of its index, for the banks of the reads.
+        const int zch = (lane & 7) ^ (lane >> 4 & 1) << 2, ach = lane & 3;
+        int zo[6], ao[3];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            ra[set][i] = *reinterpret_cast<const uint4*>(Ap + size_t(min(k0 + ar + 64 * i, last)) * lda);
+        for (int i = 0; i < 6; ++i)
+            zo[i] = 4 * (((wave * 6 + i) * 8 + (lane >> 3)) * ldz + (n0 + zch * 4 < ldz ? n0 + zch * 4 : 0));
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            rz[set][i] = *reinterpret_cast<const float4*>(Zp + size_t(min(k0 + zr + 32 * i, last)) * ldz);
-    };
+        for (int i = 0; i < 3; ++i)
+            ao[i] = 2 * (((wave * 3 + i) * 16 + (lane >> 2)) * lda + (m0 + ach * 8 < lda ? m0 + ach * 8 : 0));
+        auto load = [&](int slab) {
+            auto rows = [&](const void* base, int bytes) {  // the slab's rows of the batch
+                const int left = slab < slabs ? (a.B - slab * KS < KS ? a.B - slab * KS : KS) : 0;
+                return __builtin_amdgcn_make_buffer_rsrc(
+                    const_cast<char*>(static_cast<const char*>(base)) + size_t(slab < slabs ? slab : 0) * KS * bytes, 0,
+                    __builtin_amdgcn_readfirstlane(left * bytes), 0x00020000);
+            };
+            typedef __attribute__((address_space(3))) void lds_void;
+            const auto Z = rows(y.Z, 4 * ldz), A = rows(y.A, 2 * lda);
+            float* zs = Zs[slab % NB] + wave * 6 * 256;
+            bf16* as = As[slab % NB] + wave * 3 * 512;
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(Z, (lds_void*)(zs + i * 256), 16, zo[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(A, (lds_void*)(as + i * 512), 16, ao[i], 0, 0, 0);
+        };
+        // all but the newest slab's nine loads are done
+        auto ready = [] {
+            __builtin_amdgcn_s_waitcnt(0x0f79);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        load(0);
+        load(1);
+        load(2);
+        ready();
+        for (int k = 0; k < slabs; ++k) {
+            load(k + 3);
+            ready();
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // none may land after this block's LDS is another's
+        return;
+    }
+    const int c = lane & 15, kk = lane >> 4, wm = (wave & 1) * 16, wn = (wave >> 1) * 16;
     fx4 acc = {0.f, 0.f, 0.f, 0.f};
     const bool active = m0 + wm <= M && n0 + wn < N;
-    auto slab = [&](int set, int k0) {
-        const int left = a.B - k0;
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool in = ar + 64 * i < left;
-            uint4 v = ra[set][i];
-            v.x = in ? v.x : 0u;
-            v.y = in ? v.y : 0u;
-            v.z = in ? v.z : 0u;
-            v.w = in ? v.w : 0u;
-            *reinterpret_cast<uint4*>(As + (ar + 64 * i) * LA + ach * 8) = v;
-            const int one = M - (m0 + ach * 8);  // the column of ones, if it is among these
-            if (one >= 0 && one < 8) As[(ar + 64 * i) * LA + ach * 8 + one] = bf16(0x3f80);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const bool in = zr + 32 * i < left;
-            float4 v = rz[set][i];
-            v.x = in ? v.x : 0.f;
-            v.y = in ? v.y : 0.f;
-            v.z = in ? v.z : 0.f;
-            v.w = in ? v.w : 0.f;
-            *reinterpret_cast<float4*>(Zs + (zr + 32 * i) * LZ + zch * 4) = v;
-        }
-        __syncthreads();
-        load(set, k0 + 2 * KS);
-        if (!active) return;
-        // operands of eight matrix instructions are read while the eight
-        // before them run (a barrier to the scheduler keeps them apart)
-        const bf16* pa = As + kk * LA + wm + c;
-        const float* pz = Zs + kk * LZ + wn + c;
-        const int groups = left >= KS ? KS / 32 : (left + 31) / 32;  // of 8 x 4 rows
-        float x[2][8], z[2][8];
-        auto read = [&](int h, int g) {
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                x[h][u] = bf16_to(pa[4 * (8 * g + u) * LA]);
-                z[h][u] = pz[4 * (8 * g + u) * LZ];
-            }
-        };
-        read(0, 0);
-        for (int g = 0; g < groups; g += 2) {
-            read(1, min(g + 1, KS / 32 - 1));
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0][u], z[0][u], acc, 0, 0, 0);
-            read(0, min(g + 2, KS / 32 - 1));
-            __builtin_amdgcn_sched_barrier(0);
-            if (g + 1 < groups)
-#pragma unroll
-                for (int u = 0; u < 8; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[1][u], z[1][u], acc, 0, 0, 0);
-        }
-    };
-    load(0, 0);
-    load(1, KS);
-    for (int k0 = 0; k0 < a.B; k0 += 2 * KS) {
-        slab(0, k0);
-        if (k0 + KS < a.B) slab(1, k0 + KS);
-    }
+    // this thread's outputs, and what Adam needs of them: read now, these loads
+    // would be most of the kernel's end
     const int n = n0 + wn + c;
-    if (!active || n >= N) return;
+    size_t at[4];
+    bool mine[4];
+    float aw[4], am[4], av[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int m = m0 + wm + 4 * kk + r;
-        if (m > M) continue;
-        const size_t i = m < M ? y.woff + size_t(m) * N + n : y.boff + size_t(n);
+        mine[r] = active && n < N && m <= M;
+        at[r] = !mine[r] ? 0 : m < M ? y.woff + size_t(m) * N + n : y.boff + size_t(n);
+        if (a.adam) {
+            aw[r] = a.w[at[r]];
+            am[r] = a.m[at[r]];
+            av[r] = a.v[at[r]];
+        }
+    }
+    // Group by group, across slabs: the operands of the group after the next are
+    // read while one is multiplied.
+    uint32_t raw[2][8];  // BF16
+    float x[2][8], z[3][8];
+    const bool one = m0 + wm + c == M;
+    auto read = [&](int t, const bf16* pa, const float* pz, int g, int u) {
+        raw[t & 1][u] = pa[(32 * g + 4 * u) * L];
+        z[t % 3][u] = pz[(32 * g + 4 * u) * L];
+    };
+    static_assert(NG % 6 == 0, "a slab begins with the first of each register set");
+    const int zc = wn + c;
+    const bf16* const pa0 = As[0] + kk * L + wm + c;
+    const float* const pz0 = Zs[0] + kk * L + (((zc >> 2) ^ (kk >> 1 & 1) << 2) << 2 | (zc & 3));
+    __syncthreads();
+    auto convert = [&](int t, int u, auto ones) {
+        x[t & 1][u] = __builtin_bit_cast(float, raw[t & 1][u] << 16);
+        if (ones) x[t & 1][u] = one ? 1.f : x[t & 1][u];
+    };
+    auto chain = [&](auto ones) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            read(0, pa0, pz0, 0, u);
+            read(1, pa0, pz0, 1, u);
+            convert(0, u, ones);
+        }
+        const bf16* pa = pa0;
+        const float* pz = pz0;
+        for (int k = 0; k < slabs; ++k) {
+            const int next = (k + 1) % NB;
+            const bf16* const qa = pa0 + next * KS * L;
+            const float* const qz = pz0 + next * KS * L;
+            // whole slabs: rows past the batch are zero
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                // in order, so that the reads and conversions issue while a matrix
+                // instruction keeps the next one waiting
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[g & 1][u], z[g % 3][u], acc, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    convert(g + 1, u, ones);
+                    if (g + 2 < NG)
+                        read(g + 2, pa, pz, g + 2, u);
+                    else
+                        read(g + 2, qa, qz, g + 2 - NG, u);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            pa = qa;
+            pz = qz;
+            __syncthreads();
+        }
+    };
+    if (M >= m0 && M < m0 + 32)  // the column of ones is in this block
+        chain(std::true_type{});
+    else
+        chain(std::false_type{});
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (!mine[r]) continue;
         if (!a.adam) {
-            a.g[i] = acc[r];
+            a.g[at[r]] = acc[r];
             continue;
         }
-        const float wi = adam_step(a.w, a.m, a.v, i, acc[r], a.lr, a.b1, a.b2, a.eps, a.c1, a.c2);
+        adam_step(aw[r], am[r], av[r], acc[r], a.lr, a.b1, a.b2, a.eps, a.c1, a.c2);
+        a.w[at[r]] = aw[r];
+        a.m[at[r]] = am[r];
+        a.v[at[r]] = av[r];
+        const int m = m0 + wm + 4 * kk + r;
         if (m < M) {
-            const bf16 h = bf16_from(wi);
+            const bf16 h = bf16_from(aw[r]);
             y.wp[size_t(m) * y.ldw + n] = h;
             if (y.wt) y.wt[size_t(n) * y.ldt + m] = h;
         }
@@ -797,7 +853,7 @@ static int mlp_dw(qcs_mlp* n, int B, bool adam, float lr, float* loss) {
         y.block0 = a.blocks;
         a.blocks += y.nblk * uint32_t((y.M + 1 + 31) / 32);
     }
-    hipLaunchKernelGGL(k_mlp_dw, dim3(a.blocks + 1), dim3(256), 0, n->stream, a);
+    hipLaunchKernelGGL(k_mlp_dw, dim3(a.blocks + 1), dim3(512), 0, n->stream, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? QCS_OK : set_error(QCS_EDEVICE, "mlp gradients: %s", hipGetErrorString(e));
 }
