@@ -509,7 +509,7 @@ struct TileGate {
     uint64_t ctrl = 0;    // bits that must be 1
     uint8_t nm = 0;       // matrix entries (complex)
     double f = 1;         // fraction of the state's bytes its own launch moves
-    const qcs_gate* src = nullptr;
+    const qcs_gate* src = nullptr;  // null: several gates in one
     const double* mat = nullptr;
     uint32_t dim = 0, b0 = 0;  // matrix dimension, first row and column of its block
 };
@@ -611,6 +611,7 @@ static std::vector<TileGate> tile_gates(const qcs_gate* gates, uint32_t n, uint3
                     drop(t, x);
                     drop(c, x);
                     gone[x] = 1;
+                    D.src = nullptr;
                     D.D ^= 1ull << c;
                     if (has)
                         drop(c, d);
@@ -1067,7 +1068,7 @@ static int run_tiles(qcs_register* r, const qcs_gate* gates, uint32_t n) {
         // 10 / 14 / 23 against 12 / 13 / 14; on 20 qubits 15 / 18 / 37 against
         // 18 / 18 / 23; on 25 qubits, by worth, 208 / 382 / 602 against
         // 177 / 211 / 225).
-        const bool pass = P.g[P.head].op != kNoTile && (big ? worth > 1.2 : take.size() > 2);
+        const bool pass = P.g[P.head].op != kNoTile && (!P.g[P.head].src || (big ? worth > 1.2 : take.size() > 2));
         if (!pass) take.assign(1, P.head);
         int prev = -1;
         size_t k = 0;

@@ -106,3 +106,27 @@ def test_refused_gate_ends_the_circuit(width):
         g.apply_circuit([(G.HadamardGate(), [3]), (G.HadamardGate(), [n])], fuse_width=width)
     assert np.array_equal(g.getRegisterStorage(), psi)
     g.close()
+
+
+@pytest.mark.parametrize("n", [3, 6, 12, 16, 23])
+@pytest.mark.parametrize("count", [1, 2, 3])
+def test_few_gates(n, count):
+    """Lists too short for a pass, of which a CNOT, Rz, CNOT in the middle is
+    one gate to the planner and has no launch of its own: on registers of one
+    tile, of several and above 64 MiB."""
+    rng = np.random.default_rng(10 * n + count)
+    psi = random_state(rng, n)
+    for k in range(4):
+        a, b, c = (int(x) for x in rng.permutation(n)[:3])
+        seq = [(G.CNOTGate(), [a, b]), (G.RzGate(0.7 + k), [a]), (G.CNOTGate(), [a, b])]
+        if k & 1:
+            seq += [(G.CNOTGate(), [b, c]), (G.RzGate(0.4), [b]), (G.CNOTGate(), [b, c])]
+        if k & 2:
+            seq.insert(int(rng.integers(len(seq))), (G.RyGate(0.3), [c]))
+        seq = seq * (count - 1) + seq
+        g = QubitRegister(n)
+        g.setRegisterStorageFastNoNormalize(psi.copy())
+        g.apply_circuit(seq)
+        got = np.asarray(g.getRegisterStorage())
+        g.close()
+        assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12, k
