@@ -37,6 +37,9 @@ struct TileGeo {
     uint8_t pos[kTileMax + 4];  // tile qubits, ascending
 };
 
+// An amplitude: four registers in a row, as LDS reads and writes take them.
+typedef double Amp __attribute__((ext_vector_type(2)));
+
 // Operation codes of a pass's stream: base + register bit, pair or triple.
 enum : uint32_t {
     kOpGen1 = 0,    // + J: 2x2 on register bit J (8 reals)
@@ -82,8 +85,26 @@ constexpr uint32_t kPickBit = 1u << 24;  // the bit's number at 16..20
 // and a branch on the lanes makes the compiler route the whole loop through
 // masked control flow (1150 cycles against 480 for a U(2) on a tile of 4096).
 // Same operations in the same order as the gate kernels. m: matrix entries.
+// The amplitudes are in registers of fixed numbers, so that the halves of one
+// can be named here and whole ones outside.
 #if defined(__HIP_DEVICE_COMPILE__)
-#define QA(I, C) "%[a" #I #C "]"
+#define QA(I, C) QA_##I##C
+#define QA_0x "v[32:33]"
+#define QA_0y "v[34:35]"
+#define QA_1x "v[36:37]"
+#define QA_1y "v[38:39]"
+#define QA_2x "v[40:41]"
+#define QA_2y "v[42:43]"
+#define QA_3x "v[44:45]"
+#define QA_3y "v[46:47]"
+#define QA_4x "v[48:49]"
+#define QA_4y "v[50:51]"
+#define QA_5x "v[52:53]"
+#define QA_5y "v[54:55]"
+#define QA_6x "v[56:57]"
+#define QA_6y "v[58:59]"
+#define QA_7x "v[60:61]"
+#define QA_7y "v[62:63]"
 #define Q_BIT(I) "s_bitcmp1_b32 %[mask], " #I "\n\ts_cbranch_scc0 9f\n\t"  // to 9 unless bit I of the mask is set
 // the orbit {I, K} times the 2x2 matrix
 #define Q_GEN(I, K)                                                                                   \
@@ -162,7 +183,7 @@ constexpr uint32_t kPickBit = 1u << 24;  // the bit's number at 16..20
              "v_mul_f64 " QA(I, y) ", -1.0, " QA(I, y) "\n9:\n\t"
 #define Q_IF(CODE, LABEL) "s_cmp_eq_u32 %[code], " #CODE "\n\ts_cbranch_scc1 " #LABEL "f\n\t"
 #define Q_DONE "s_branch 8f\n"
-__device__ __forceinline__ void tile_simple(double2 (&a)[8], uint32_t code, uint32_t mask, const double (&m)[8],
+__device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t mask, const double (&m)[8],
                                             uint64_t on, uint32_t tid, uint32_t tile) {
     double t0, t1, t2, t3;
     uint64_t save;
@@ -224,11 +245,9 @@ __device__ __forceinline__ void tile_simple(double2 (&a)[8], uint32_t code, uint
         "54:\n\t" Q_A00(0, 1, 4) Q_A00(2, 3, 6) Q_DONE
         "55:\n\t" Q_A00(0, 2, 4) Q_A00(1, 3, 5)
         "8:\n\ts_mov_b64 exec, %[save]"
-        : [a0x] "+&v"(a[0].x), [a0y] "+&v"(a[0].y), [a1x] "+&v"(a[1].x), [a1y] "+&v"(a[1].y), [a2x] "+&v"(a[2].x),
-          [a2y] "+&v"(a[2].y), [a3x] "+&v"(a[3].x), [a3y] "+&v"(a[3].y), [a4x] "+&v"(a[4].x), [a4y] "+&v"(a[4].y),
-          [a5x] "+&v"(a[5].x), [a5y] "+&v"(a[5].y), [a6x] "+&v"(a[6].x), [a6y] "+&v"(a[6].y), [a7x] "+&v"(a[7].x),
-          [a7y] "+&v"(a[7].y), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3), [save] "=&s"(save),
-          [v] "=&v"(v), [z] "=&s"(z)
+        : "+{v[32:35]}"(a[0]), "+{v[36:39]}"(a[1]), "+{v[40:43]}"(a[2]), "+{v[44:47]}"(a[3]), "+{v[48:51]}"(a[4]),
+          "+{v[52:55]}"(a[5]), "+{v[56:59]}"(a[6]), "+{v[60:63]}"(a[7]), [t0] "=&v"(t0),
+          [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3), [save] "=&s"(save), [v] "=&v"(v), [z] "=&s"(z)
         : [r00] "s"(m[0]), [i00] "s"(m[1]), [r01] "s"(m[2]), [i01] "s"(m[3]), [r10] "s"(m[4]), [i10] "s"(m[5]),
           [r11] "s"(m[6]), [i11] "s"(m[7]), [code] "s"(code), [mask] "s"(mask), [on] "s"(on),
           [tid] "v"(tid), [zt] "s"(zt)
@@ -255,10 +274,10 @@ __device__ __forceinline__ void tile_simple(double2 (&a)[8], uint32_t code, uint
 #else
 // The same in C++: what the host compiler sees of the kernel, and a statement
 // of what each code does.
-__host__ __device__ inline void tile_simple(double2 (&a)[8], uint32_t code, uint32_t mask, const double (&m)[8],
+__host__ __device__ inline void tile_simple(Amp (&a)[8], uint32_t code, uint32_t mask, const double (&m)[8],
                                             uint64_t on, uint32_t tid, uint32_t tile) {
     if (!on) return;
-    auto mul = [](double2& x, double r, double i) { x = double2{r * x.x - i * x.y, r * x.y + i * x.x}; };
+    auto mul = [](Amp& x, double r, double i) { x = Amp{r * x.x - i * x.y, r * x.y + i * x.x}; };
     for (int i = 0; i < 8; ++i) {
         if (code >= kOpZ) {
             const uint64_t zt = uint32_t(__builtin_bit_cast(uint64_t, m[2]));
@@ -271,18 +290,18 @@ __host__ __device__ inline void tile_simple(double2 (&a)[8], uint32_t code, uint
         const uint32_t J = code & 3;  // register bit of the one-qubit codes
         if (code < kOpDiagR) {
             if (i >> J & 1) continue;
-            double2 &x = a[i], &y = a[i | 1 << J];
-            const double2 p = x, q = y;
+            Amp &x = a[i], &y = a[i | 1 << J];
+            const Amp p = x, q = y;
             if (code >= kOpReal && code < kOpImag) {
-                x = double2{m[0] * p.x + m[1] * q.x, m[0] * p.y + m[1] * q.y};
-                y = double2{m[2] * p.x + m[3] * q.x, m[2] * p.y + m[3] * q.y};
+                x = Amp{m[0] * p.x + m[1] * q.x, m[0] * p.y + m[1] * q.y};
+                y = Amp{m[2] * p.x + m[3] * q.x, m[2] * p.y + m[3] * q.y};
             } else if (code >= kOpImag && code < kOpX) {
-                x = double2{m[0] * p.x - m[1] * q.y, m[0] * p.y + m[1] * q.x};
-                y = double2{m[3] * q.x - m[2] * p.y, m[3] * q.y + m[2] * p.x};
+                x = Amp{m[0] * p.x - m[1] * q.y, m[0] * p.y + m[1] * q.x};
+                y = Amp{m[3] * q.x - m[2] * p.y, m[3] * q.y + m[2] * p.x};
             } else if (code < kOpReal) {
-                x = double2{m[0] * p.x - m[1] * p.y + m[2] * q.x - m[3] * q.y,
+                x = Amp{m[0] * p.x - m[1] * p.y + m[2] * q.x - m[3] * q.y,
                             m[0] * p.y + m[1] * p.x + m[2] * q.y + m[3] * q.x};
-                y = double2{m[4] * p.x - m[5] * p.y + m[6] * q.x - m[7] * q.y,
+                y = Amp{m[4] * p.x - m[5] * p.y + m[6] * q.x - m[7] * q.y,
                             m[4] * p.y + m[5] * p.x + m[6] * q.y + m[7] * q.x};
             } else {
                 std::swap(x, y);
@@ -313,8 +332,8 @@ __host__ __device__ inline void tile_simple(double2 (&a)[8], uint32_t code, uint
 
 // Generic blocks: y = M x on the orbit idx[0..D), in the lanes that are on.
 template <int R, int D, typename M>
-__host__ __device__ __forceinline__ void tile_rows(double2 (&a)[1 << R], const int (&idx)[D], M m, bool on) {
-    double2 x[D];
+__host__ __device__ __forceinline__ void tile_rows(Amp (&a)[1 << R], const int (&idx)[D], M m, bool on) {
+    Amp x[D];
 #pragma unroll
     for (int c = 0; c < D; ++c) x[c] = a[idx[c]];
 #pragma unroll
@@ -339,7 +358,7 @@ template <int A, int B> __host__ __device__ constexpr int zero2(int i) {  // zer
 }
 
 template <int R, int A, int B, typename M>
-__host__ __device__ __forceinline__ void tile_gen2(double2 (&a)[1 << R], uint32_t mask, M m, bool on) {
+__host__ __device__ __forceinline__ void tile_gen2(Amp (&a)[1 << R], uint32_t mask, M m, bool on) {
 #pragma unroll
     for (int p = 0; p < 1 << (R - 2); ++p) {
         const int i = zero2<A, B>(p);
@@ -349,7 +368,7 @@ __host__ __device__ __forceinline__ void tile_gen2(double2 (&a)[1 << R], uint32_
 }
 
 template <int R, typename M>
-__host__ __device__ __forceinline__ void tile_generic(double2 (&a)[1 << R], uint32_t code, uint32_t mask, M m, bool on) {
+__host__ __device__ __forceinline__ void tile_generic(Amp (&a)[1 << R], uint32_t code, uint32_t mask, M m, bool on) {
     static_assert(R == 3, "register codes are written out for three register qubits");
     if (code == kOpGen2)
         tile_gen2<R, 0, 1>(a, mask, m, on);
@@ -383,20 +402,27 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 // gate in FP32 a 27-qubit circuit of 867 gates came out 1.3e-6 off in its
 // expectation values, in dense FP32 blocks 4e-7, in FP64 passes 2e-8.)
 //
-// 592 gates on 25 qubits in complex128: 8 ms, of them in dense blocks of five
-// qubits 18.8 ms; 600 gates on 16 qubits from a graph: 0.32 ms, in one launch
-// per gate 1.4 ms; the 27-qubit circuit 14.4 ms, in dense blocks 18.7 ms. Its
-// first pass (102 gates in 12 rounds) takes 3.5 ms where its bytes take 0.43:
-// vector instructions bound a pass of many gates, bytes one of few.
-// The
-// first and the last round hold the top R tile qubits, the layout of the
-// global loads and stores, so they need no LDS.
+// 592 gates on 25 qubits in complex128: 8.5 ms, in dense blocks of five qubits
+// 19.6 ms; 600 gates on 16 qubits from a graph: 0.38 ms, one launch a gate
+// 1.44 ms; the 27-qubit circuit 13.7 ms, in dense blocks 19.2 ms. Vector
+// instructions bound a pass of many gates, bytes one of few.
+//
+// The first and the last round hold the top R tile qubits, the layout of the
+// global loads and stores, so they need no LDS. An exchange takes 50 vector
+// instructions: the register bits add to a place by XOR of scalars, the places
+// of a round's reads serve the writes that end it, and an amplitude stays in
+// one register quadruple from the read through all operations to the write.
+// (Places formed per amplitude from the thread's index, twice, and amplitudes
+// in halves that were moved together for each write, took 170: 8.86 ms on 25
+// qubits, 14.6 on 27, 0.395 on 16.)
 template <typename T, int R, bool NT>
 __global__ __launch_bounds__(1 << (kTileMax - R), 4) void k_tile(cv<T>* __restrict__ psi, TileGeo geo,
                                                                  const uint32_t* __restrict__ stream, uint32_t words_total,
                                                                  uint64_t boff) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    double2* s = reinterpret_cast<double2*>(smem_raw);
+    // aligned to its size, so that places in it are joined by XOR
+    extern __shared__ __attribute__((aligned(sizeof(Amp) << kTileMax))) unsigned char smem_raw[];
+    typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
+    typedef __attribute__((address_space(3))) Amp* lds_amp;
     typedef const __attribute__((address_space(4))) uint32_t* words;
     typedef const __attribute__((address_space(4))) double* reals;
     words w = (words)stream;
@@ -418,31 +444,38 @@ __global__ __launch_bounds__(1 << (kTileMax - R), 4) void k_tile(cv<T>* __restri
         for (int i = 0; i < R; ++i) hi[k] |= uint64_t(k >> i & 1) << geo.pos[t - R + i];
     }
     cv<T>* p = psi + (base | off);
-    double2 a[1 << R];
+    Amp a[1 << R] = {};  // threads past the tile hold zeros, in LDS past the tile's
     if (active) {
 #pragma unroll
         for (int k = 0; k < 1 << R; ++k) {
             const cv<T> v = ldamp<T, NT>(p + hi[k]);
-            a[k] = double2{double(v.x), double(v.y)};
+            a[k] = Amp{double(v.x), double(v.y)};
         }
     }
     uint32_t regs = 0;
 #pragma unroll
     for (uint32_t i = 0; i < R; ++i) regs |= (t - R + i) << (8 * i);
-    // position of the thread's amplitude k in LDS: its slot with k's bits set
-    auto exchange = [&](auto&& f) {
-        uint32_t slot = tid;
+    // The thread's amplitude 0 in LDS, and what the register bits add to a
+    // place there (XOR): kept from a round's reads for the writes that end it.
+    uint32_t slot = 0, add[R] = {};
+    auto layout = [&](uint32_t regs) {
+        slot = tid;
 #pragma unroll
-        for (int i = 0; i < R; ++i) slot = tile_zero(slot, regs >> (8 * i) & 255);
-        slot = tile_slot(slot);
-#pragma unroll
-        for (int k = 0; k < 1 << R; ++k) {
-            uint32_t c = 0;
-#pragma unroll
-            for (int i = 0; i < R; ++i) c |= uint32_t(k >> i & 1) << (regs >> (8 * i) & 255);
-            if (active) f(s[slot ^ tile_slot(c)], a[k]);
+        for (int i = 0; i < R; ++i) {
+            slot = tile_zero(slot, regs >> (8 * i) & 255);
+            add[i] = tile_slot(1u << (regs >> (8 * i) & 255)) * uint32_t(sizeof(Amp));
+            asm("" : "+s"(add[i]));  // stays a scalar
         }
+        slot = uint32_t(reinterpret_cast<uintptr_t>((lds_bytes)smem_raw)) | tile_slot(slot) * uint32_t(sizeof(Amp));
     };
+    auto place = [&](int k) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (k >> i & 1) c ^= add[i];
+        return (lds_amp)(slot ^ c);
+    };
+    layout(regs);
     uint32_t head = w[0], lane = w[1], mask = w[2], blk = w[3];
     for (;;) {
         uint32_t code = head & 0xffff;
@@ -474,10 +507,12 @@ __global__ __launch_bounds__(1 << (kTileMax - R), 4) void k_tile(cv<T>* __restri
         if (code == kOpRound) {
             // from the layout of the round before to this one's; a thread
             // writes back only what it alone has read, so one barrier is enough
-            exchange([](double2& x, double2& y) { x = y; });
+#pragma unroll
+            for (int k = 0; k < 1 << R; ++k) *place(k) = a[k];
             __syncthreads();
-            regs = lane;
-            exchange([](double2& x, double2& y) { y = x; });
+            layout(lane);
+#pragma unroll
+            for (int k = 0; k < 1 << R; ++k) a[k] = *place(k);
         } else if ((tile & blk) == blk) {
             tile_generic<R>(a, code, mask, (reals)body, (tid & (lane & 0xffff)) == lane >> 16);
         }
@@ -985,7 +1020,7 @@ template <typename T>
 static int tile_launch(qcs_register* r, const TileGeo& geo, const uint32_t* stream, uint32_t words, bool nt) {
     const uint64_t tiles = r->A >> geo.t;
     const unsigned threads = std::max(64u, 1u << (geo.t - kTileReg));
-    const size_t shm = sizeof(double2) << geo.t;
+    const size_t shm = std::max<size_t>(sizeof(Amp) << geo.t, sizeof(Amp) * threads << kTileReg);
     for (uint64_t boff = 0; boff < tiles; boff += kMaxBlocks) {
         const unsigned grid = unsigned(std::min(kMaxBlocks, tiles - boff));
         if (nt)
