@@ -937,9 +937,7 @@ int qcs_mlp_create(uint32_t in_dim, uint32_t hidden, uint32_t layers, uint64_t s
               hipMalloc(reinterpret_cast<void**>(&n->m), sizeof(float) * off) == hipSuccess &&
               hipMalloc(reinterpret_cast<void**>(&n->v), sizeof(float) * off) == hipSuccess &&
               hipMalloc(reinterpret_cast<void**>(&n->wpack), sizeof(bf16) * packed) == hipSuccess &&
-              hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) == hipSuccess &&
-              hipStreamCreateWithFlags(&n->up, hipStreamNonBlocking) == hipSuccess &&
-              hipEventCreateWithFlags(&n->up_ev, hipEventDisableTiming) == hipSuccess;
+              hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) == hipSuccess;
     if (!ok) {
         (void)hipGetLastError();
         qcs_mlp_destroy(n);
@@ -986,7 +984,9 @@ static constexpr uint32_t kMlpSlice = 65536;
 // stages at once from pageable memory), on a stream of their own, so that the
 // copy of a piece runs while the piece before it is computed; on one stream a
 // pageable copy waits for the launches before it. 65536 rows of 17: 471 us
-// on one stream, 330 us so.
+// on one stream, 330 us so. The stream comes with the first call of more than
+// one piece: it takes as long to make as the rest of a network (0.9 ms with
+// it, 0.5 without).
 static constexpr size_t kMlpPiece = size_t(1) << 20;
 
 int qcs_mlp_forward(qcs_mlp* n, const float* x, uint32_t batch, float* y) {
@@ -1001,10 +1001,15 @@ int qcs_mlp_forward(qcs_mlp* n, const float* x, uint32_t batch, float* y) {
         for (uint32_t p0 = 0; p0 < B; p0 += piece) {
             const uint32_t P = std::min(piece, B - p0);
             float* xd = n->xin + size_t(p0) * n->in;
+            const bool apart = piece < B;
+            if (apart && !n->up && hipStreamCreateWithFlags(&n->up, hipStreamNonBlocking) != hipSuccess)
+                return set_error(QCS_EDEVICE, "upload stream");
+            if (apart && !n->up_ev && hipEventCreateWithFlags(&n->up_ev, hipEventDisableTiming) != hipSuccess)
+                return set_error(QCS_EDEVICE, "upload event");
             if (hipMemcpyAsync(xd, x + size_t(b0 + p0) * n->in, sizeof(float) * P * n->in, hipMemcpyHostToDevice,
-                               n->up) != hipSuccess ||
-                hipEventRecord(n->up_ev, n->up) != hipSuccess ||
-                hipStreamWaitEvent(n->stream, n->up_ev, 0) != hipSuccess)
+                               apart ? n->up : n->stream) != hipSuccess ||
+                (apart && (hipEventRecord(n->up_ev, n->up) != hipSuccess ||
+                           hipStreamWaitEvent(n->stream, n->up_ev, 0) != hipSuccess)))
                 return set_error(QCS_EDEVICE, "input upload failed");
             if (const int e = mlp_rows(n, int(P), xd, nullptr, nullptr, false, n->out + p0)) return e;
         }
