@@ -53,11 +53,10 @@ enum : uint32_t {
     kOpSwap = 28,   // + pair: exchange
     kOpSwapP = 32,  // + pair: exchange times m0
     kOpZ = 36,      // + set of register bits: times re - i im (even parity) or re + i im (odd)
-    kOpHalf = 44,   // + set of register bits: odd parity times m0
-    kOpGen2 = 52,   // + pair: 4x4 (from here on handled outside the inner loop)
-    kOpGen3 = 56,   // 8x8
-    kOpRound = 57,  // the thread mask holds the register positions, a byte each
-    kOpEnd = 58,
+    kOpGen2 = 44,   // + pair: 4x4 (from here on handled outside the inner loop)
+    kOpGen3 = 48,   // 8x8
+    kOpRound = 49,  // the thread mask holds the register positions, a byte each
+    kOpEnd = 50,
 };
 
 // A stream is a list of records: code | words << 16, thread mask | thread
@@ -156,7 +155,6 @@ constexpr uint32_t kPickBit = 1u << 24;  // the bit's number at 16..20
     "v_fma_f64 " QA(I, x) ", " R ", " QA(I, x) ", -%[t0]\n\t"
 #define Q_MULB(I, R, J) Q_BIT(I) Q_MUL(I, R, J) "9:\n\t"
 #define Q_M0(I) Q_MULB(I, "%[r00]", "%[i00]")
-#define Q_H(I) Q_MUL(I, "%[r00]", "%[i00]")
 #define Q_M1(I) Q_MULB(I, "%[r01]", "%[i01]")
 // a[I] times r00 - i t2 (even register parity) or r00 + i t2 (odd)
 #define Q_ZE(I)                                                                                       \
@@ -199,8 +197,7 @@ __device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
         Q_GEN(0, 1) Q_GEN(2, 3) Q_GEN(4, 5) Q_GEN(6, 7) Q_DONE
         "21:\n\t" Q_GEN(0, 2) Q_GEN(1, 3) Q_GEN(4, 6) Q_GEN(5, 7) Q_DONE
         "22:\n\t" Q_GEN(0, 4) Q_GEN(1, 5) Q_GEN(2, 6) Q_GEN(3, 7) Q_DONE
-        "20:\n\ts_cmp_gt_u32 %[code], 35\n\ts_cbranch_scc1 40f\n\t"
-        "s_cmp_gt_u32 %[code], 10\n\ts_cbranch_scc1 30f\n\t" Q_IF(8, 23) Q_IF(9, 24) Q_IF(10, 25)
+        "20:\n\ts_cmp_gt_u32 %[code], 10\n\ts_cbranch_scc1 30f\n\t" Q_IF(8, 23) Q_IF(9, 24) Q_IF(10, 25)
         Q_IF(5, 26) Q_IF(6, 27)
         Q_REAL(0, 1) Q_REAL(2, 3) Q_REAL(4, 5) Q_REAL(6, 7) Q_DONE
         "26:\n\t" Q_REAL(0, 2) Q_REAL(1, 3) Q_REAL(4, 6) Q_REAL(5, 7) Q_DONE
@@ -208,11 +205,11 @@ __device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
         "23:\n\t" Q_IMAG(0, 1) Q_IMAG(2, 3) Q_IMAG(4, 5) Q_IMAG(6, 7) Q_DONE
         "24:\n\t" Q_IMAG(0, 2) Q_IMAG(1, 3) Q_IMAG(4, 6) Q_IMAG(5, 7) Q_DONE
         "25:\n\t" Q_IMAG(0, 4) Q_IMAG(1, 5) Q_IMAG(2, 6) Q_IMAG(3, 7) Q_DONE
-        "30:\n\ts_cmp_gt_u32 %[code], 14\n\ts_cbranch_scc1 60f\n\t" Q_IF(13, 31) Q_IF(14, 32)
+        "30:\n\ts_cmp_gt_u32 %[code], 14\n\ts_cbranch_scc1 40f\n\t" Q_IF(13, 31) Q_IF(14, 32)
         Q_SWAP(0, 0, 1) Q_SWAP(2, 2, 3) Q_SWAP(4, 4, 5) Q_SWAP(6, 6, 7) Q_DONE
         "31:\n\t" Q_SWAP(0, 0, 2) Q_SWAP(1, 1, 3) Q_SWAP(4, 4, 6) Q_SWAP(5, 5, 7) Q_DONE
         "32:\n\t" Q_SWAP(0, 0, 4) Q_SWAP(1, 1, 5) Q_SWAP(2, 2, 6) Q_SWAP(3, 3, 7) Q_DONE
-        "40:\n\ts_cmp_gt_u32 %[code], 43\n\ts_cbranch_scc1 70f\n\t"
+        "40:\n\ts_cmp_lt_u32 %[code], 36\n\ts_cbranch_scc1 60f\n\t"
         // t2 = im or -im by the parity of the thread's and the tile's bits
         "s_lshr_b32 %[z], %[mask], 8\n\t"
         "v_and_b32 %[v], %[z], %[tid]\n\t"
@@ -231,14 +228,6 @@ __device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
         "65:\n\t" Q_ZE(0) Q_ZO(1) Q_ZE(2) Q_ZO(3) Q_ZO(4) Q_ZE(5) Q_ZO(6) Q_ZE(7) Q_DONE
         "66:\n\t" Q_ZE(0) Q_ZE(1) Q_ZO(2) Q_ZO(3) Q_ZO(4) Q_ZO(5) Q_ZE(6) Q_ZE(7) Q_DONE
         "67:\n\t" Q_ZE(0) Q_ZO(1) Q_ZO(2) Q_ZE(3) Q_ZO(4) Q_ZE(5) Q_ZE(6) Q_ZO(7) Q_DONE
-        "70:\n\t" Q_IF(46, 72) Q_IF(47, 73) Q_IF(48, 74) Q_IF(49, 75) Q_IF(50, 76) Q_IF(51, 77)
-        Q_H(1) Q_H(3) Q_H(5) Q_H(7) Q_DONE
-        "72:\n\t" Q_H(2) Q_H(3) Q_H(6) Q_H(7) Q_DONE
-        "73:\n\t" Q_H(1) Q_H(2) Q_H(5) Q_H(6) Q_DONE
-        "74:\n\t" Q_H(4) Q_H(5) Q_H(6) Q_H(7) Q_DONE
-        "75:\n\t" Q_H(1) Q_H(3) Q_H(4) Q_H(6) Q_DONE
-        "76:\n\t" Q_H(2) Q_H(3) Q_H(4) Q_H(5) Q_DONE
-        "77:\n\t" Q_H(1) Q_H(2) Q_H(4) Q_H(7) Q_DONE
         "60:\n\t" Q_IF(24, 41) Q_IF(25, 42) Q_IF(16, 43) Q_IF(17, 44) Q_IF(18, 45) Q_IF(20, 46) Q_IF(21, 47)
         Q_IF(22, 48) Q_IF(28, 50) Q_IF(29, 51) Q_IF(30, 52) Q_IF(32, 53) Q_IF(33, 54) "s_branch 55f\n"
         "41:\n\t" Q_M0(0) Q_M0(1) Q_M0(2) Q_M0(3) Q_M0(4) Q_M0(5) Q_M0(6) Q_M0(7) Q_DONE
@@ -271,7 +260,6 @@ __device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
 #undef Q_MULB
 #undef Q_M0
 #undef Q_M1
-#undef Q_H
 #undef Q_REAL
 #undef Q_IMAG
 #undef Q_ZE
@@ -291,15 +279,11 @@ __host__ __device__ inline void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
     if (!on) return;
     auto mul = [](Amp& x, double r, double i) { x = Amp{r * x.x - i * x.y, r * x.y + i * x.x}; };
     for (int i = 0; i < 8; ++i) {
-        if (code >= kOpZ && code < kOpHalf) {
+        if (code >= kOpZ) {
             const uint64_t zt = uint32_t(__builtin_bit_cast(uint64_t, m[2]));
             const bool odd = (__builtin_popcount(i & (code - kOpZ)) + __builtin_popcount(tid & mask >> 8) +
                               __builtin_popcount(tile & zt)) & 1;
             mul(a[i], m[0], odd ? m[1] : -m[1]);
-            continue;
-        }
-        if (code >= kOpHalf) {
-            if (__builtin_popcount(i & (code - kOpHalf)) & 1) mul(a[i], m[0], m[1]);
             continue;
         }
         if (!(mask >> i & 1)) continue;
@@ -316,9 +300,9 @@ __host__ __device__ inline void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
                 y = Amp{m[3] * q.x - m[2] * p.y, m[3] * q.y + m[2] * p.x};
             } else if (code < kOpReal) {
                 x = Amp{m[0] * p.x - m[1] * p.y + m[2] * q.x - m[3] * q.y,
-                        m[0] * p.y + m[1] * p.x + m[2] * q.y + m[3] * q.x};
+                            m[0] * p.y + m[1] * p.x + m[2] * q.y + m[3] * q.x};
                 y = Amp{m[4] * p.x - m[5] * p.y + m[6] * q.x - m[7] * q.y,
-                        m[4] * p.y + m[5] * p.x + m[6] * q.y + m[7] * q.x};
+                            m[4] * p.y + m[5] * p.x + m[6] * q.y + m[7] * q.x};
             } else {
                 std::swap(x, y);
                 if (code >= kOpAnti) {
@@ -418,9 +402,9 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 // gate in FP32 a 27-qubit circuit of 867 gates came out 1.3e-6 off in its
 // expectation values, in dense FP32 blocks 4e-7, in FP64 passes 2e-8.)
 //
-// 592 gates on 25 qubits in complex128: 8.4 ms, in dense blocks of five qubits
-// 19.6 ms; 600 gates on 16 qubits from a graph: 0.37 ms, one launch a gate
-// 1.44 ms; the 27-qubit circuit 13.2 ms, in dense blocks 19.2 ms. Vector
+// 592 gates on 25 qubits in complex128: 8.5 ms, in dense blocks of five qubits
+// 19.6 ms; 600 gates on 16 qubits from a graph: 0.38 ms, one launch a gate
+// 1.44 ms; the 27-qubit circuit 13.7 ms, in dense blocks 19.2 ms. Vector
 // instructions bound a pass of many gates, bytes one of few.
 //
 // The first and the last round hold the top R tile qubits, the layout of the
@@ -894,20 +878,6 @@ static void tile_emit(const std::vector<const TileGate*>& g, const std::vector<T
         else
             blkbit[q] = uint8_t(b++);
     }
-    // A phase by the parity of register bits alone, z or its conjugate, is the
-    // factor z / conj(z) on the odd half of the amplitudes and conj(z) on all;
-    // what is on all is collected to the end of the pass, which pays from
-    // three such gates on (27 qubits, 61 of 118 gates of a pass are phases, 35
-    // of these in registers; the circuit of 867 gates 13.7 ms with every one on
-    // all amplitudes, 13.2 on halves).
-    auto in_registers = [](const TileGate& o, const TileRound& rd) {
-        const hcplx z = entry(o, 1, 1);
-        return o.op == kOpZ && !(o.D & ~rd.regs) && std::abs(z.re * z.re + z.im * z.im - 1) < 1e-12;
-    };
-    int halves = 0;
-    for (const TileRound& rd : rounds)
-        for (const int oi : rd.ops) halves += in_registers(*g[oi], rd) ? 1 : 0;
-    hcplx all{1, 0};
     for (const TileRound& rd : rounds) {
         uint8_t rq[kTileReg];
         uint32_t packed = 0;
@@ -983,15 +953,6 @@ static void tile_emit(const std::vector<const TileGate*>& g, const std::vector<T
                     else
                         zl |= 1u << lanebit(q);
                 }
-                if (halves > 2 && in_registers(o, rd)) {
-                    const hcplx z = entry(o, 1, 1);
-                    const double nn = z.re * z.re + z.im * z.im;
-                    code = kOpHalf + zr;
-                    put(hcplx{(z.re * z.re - z.im * z.im) / nn, 2 * z.re * z.im / nn});
-                    all = hcplx{all.re * z.re + all.im * z.im, all.im * z.re - all.re * z.im};
-                    record(lane);
-                    continue;
-                }
                 code += zr;
                 rmask = zl << 8;
                 put(entry(o, 1, 1));
@@ -1044,10 +1005,6 @@ static void tile_emit(const std::vector<const TileGate*>& g, const std::vector<T
             }
             record(lane);
         }
-    }
-    if (halves > 2) {
-        out.insert(out.end(), {kOpScale | (kHead + 4) << 16, 0, (1u << (1 << kTileReg)) - 1, 0, 0, 0, 0, 0});
-        std::memcpy(&out[out.size() - 4], &all, sizeof all);
     }
     out.insert(out.end(), {kOpEnd, 0, 0, 0});
     out.resize(out.size() + kTail, 0);

@@ -130,38 +130,3 @@ def test_few_gates(n, count):
         got = np.asarray(g.getRegisterStorage())
         g.close()
         assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12, k
-
-
-class Phases(G.RzGate):
-    """diag(conj(z), z), of any magnitude."""
-
-    def __init__(self, z):
-        super().__init__(0.0)
-        self._m = np.diag([np.conj(z), z])
-
-
-@pytest.mark.parametrize("n", [3, 6, 12, 14])
-@pytest.mark.parametrize("count", [1, 2, 3, 8])
-@pytest.mark.parametrize("size", [1.0, 0.75])
-def test_parity_phases(n, count, size):
-    """Phases by the parity of each set of three neighbours, as many as a pass
-    takes one by one and more, by unit factors and by others: what all of them
-    have in common is left to the end of the pass. Each gate rounds an
-    amplitude (at most 1) a few times at 1.1e-16; the tolerance is that of the
-    lists above."""
-    rng = np.random.default_rng(7 * n + count)
-    psi = random_state(rng, n)
-    a = int(rng.integers(n - 2))
-    seq = []
-    for k in range(count):
-        s = [a + i for i in range(3) if (k % 7 + 1) >> i & 1]
-        down = [(G.CNOTGate(), [q, p]) for p, q in zip(s, s[1:])]
-        z = size * np.exp(1j * (0.3 + k))
-        seq += down + [(Phases(z), [s[-1]])] + down[::-1] + [(G.RxGate(0.2 + k), [s[0]])]
-    seq += [(G.HadamardGate(), [q]) for q in range(n)]
-    g = QubitRegister(n)
-    g.setRegisterStorageFastNoNormalize(psi.copy())
-    g.apply_circuit(seq)
-    got = np.asarray(g.getRegisterStorage())
-    g.close()
-    assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12
