@@ -370,8 +370,8 @@ int qcs_apply_circuit(qcs_register* r, const qcs_gate* gates, uint32_t n, uint32
             QCS_REQUIRE(gates[i].qubits[j] < r->n, "gate %u: qubit out of range", i);
     // Every width runs the list in passes of many gates (circuit.hip), which
     // beat dense blocks of the width: 25 qubits complex128, 592 gates, width 5
-    // 20.0 ms in dense blocks, 9.5 ms in passes; 28 qubits, 252 gates 37.0
-    // against 25.5 ms; 27 qubits complex64, 867 gates 19.2 against 14.7 ms
+    // 20.0 ms in dense blocks, 8.5 ms in passes; 28 qubits, 252 gates 37.0
+    // against 25.5 ms at most; 27 qubits complex64, 867 gates 19.2 against 13.4 ms
     // (host fusion, launches and waits included). The width stays what the
     // caller gets told, and what is refused.
     if (fuse_width == QCS_FUSE_AUTO) {

@@ -86,7 +86,9 @@ constexpr uint32_t kPickBit = 1u << 24;  // the bit's number at 16..20
 // masked control flow (1150 cycles against 480 for a U(2) on a tile of 4096).
 // Same operations in the same order as the gate kernels. m: matrix entries.
 // The amplitudes are in registers of fixed numbers, so that the halves of one
-// can be named here and whole ones outside.
+// can be named here and whole ones outside. A taken branch costs a wave 30
+// cycles: matrices are reached over the fewest, then the phases of kOpZ (13.4
+// ms against 13.7 with those a branch later, 867 gates on 27 qubits).
 #if defined(__HIP_DEVICE_COMPILE__)
 #define QA(I, C) QA_##I##C
 #define QA_0x "v[32:33]"
@@ -197,7 +199,8 @@ __device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
         Q_GEN(0, 1) Q_GEN(2, 3) Q_GEN(4, 5) Q_GEN(6, 7) Q_DONE
         "21:\n\t" Q_GEN(0, 2) Q_GEN(1, 3) Q_GEN(4, 6) Q_GEN(5, 7) Q_DONE
         "22:\n\t" Q_GEN(0, 4) Q_GEN(1, 5) Q_GEN(2, 6) Q_GEN(3, 7) Q_DONE
-        "20:\n\ts_cmp_gt_u32 %[code], 10\n\ts_cbranch_scc1 30f\n\t" Q_IF(8, 23) Q_IF(9, 24) Q_IF(10, 25)
+        "20:\n\ts_cmp_gt_u32 %[code], 35\n\ts_cbranch_scc1 40f\n\t"
+        "s_cmp_gt_u32 %[code], 10\n\ts_cbranch_scc1 30f\n\t" Q_IF(8, 23) Q_IF(9, 24) Q_IF(10, 25)
         Q_IF(5, 26) Q_IF(6, 27)
         Q_REAL(0, 1) Q_REAL(2, 3) Q_REAL(4, 5) Q_REAL(6, 7) Q_DONE
         "26:\n\t" Q_REAL(0, 2) Q_REAL(1, 3) Q_REAL(4, 6) Q_REAL(5, 7) Q_DONE
@@ -205,11 +208,11 @@ __device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
         "23:\n\t" Q_IMAG(0, 1) Q_IMAG(2, 3) Q_IMAG(4, 5) Q_IMAG(6, 7) Q_DONE
         "24:\n\t" Q_IMAG(0, 2) Q_IMAG(1, 3) Q_IMAG(4, 6) Q_IMAG(5, 7) Q_DONE
         "25:\n\t" Q_IMAG(0, 4) Q_IMAG(1, 5) Q_IMAG(2, 6) Q_IMAG(3, 7) Q_DONE
-        "30:\n\ts_cmp_gt_u32 %[code], 14\n\ts_cbranch_scc1 40f\n\t" Q_IF(13, 31) Q_IF(14, 32)
+        "30:\n\ts_cmp_gt_u32 %[code], 14\n\ts_cbranch_scc1 60f\n\t" Q_IF(13, 31) Q_IF(14, 32)
         Q_SWAP(0, 0, 1) Q_SWAP(2, 2, 3) Q_SWAP(4, 4, 5) Q_SWAP(6, 6, 7) Q_DONE
         "31:\n\t" Q_SWAP(0, 0, 2) Q_SWAP(1, 1, 3) Q_SWAP(4, 4, 6) Q_SWAP(5, 5, 7) Q_DONE
         "32:\n\t" Q_SWAP(0, 0, 4) Q_SWAP(1, 1, 5) Q_SWAP(2, 2, 6) Q_SWAP(3, 3, 7) Q_DONE
-        "40:\n\ts_cmp_lt_u32 %[code], 36\n\ts_cbranch_scc1 60f\n\t"
+        "40:\n\t"
         // t2 = im or -im by the parity of the thread's and the tile's bits
         "s_lshr_b32 %[z], %[mask], 8\n\t"
         "v_and_b32 %[v], %[z], %[tid]\n\t"
@@ -300,9 +303,9 @@ __host__ __device__ inline void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
                 y = Amp{m[3] * q.x - m[2] * p.y, m[3] * q.y + m[2] * p.x};
             } else if (code < kOpReal) {
                 x = Amp{m[0] * p.x - m[1] * p.y + m[2] * q.x - m[3] * q.y,
-                            m[0] * p.y + m[1] * p.x + m[2] * q.y + m[3] * q.x};
+                        m[0] * p.y + m[1] * p.x + m[2] * q.y + m[3] * q.x};
                 y = Amp{m[4] * p.x - m[5] * p.y + m[6] * q.x - m[7] * q.y,
-                            m[4] * p.y + m[5] * p.x + m[6] * q.y + m[7] * q.x};
+                        m[4] * p.y + m[5] * p.x + m[6] * q.y + m[7] * q.x};
             } else {
                 std::swap(x, y);
                 if (code >= kOpAnti) {
@@ -403,8 +406,8 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 // expectation values, in dense FP32 blocks 4e-7, in FP64 passes 2e-8.)
 //
 // 592 gates on 25 qubits in complex128: 8.5 ms, in dense blocks of five qubits
-// 19.6 ms; 600 gates on 16 qubits from a graph: 0.38 ms, one launch a gate
-// 1.44 ms; the 27-qubit circuit 13.7 ms, in dense blocks 19.2 ms. Vector
+// 19.6 ms; 600 gates on 16 qubits from a graph: 0.37 ms, one launch a gate
+// 1.44 ms; the 27-qubit circuit 13.4 ms, in dense blocks 19.2 ms. Vector
 // instructions bound a pass of many gates, bytes one of few.
 //
 // The first and the last round hold the top R tile qubits, the layout of the

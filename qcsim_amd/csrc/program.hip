@@ -8,7 +8,7 @@
 // owns, and its launches captured from the register's stream into a
 // hipGraph. Running it is one graph launch on the same stream, so a sequence
 // of small-state gates costs a launch for some tens of gates instead of one
-// for each (600 gates on 16 qubits: 380 us against 1442). Programs hold only
+// for each (600 gates on 16 qubits: 373 us against 1433). Programs hold only
 // gate launches (no reductions, measurements or host work) and no memset
 // nodes; a program whose register has since exchanged its state buffer
 // (qcs_swap_state) is captured again before it runs.
