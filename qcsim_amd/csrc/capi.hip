@@ -46,6 +46,7 @@ int check_launch(qcs_register* r, const char* what) {
 
 int qft_sequence(qcs_register* r, uint32_t sq, uint32_t eq, int do_swap, int inverse);
 int fuse_check(const qcs_gate* gates, uint32_t n, uint32_t width);
+int fuse_stream(const qcs_gate* gates, uint32_t n, uint32_t width, const std::function<int(const qcs_gate&)>& emit);
 
 int stage_upload(qcs_register* r, const void* src, size_t bytes, const void** dev) {
     if (bytes > r->mat_bytes) return set_error(QCS_EINVAL, "parameter block too large");
@@ -368,16 +369,20 @@ int qcs_apply_circuit(qcs_register* r, const qcs_gate* gates, uint32_t n, uint32
     for (uint32_t i = 0; i < n; ++i)
         for (uint32_t j = 0; j < gates[i].k && j < 5; ++j)
             QCS_REQUIRE(gates[i].qubits[j] < r->n, "gate %u: qubit out of range", i);
-    // Every width runs the list in passes of many gates (circuit.hip), which
+    // The list runs in passes of many gates (circuit.hip) at every width, which
     // beat dense blocks of the width: 25 qubits complex128, 592 gates, width 5
     // 20.0 ms in dense blocks, 8.5 ms in passes; 28 qubits, 252 gates 37.0
     // against 25.5 ms at most; 27 qubits complex64, 867 gates 19.2 against 13.4 ms
     // (host fusion, launches and waits included). The width stays what the
-    // caller gets told, and what is refused.
+    // caller gets told, and what is refused. Where dense blocks still win
+    // (fused_blocks), each is launched as soon as it is built.
     if (fuse_width == QCS_FUSE_AUTO) {
         std::vector<qcs_gate> fused;
         if (const int e = pick_fusion(r, gates, n, fused, &fuse_width)) return e;
         r->last_fuse_width = fuse_width;
+        if (fused_blocks(r, fuse_width)) return run_gates(r, fused.data(), uint32_t(fused.size()));
+    } else if (fused_blocks(r, fuse_width)) {
+        return fuse_stream(gates, n, fuse_width, [&](const qcs_gate& g) { return run_gates(r, &g, 1); });
     } else if (const int e = fuse_check(gates, n, fuse_width)) {
         return e;
     }

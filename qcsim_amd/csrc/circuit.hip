@@ -476,7 +476,7 @@ __global__ __launch_bounds__(1 << (kTileMax - R), 4) void k_tile(cv<T>* __restri
 #pragma unroll
         for (int i = 0; i < R; ++i)
             if (k >> i & 1) c ^= add[i];
-        return (lds_amp)(slot ^ c);
+        return (lds_amp)(uintptr_t)(slot ^ c);
     };
     layout(regs);
     uint32_t head = w[0], lane = w[1], mask = w[2], blk = w[3];

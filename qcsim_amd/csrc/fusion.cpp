@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <complex>
 #include <cstring>
+#include <functional>
 #include <vector>
 
 #include "qcsim_amd.h"
@@ -233,8 +234,7 @@ int fuse_check(const qcs_gate* gates, uint32_t n, uint32_t width) {
     return QCS_OK;
 }
 
-int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate>& out) {
-    out.clear();
+int fuse_stream(const qcs_gate* gates, uint32_t n, uint32_t width, const std::function<int(const qcs_gate&)>& emit) {
     if (const int e = fuse_check(gates, n, width)) return e;
     Pending P;
     P.mask.resize(n);
@@ -329,9 +329,18 @@ int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate
                 prev = i;
             }
         }
-        out.push_back(block_gate(gates, P, take));
+        // the block leaves (ascending indices) as one gate, at once
+        if (const int e = emit(block_gate(gates, P, take))) return e;
     }
     return QCS_OK;
+}
+
+int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate>& out) {
+    out.clear();
+    return fuse_stream(gates, n, width, [&](const qcs_gate& g) {
+        out.push_back(g);
+        return QCS_OK;
+    });
 }
 
 }  // namespace qcs

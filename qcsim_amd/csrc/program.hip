@@ -21,6 +21,7 @@
 
 namespace qcs {
 int fuse_check(const qcs_gate* gates, uint32_t n, uint32_t width);
+int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate>& out);
 
 // The inverse of a gate: conjugate transpose of its matrix; the phase of
 // the iSWAP kernels flips (their matrix is implied by the trait).
@@ -123,13 +124,16 @@ int qcs_program_create(qcs_register* r, const qcs_gate* gates, uint32_t n, uint3
     p->r = r;
     if (fuse_width >= 2) {
         std::vector<qcs_gate> fused;
-        uint32_t picked = 0;
-        const int e = fuse_width == QCS_FUSE_AUTO ? pick_fusion(r, seq.data(), uint32_t(seq.size()), fused, &picked)
-                                                  : fuse_check(seq.data(), uint32_t(seq.size()), fuse_width);
+        uint32_t picked = fuse_width;
+        const uint32_t m = uint32_t(seq.size());
+        const int e = fuse_width == QCS_FUSE_AUTO   ? pick_fusion(r, seq.data(), m, fused, &picked)
+                      : fused_blocks(r, fuse_width) ? fuse(seq.data(), m, fuse_width, fused)
+                                                    : fuse_check(seq.data(), m, fuse_width);
         if (e) {
             delete p;
             return e;
         }
+        if (fused_blocks(r, picked)) seq.swap(fused);
     }
     p->gates.swap(seq);
     for (const auto& g : p->gates) p->param_bytes += gates_param_bound(r, g);

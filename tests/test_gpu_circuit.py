@@ -130,3 +130,24 @@ def test_few_gates(n, count):
         got = np.asarray(g.getRegisterStorage())
         g.close()
         assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12, k
+
+
+@pytest.mark.parametrize("n,width", [(27, 5), (28, 4), (28, 5), (28, "auto")])
+def test_large_complex64_circuit_and_its_inverse(n, width):
+    """Where complex64 circuits go over to dense blocks: a list fused to the
+    width, then as a program with the inverse order, from |0> back to |0>. An
+    FP32 block of 32 rows errs by at most 32 * 6e-8 of an amplitude and the 30
+    gates make at most 12 blocks each way: 5e-5."""
+    rng = np.random.default_rng(n)
+    seq = [(G.SingleQubitGate(G.haar_u2(rng)), [int(q)]) for q in rng.permutation(n)[:20]]
+    for at in sorted(rng.integers(0, 20, 10), reverse=True):
+        seq.insert(int(at), (G.CNOTGate(), [int(q) for q in rng.choice(n, 2, replace=False)]))
+    g = QubitRegister(n, precision="c64")
+    g.setToBasisState(0)
+    g.apply_circuit(seq, width)
+    prog = g.compile_program(seq, width, adjoint=True)
+    prog.run()
+    amp = g.getBasisStateAmplitude(0)
+    prog.close()
+    g.close()
+    assert abs(amp - 1) < 5e-5
