@@ -21,6 +21,8 @@
 // with a fixed grid and a fixed combination order.
 #include <algorithm>
 #include <map>
+#include <set>
+#include <unordered_map>
 #include <vector>
 
 #include "common.h"
@@ -515,12 +517,33 @@ static int pauli_t(qcs_register* r, uint32_t nterms, const uint64_t* xmask, cons
     const uint32_t n = r->n, t = std::max<uint32_t>(2, std::min<uint32_t>(n, kPtMax));
     const uint64_t low = (1ull << std::min<uint32_t>(n, sizeof(T) == 8 ? 3 : 4)) - 1;
     const uint32_t ntiles = n > t ? 1u << (n - t) : 1, nb = std::min<uint32_t>(ntiles, kPtBlocks);
+    // In units of one read of the state, a slot of a tile pass costs a twelfth
+    // of the pass and 0.05 for its trips to LDS, and a pass of k_pauli 1.25 for
+    // 16 terms of one x mask. So an x mask whose terms share few slots (z masks
+    // all over the register) is faster apart, where reading counts (30 qubits,
+    // 32 random z masks with one x mask: 10.5 ms in tile passes, 5.9 apart).
+    constexpr uint32_t kApart = 10;  // slots that cost more than a pass of k_pauli
+    std::unordered_map<uint64_t, uint32_t> sharing;
+    const bool big = r->A * r->amp_bytes() > size_t(256) << 20;
+    for (uint32_t i = 0; big && i < nterms; ++i) ++sharing[xmask[i]];
+    std::map<uint64_t, bool> decided;
+    auto apart = [&](uint64_t x) {
+        const uint32_t terms = big ? sharing[x] : 0;
+        if (terms < kApart) return false;
+        const auto it = decided.find(x);
+        if (it != decided.end()) return it->second;
+        const uint64_t S = pauli_tile_qubits({x}, low, n, t);
+        std::set<std::pair<uint64_t, int>> slots;
+        for (uint32_t i = 0; i < nterms; ++i)
+            if (xmask[i] == x) slots.insert({zmask[i] & full & ~S, __builtin_popcountll(x & zmask[i]) & 1});
+        return decided[x] = (1.0 / kPtSlots + 0.05) * double(slots.size()) > 1.25 * ((terms + 15) / 16);
+    };
     std::vector<uint32_t> rest;
     std::vector<uint64_t> wide, xs;
     std::map<uint64_t, std::vector<uint32_t>> wides;
     for (uint32_t i = 0; i < nterms; ++i) {
         const uint64_t x = xmask[i];
-        if (__builtin_popcountll(x | low) <= int(t)) {
+        if (__builtin_popcountll(x | low) <= int(t) && !(x && apart(x))) {
             rest.push_back(i);
         } else {
             if (!wides.count(x)) wide.push_back(x);

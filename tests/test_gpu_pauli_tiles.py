@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from qcsim_amd import QubitRegister
+from qcsim_amd import gates as G
 from refmath import random_state
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +48,21 @@ def test_terms_equal_reference(kind, n, precision):
     want = np.array([reference(psi, x, z) for x, z in terms])
     # sums of 2^n products in FP64 whatever the state's type
     assert np.max(np.abs(got - want)) < 1e-13
+
+
+@pytest.mark.parametrize("count", [1, 9, 10, 17])
+def test_terms_of_one_x_mask_on_a_large_state(count):
+    """Above 256 MiB, terms that share an x mask but no z bits outside a tile
+    leave the tile passes from some number on: together and one by one, which
+    always is a tile pass, they are the same FP64 sums in another order."""
+    rng = np.random.default_rng(count)
+    g = QubitRegister(25)
+    g.setToEqualSuperposition()
+    for q in range(25):
+        g.ApplyGate(G.SingleQubitGate(G.haar_u2(rng)), q)
+    x = [3 << 11] * count + [1]
+    z = [int(v) for v in rng.integers(0, 1 << 25, count + 1)]
+    got = g.pauli_expectation(x, z)
+    want = [float(g.pauli_expectation([a], [b])[0]) for a, b in zip(x, z)]
+    g.close()
+    assert np.max(np.abs(got - np.array(want))) < 1e-13
