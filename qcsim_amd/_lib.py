@@ -25,6 +25,14 @@ _PU32 = C.POINTER(C.c_uint32)
 _PU64 = C.POINTER(C.c_uint64)
 
 
+class _Mat:
+    """A gate's matrix: a pointer to doubles, or their bytes."""
+
+    @staticmethod
+    def from_param(m):
+        return m if type(m) is bytes else _PD.from_param(m)
+
+
 class QcsGate(C.Structure):
     """struct qcs_gate (include/qcsim_amd.h)."""
 
@@ -51,7 +59,7 @@ SIGNATURES = {
     "qcs_set_basis_state": (_I, [_P, _U64]),
     "qcs_fill": (_I, [_P, _D, _D]),
     "qcs_scale": (_I, [_P, _D, _D]),
-    "qcs_apply_gate": (_I, [_P, _U32, _U32, _U32, _U32, _U32, _P]),  # the matrix: bytes or a pointer
+    "qcs_apply_gate": (_I, [_P, _U32, _U32, _U32, _U32, _U32, _Mat]),
     "qcs_apply_dense": (_I, [_P, _U32, _PU32, _PD]),
     "qcs_apply_circuit": (_I, [_P, C.POINTER(QcsGate), _U32, _U32]),
     "qcs_apply_diagonal": (_I, [_P, _PD, _U64]),

@@ -36,10 +36,11 @@ _C128 = np.dtype(np.complex128)
 _PAD = [(0,) * (5 - k) for k in range(6)]  # qubit slots a gate of k qubits leaves
 
 
-def _mat_bytes(m: np.ndarray) -> bytes:
-    """A matrix as the C-ABI reads it. A pointer argument takes bytes at a tenth
-    of what numpy's ctypes interface costs (0.1 against 1 us)."""
-    return m.tobytes() if m.dtype is _C128 else _mat_buf(m).tobytes()
+def _mat_bytes(m) -> bytes:
+    """A matrix, or what converts to one, as the C-ABI reads it. A pointer
+    argument takes bytes at a tenth of what numpy's ctypes interface costs (0.1
+    against 1 us)."""
+    return m.tobytes() if getattr(m, "dtype", None) is _C128 else _mat_buf(m).tobytes()
 
 
 def _mat_buf(m: np.ndarray) -> np.ndarray:
