@@ -15,67 +15,18 @@
 // small ones. The passes are bound by the vector ALUs (8 FMA per amplitude
 // and U(2)) and the LDS exchange of each round (32 B per amplitude, the price
 // of two U(2)).
-//
-// Gates commute when they act diagonally on every qubit they share, so a
-// pass takes, in list order, each gate that fits it and commutes with all
-// gates left out before it; what is left keeps its order. The gates
-// themselves are those of the gate kernels (same traits, same matrix
-// entries), applied one by one.
+// How a list is cut is in circuit_plan.cpp.
 #include <algorithm>
 #include <cstring>
 #include <vector>
 
+#include "circuit_plan.h"
 #include "common.h"
 
 namespace qcs {
 
-constexpr int kTileReg = 3;    // register qubits of a round
-constexpr int kTileMax = 12;   // tile qubits: 4096 amplitudes, 64 KiB of LDS
-
-struct TileGeo {
-    uint32_t t;
-    uint8_t pos[kTileMax + 4];  // tile qubits, ascending
-};
-
 // An amplitude: four registers in a row, as LDS reads and writes take them.
 typedef double Amp __attribute__((ext_vector_type(2)));
-
-// Operation codes of a pass's stream: base + register bit, pair or triple.
-enum : uint32_t {
-    kOpGen1 = 0,    // + J: 2x2 on register bit J (8 reals)
-    kOpReal = 4,    // + J: real 2x2 (4 reals): H, Ry
-    kOpImag = 8,    // + J: real diagonal, imaginary off-diagonal (r00, i01, i10, r11): Rx
-    kOpX = 12,      // + J: exchange
-    kOpAnti = 16,   // + J: (m01, m10)
-    kOpDiagR = 20,  // + J: (m00, m11) by register bit J
-    kOpScale = 24,  // times m0
-    kOpNeg = 25,    // sign change
-    kOpSwap = 28,   // + pair: exchange
-    kOpSwapP = 32,  // + pair: exchange times m0
-    kOpZ = 36,      // + set of register bits: times re - i im (even parity) or re + i im (odd)
-    kOpGen2 = 44,   // + pair: 4x4 (from here on handled outside the inner loop)
-    kOpGen3 = 48,   // 8x8
-    kOpRound = 49,  // the thread mask holds the register positions, a byte each
-    kOpEnd = 50,
-};
-
-// A stream is a list of records: code | words << 16, thread mask | thread
-// value << 16, register mask | kPickBit with its tile-index bit, tile-index
-// mask, then the matrix entries. An operation applies to the threads whose
-// masked bits equal the value, where every masked tile-index bit is 1, and to
-// the amplitudes (for exchanges and matrices: the orbits, by their first
-// amplitude) in the register mask. With kPickBit the second complex entry
-// takes the place of the first where that tile-index bit is 1.
-//
-// kOpZ applies to every amplitude, by the parity of its register bits, of the
-// thread bits in bits 8.. of the register mask and of the tile-index bits in
-// the low word of the third real; its factor is in the first two.
-//
-// The first round is there from the start; kOpRound begins the next one.
-// After the end come kTail words that may be read ahead.
-constexpr uint32_t kHead = 4;
-constexpr uint32_t kTail = 20;
-constexpr uint32_t kPickBit = 1u << 24;  // the bit's number at 16..20
 
 // The operations on one qubit, exchanges and factors, in place on a thread's
 // amplitudes a[0..8) for the lanes in `on`. On the device they are one
@@ -275,62 +226,8 @@ __device__ __forceinline__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t
 #undef Q_IF
 #undef Q_DONE
 #else
-// The same in C++: what the host compiler sees of the kernel, and a statement
-// of what each code does.
-__host__ __device__ inline void tile_simple(Amp (&a)[8], uint32_t code, uint32_t mask, const double (&m)[8],
-                                            uint64_t on, uint32_t tid, uint32_t tile) {
-    if (!on) return;
-    auto mul = [](Amp& x, double r, double i) { x = Amp{r * x.x - i * x.y, r * x.y + i * x.x}; };
-    for (int i = 0; i < 8; ++i) {
-        if (code >= kOpZ) {
-            const uint64_t zt = uint32_t(__builtin_bit_cast(uint64_t, m[2]));
-            const bool odd = (__builtin_popcount(i & (code - kOpZ)) + __builtin_popcount(tid & mask >> 8) +
-                              __builtin_popcount(tile & zt)) & 1;
-            mul(a[i], m[0], odd ? m[1] : -m[1]);
-            continue;
-        }
-        if (!(mask >> i & 1)) continue;
-        const uint32_t J = code & 3;  // register bit of the one-qubit codes
-        if (code < kOpDiagR) {
-            if (i >> J & 1) continue;
-            Amp &x = a[i], &y = a[i | 1 << J];
-            const Amp p = x, q = y;
-            if (code >= kOpReal && code < kOpImag) {
-                x = Amp{m[0] * p.x + m[1] * q.x, m[0] * p.y + m[1] * q.y};
-                y = Amp{m[2] * p.x + m[3] * q.x, m[2] * p.y + m[3] * q.y};
-            } else if (code >= kOpImag && code < kOpX) {
-                x = Amp{m[0] * p.x - m[1] * q.y, m[0] * p.y + m[1] * q.x};
-                y = Amp{m[3] * q.x - m[2] * p.y, m[3] * q.y + m[2] * p.x};
-            } else if (code < kOpReal) {
-                x = Amp{m[0] * p.x - m[1] * p.y + m[2] * q.x - m[3] * q.y,
-                        m[0] * p.y + m[1] * p.x + m[2] * q.y + m[3] * q.x};
-                y = Amp{m[4] * p.x - m[5] * p.y + m[6] * q.x - m[7] * q.y,
-                        m[4] * p.y + m[5] * p.x + m[6] * q.y + m[7] * q.x};
-            } else {
-                std::swap(x, y);
-                if (code >= kOpAnti) {
-                    mul(x, m[0], m[1]);
-                    mul(y, m[2], m[3]);
-                }
-            }
-        } else if (code < kOpScale) {
-            i >> J & 1 ? mul(a[i], m[2], m[3]) : mul(a[i], m[0], m[1]);
-        } else if (code == kOpScale) {
-            mul(a[i], m[0], m[1]);
-        } else if (code == kOpNeg) {
-            mul(a[i], -1, 0);
-        } else {
-            const uint32_t pair = code & 3;
-            const int A = pair == 2 ? 1 : 0, B = pair == 0 ? 1 : 2;
-            if (i >> A & 1 || i >> B & 1) continue;
-            std::swap(a[i | 1 << A], a[i | 1 << B]);
-            if (code >= kOpSwapP) {
-                mul(a[i | 1 << A], m[0], m[1]);
-                mul(a[i | 1 << B], m[0], m[1]);
-            }
-        }
-    }
-}
+__device__ void tile_simple(Amp (&a)[8], uint32_t code, uint32_t mask, const double (&m)[8], uint64_t on, uint32_t tid,
+                            uint32_t tile);
 #endif
 
 // Generic blocks: y = M x on the orbit idx[0..D), in the lanes that are on.
@@ -420,8 +317,7 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 // qubits, 14.6 on 27, 0.395 on 16.)
 template <typename T, int R, bool NT>
 __global__ __launch_bounds__(1 << (kTileMax - R), 4) void k_tile(cv<T>* __restrict__ psi, TileGeo geo,
-                                                                 const uint32_t* __restrict__ stream, uint32_t words_total,
-                                                                 uint64_t boff) {
+                                                                 const uint32_t* __restrict__ stream, uint64_t boff) {
     // aligned to its size, so that places in it are joined by XOR
     extern __shared__ __attribute__((aligned(sizeof(Amp) << kTileMax))) unsigned char smem_raw[];
     typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
@@ -536,491 +432,10 @@ __global__ __launch_bounds__(1 << (kTileMax - R), 4) void k_tile(cv<T>* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Planning (host).
-
-struct TileGate {
-    uint32_t op;          // kOpGen1, kOpX, ... (base code); kNoTile: not for a tile
-    uint32_t nt = 0;      // targets
-    uint8_t tq[3];        // in matrix bit order
-    uint64_t T = 0;       // qubits acted on other than diagonally
-    uint64_t D = 0;       // qubits acted on diagonally
-    uint64_t ctrl = 0;    // bits that must be 1
-    uint8_t nm = 0;       // matrix entries (complex)
-    double f = 1;         // fraction of the state's bytes its own launch moves
-    const qcs_gate* src = nullptr;  // null: several gates in one
-    const double* mat = nullptr;
-    uint32_t dim = 0, b0 = 0;  // matrix dimension, first row and column of its block
-};
-constexpr uint32_t kNoTile = ~0u;
-
-static hcplx entry(const TileGate& g, uint32_t r, uint32_t c) {
-    const double* m = g.mat + 2 * ((g.b0 + r) * g.dim + g.b0 + c);
-    return hcplx{m[0], m[1]};
-}
-
-static bool is(hcplx z, double re) { return z.re == re && z.im == 0.0; }
-
-// The gate as qcs_apply_gate / qcs_apply_dense dispatches it.
-static TileGate tile_gate(const qcs_gate& g) {
-    TileGate o;
-    const bool dense = (g.flags & QCS_GATE_DENSE) || g.k > 3;
-    const uint32_t t = dense ? 0 : g.traits;
-    for (uint32_t i = 0; i < g.k && i < 5; ++i) o.T |= 1ull << g.qubits[i];
-    o.op = kNoTile;
-    if (g.k > 3) return o;
-    o.mat = g.mat;
-    o.dim = 1u << g.k;
-    for (uint32_t i = 0; i < g.k; ++i) o.tq[i] = uint8_t(g.qubits[i]);
-    const bool swap = g.k >= 2 && (t & QCS_TRAIT_SWAP);
-    if (swap || (g.k == 2 && (t & (QCS_TRAIT_ISWAP | QCS_TRAIT_ISWAPDAG)))) {
-        o.op = swap ? kOpSwap : kOpSwapP;
-        o.nt = 2;
-        o.nm = swap ? 0 : 1;
-        o.b0 = t & QCS_TRAIT_ISWAP ? 1 : 0;  // sign of the factor +-i
-        o.T = 1ull << g.qubits[0] | 1ull << g.qubits[1];
-        o.ctrl = g.k == 3 ? 1ull << g.qubits[2] : 0;
-        o.D = o.ctrl;
-        o.f = g.k == 3 ? 0.25 : 0.5;
-        return o;
-    }
-    const bool two = g.k == 3 && (t & QCS_TRAIT_CONTROLLED) && (t & QCS_TRAIT_CTRL_Q1);
-    const bool one = !two && g.k >= 2 && (t & QCS_TRAIT_CONTROLLED);
-    const uint32_t nc = two ? 2 : one ? 1 : 0;
-    o.nt = g.k - nc;
-    o.b0 = o.dim - (1u << o.nt);
-    for (uint32_t i = o.nt; i < g.k; ++i) o.ctrl |= 1ull << g.qubits[i];
-    o.D = o.ctrl;
-    o.T &= ~o.ctrl;
-    o.f = nc == 2 ? 0.25 : nc == 1 ? 0.5 : 1;
-    if (o.nt > 1) {
-        o.op = o.nt == 2 ? kOpGen2 : kOpGen3;
-        o.nm = o.nt == 2 ? 16 : 64;
-    } else if (t & QCS_TRAIT_DIAGONAL) {
-        const hcplx d0 = entry(o, 0, 0), d1 = entry(o, 1, 1);
-        if (is(d0, 1)) {
-            o.op = is(d1, -1) ? kOpNeg : kOpScale;
-            o.nm = o.op == kOpScale ? 1 : 0;
-            o.ctrl |= o.T;
-            o.f *= 0.5;
-        } else {
-            o.op = !nc && d0.re == d1.re && d0.im == -d1.im ? kOpZ : kOpDiagR;
-            o.nm = 2;
-        }
-        o.D |= o.T;
-        o.T = 0;
-    } else if (t & QCS_TRAIT_ANTIDIAGONAL) {
-        o.op = is(entry(o, 0, 1), 1) && is(entry(o, 1, 0), 1) ? kOpX : kOpAnti;
-        o.nm = o.op == kOpAnti ? 2 : 0;
-    } else {
-        const hcplx a = entry(o, 0, 0), b = entry(o, 0, 1), c = entry(o, 1, 0), d = entry(o, 1, 1);
-        const bool real = a.im == 0 && b.im == 0 && c.im == 0 && d.im == 0;
-        const bool imag = a.im == 0 && b.re == 0 && c.re == 0 && d.im == 0;
-        o.op = real ? kOpReal : imag ? kOpImag : kOpGen1;
-        o.nm = real || imag ? 2 : 4;
-    }
-    return o;
-}
-
-static int popc(uint64_t x) { return __builtin_popcountll(x); }
-
-// CNOT(c, t) Z CNOT(c, t), with Z = exp(i phi) or its conjugate by the parity
-// of qubits that include t, is such a gate too, in the parity that c joins or
-// leaves: the Rz between two CNOTs of an Ising step, and the ladders around
-// the rotations of Pauli strings. Each such sandwich becomes one gate: the
-// same factor on the same amplitude (CNOTs move amplitudes unchanged), and a
-// gate that any round can take. The gates that are left stay in order.
-static std::vector<TileGate> tile_gates(const qcs_gate* gates, uint32_t n, uint32_t nq) {
-    std::vector<TileGate> g;
-    std::vector<uint8_t> gone;
-    std::vector<std::vector<int>> on(nq);  // per qubit, the gates left that touch it
-    g.reserve(n);
-    auto drop = [&](uint32_t q, int i) { on[q].erase(std::find(on[q].begin(), on[q].end(), i)); };
-    for (uint32_t k = 0; k < n; ++k) {
-        const TileGate o = tile_gate(gates[k]);
-        if (o.op == kOpX && popc(o.ctrl) == 1) {
-            const uint32_t t = o.tq[0], c = uint32_t(__builtin_ctzll(o.ctrl));
-            auto& ot = on[t];
-            auto& oc = on[c];
-            const int d = ot.size() > 1 ? ot.back() : -1, x = d >= 0 ? ot[ot.size() - 2] : -1;
-            if (d >= 0 && g[x].op == kOpX && g[x].T == o.T && g[x].ctrl == o.ctrl) {
-                TileGate& D = g[d];
-                const bool has = D.D >> c & 1;
-                if (D.op == kOpZ && (has ? oc.size() > 1 && oc.back() == d && oc[oc.size() - 2] == x : oc.back() == x)) {
-                    drop(t, x);
-                    drop(c, x);
-                    gone[x] = 1;
-                    D.src = nullptr;
-                    D.D ^= 1ull << c;
-                    if (has)
-                        drop(c, d);
-                    else
-                        oc.push_back(d);
-                    continue;
-                }
-            }
-        }
-        for (uint64_t m = o.T | o.D; m; m &= m - 1) on[__builtin_ctzll(m)].push_back(int(g.size()));
-        g.push_back(o);
-        g.back().src = &gates[k];
-        gone.push_back(0);
-    }
-    size_t kept = 0;
-    for (size_t i = 0; i < g.size(); ++i)
-        if (!gone[i]) g[kept++] = g[i];
-    g.resize(kept);
-    return g;
-}
-
-// Gates in order with what each still waits for: a linked list of the gates
-// not placed yet.
-struct TilePlan {
-    std::vector<TileGate> g;
-    std::vector<int> next;
-    int head = -1;
-    uint32_t n = 0, t = 0;
-    uint64_t all = 0, low = 0;
-    size_t max_bytes = 0;  // of a pass's stream
-
-    size_t op_bytes(const TileGate& o) const {
-        return (kHead * 4 + 16 * o.nm + 15) / 16 * 16 + (!o.T ? 64 : 0);
-    }
-};
-
-// Gates, in order, that can run inside S before every gate left out: a gate
-// left out blocks the qubits it touches, for diagonal action only where it
-// acts diagonally itself. Returns their summed worth.
-static double tile_scan(const TilePlan& P, uint64_t S, std::vector<int>* take) {
-    uint64_t bT = 0, bD = 0;
-    double worth = 0;
-    size_t bytes = 0;
-    int left = 0;
-    const int most = int(6 * P.n) + 16;
-    for (int i = P.head; i >= 0; i = P.next[i]) {
-        const TileGate& o = P.g[i];
-        if (!(o.T & (bT | bD | ~S)) && !(o.D & bT) && o.op != kNoTile) {
-            bytes += P.op_bytes(o) + 2 * kHead * 4;
-            if (bytes > P.max_bytes) break;
-            worth += o.f;
-            if (take) take->push_back(i);
-            continue;
-        }
-        bT |= o.T;
-        bD |= o.D;
-        if (!(P.all & ~bT) || ++left > most) break;
-    }
-    return worth;
-}
-
-// The tile qubits of the next pass: the lowest ones, for whole memory lines,
-// and then, from several seeds, the qubit most tied to those already chosen
-// by the next gates (a gate of two qubits ties them, the less the more gates
-// of two qubits either has before it; a gate on one qubit counts for itself).
-static uint64_t tile_choose(const TilePlan& P) {
-    if (P.n <= P.t) return P.all;
-    constexpr float kFade = 0.6f;
-    const uint32_t n = P.n;
-    std::vector<float> tie(size_t(n) * n, 0.f), self(n, 0.f), fade(n, 1.f);
-    uint64_t seeds[6], seen = 0;
-    int ns = 0, looked = 0;
-    for (int i = P.head; i >= 0 && looked < int(8 * n); i = P.next[i], ++looked) {
-        const TileGate& o = P.g[i];
-        const uint64_t m = o.T | o.D;
-        if (!o.T || o.op == kNoTile) continue;
-        float w = 1.f;
-        for (uint64_t x = m; x; x &= x - 1) w = std::min(w, fade[__builtin_ctzll(x)]);
-        if (popc(m) == 1) {
-            self[__builtin_ctzll(m)] += w;
-            continue;
-        }
-        for (uint64_t x = m; x; x &= x - 1) {
-            const int q = __builtin_ctzll(x);
-            for (uint64_t y = m & ~(1ull << q); y; y &= y - 1) tie[size_t(q) * n + __builtin_ctzll(y)] += w;
-            fade[q] = w * kFade;
-        }
-        if (ns < 6 && !(m & seen) && popc(m | P.low) <= int(P.t)) seeds[ns++] = m;
-        seen |= m;
-    }
-    if (!ns) seeds[ns++] = 0;
-    uint64_t best = 0;
-    double best_worth = -1;
-    std::vector<float> gain(n);
-    for (int k = 0; k < ns; ++k) {
-        uint64_t S = 0;
-        std::copy(self.begin(), self.end(), gain.begin());
-        auto add = [&](uint32_t q) {
-            S |= 1ull << q;
-            for (uint32_t p = 0; p < n; ++p) gain[p] += tie[size_t(q) * n + p];
-        };
-        for (uint64_t x = P.low | seeds[k]; x; x &= x - 1) add(__builtin_ctzll(x));
-        while (popc(S) < int(P.t)) {
-            int q = -1;
-            for (uint32_t p = 0; p < n; ++p)
-                if (!(S >> p & 1) && (q < 0 || gain[p] > gain[q])) q = int(p);
-            add(uint32_t(q));
-        }
-        const double w = tile_scan(P, S, nullptr);
-        if (w > best_worth) {
-            best_worth = w;
-            best = S;
-        }
-    }
-    return best;
-}
-
-// Rounds of one pass: the same rule over the pass's gates, R register qubits
-// at a time.
-struct TileRound {
-    uint64_t regs;
-    std::vector<int> ops;  // indices into the pass's gates
-};
-
-static int round_scan(const std::vector<const TileGate*>& g, const std::vector<int>& rest, uint64_t S,
-                      std::vector<int>* take) {
-    uint64_t bT = 0, bD = 0, live = S;
-    int worth = 0;
-    for (const int i : rest) {
-        const TileGate& o = *g[i];
-        if (!(o.T & (bT | bD | ~S)) && !(o.D & bT)) {
-            worth += o.op <= kOpImag ? 2 : o.nt > 1 ? 3 : 1;
-            if (take) take->push_back(i);
-            continue;
-        }
-        bT |= o.T;
-        bD |= o.D;
-        live &= ~(bT | bD);
-        if (!take && !live) break;
-    }
-    return worth;
-}
-
-static std::vector<TileRound> tile_rounds(const std::vector<const TileGate*>& g, uint64_t tile, uint64_t top) {
-    std::vector<TileRound> out;
-    std::vector<int> rest(g.size()), take, keep;
-    for (size_t i = 0; i < g.size(); ++i) rest[i] = int(i);
-    auto place = [&](uint64_t regs) {
-        take.clear();
-        round_scan(g, rest, regs, &take);
-        keep.clear();
-        std::set_difference(rest.begin(), rest.end(), take.begin(), take.end(), std::back_inserter(keep));
-        rest.swap(keep);
-        out.push_back(TileRound{regs, take});
-    };
-    place(top);
-    while (!rest.empty()) {
-        take.clear();
-        round_scan(g, rest, top, &take);
-        if (take.size() == rest.size()) break;  // the last round takes them
-        // seeds: the qubits of the first gates that could run, each completed
-        // by the qubit that lets the most gates run
-        uint64_t best = 0, bT = 0, bD = 0, tried[8];
-        int best_worth = -1, nt = 0;
-        for (size_t k = 0; k < rest.size() && nt < 8; ++k) {
-            const TileGate& o = *g[rest[k]];
-            const bool free = !(o.T & (bT | bD)) && !(o.D & bT);
-            bT |= o.T;
-            bD |= o.D;
-            if (!o.T || !free) {
-                if (!o.T && free && best_worth < 0) {  // only diagonal gates so far: any registers do
-                    best = top;
-                    best_worth = 0;
-                }
-                if (!(tile & ~bT)) break;
-                continue;
-            }
-            uint64_t seed = o.T;
-            for (uint64_t x = o.D & tile; x && popc(seed) < kTileReg; x &= x - 1) seed |= x & -x;
-            bool again = false;
-            for (int j = 0; j < nt; ++j) again = again || tried[j] == seed;
-            if (again) continue;
-            tried[nt++] = seed;
-            while (popc(seed) < kTileReg) {
-                // partners: qubits that the next gates tie to the seed, else any with a gate
-                uint64_t cand = 0;
-                int looked = 0;
-                for (const int i : rest) {
-                    const uint64_t m = g[i]->T | g[i]->D;
-                    if ((m & seed) && (m & ~seed)) cand |= m;
-                    if (++looked > 40) break;
-                }
-                cand &= tile & ~seed;
-                if (!cand) {
-                    for (const int i : rest) cand |= g[i]->T & ~seed;
-                    cand &= tile;
-                }
-                if (!cand) cand = tile & ~seed;
-                uint64_t grown = 0;
-                int w = -1;
-                for (uint64_t x = cand; x; x &= x - 1) {
-                    const int c = round_scan(g, rest, seed | (x & -x), nullptr);
-                    if (c > w) {
-                        w = c;
-                        grown = seed | (x & -x);
-                    }
-                }
-                seed = grown;
-            }
-            const int w = round_scan(g, rest, seed, nullptr);
-            if (w > best_worth) {
-                best_worth = w;
-                best = seed;
-            }
-        }
-        place(best);
-    }
-    if (!rest.empty() || out.back().regs != top) place(top);
-    return out;
-}
-
-// A pass's stream in words, appended to `out`.
-static void tile_emit(const std::vector<const TileGate*>& g, const std::vector<TileRound>& rounds, uint64_t tile,
-                      uint32_t n, std::vector<uint32_t>& out) {
-    uint8_t local[64], blkbit[64];  // tile position of a qubit; tile-index bit of an outside one
-    for (uint32_t q = 0, i = 0, b = 0; q < n; ++q) {
-        if (tile >> q & 1)
-            local[q] = uint8_t(i++);
-        else
-            blkbit[q] = uint8_t(b++);
-    }
-    for (const TileRound& rd : rounds) {
-        uint8_t rq[kTileReg];
-        uint32_t packed = 0;
-        int nr = 0;
-        for (uint64_t x = rd.regs; x; x &= x - 1) {
-            rq[nr] = uint8_t(__builtin_ctzll(x));
-            packed |= uint32_t(local[rq[nr]]) << (8 * nr);
-            ++nr;
-        }
-        if (&rd != &rounds.front()) out.insert(out.end(), {kOpRound | kHead << 16, packed, 0, 0});
-        auto regbit = [&](uint32_t q) {
-            for (int i = 0; i < kTileReg; ++i)
-                if (rq[i] == q) return i;
-            return -1;
-        };
-        auto lanebit = [&](uint32_t q) {
-            uint32_t b = local[q];
-            for (int i = 0; i < kTileReg; ++i) b -= local[rq[i]] < local[q] ? 1 : 0;
-            return b;
-        };
-        for (const int oi : rd.ops) {
-            const TileGate& o = *g[oi];
-            uint32_t lane = 0, blk = 0, rmask = 0, rc = 0, code = o.op;
-            for (uint64_t x = o.ctrl; x; x &= x - 1) {
-                const uint32_t q = uint32_t(__builtin_ctzll(x));
-                if (!(tile >> q & 1))
-                    blk |= 1u << blkbit[q];
-                else if (regbit(q) >= 0)
-                    rc |= 1u << regbit(q);
-                else
-                    lane |= 1u << lanebit(q);
-            }
-            for (uint32_t i = 0; i < 1u << kTileReg; ++i) rmask |= (i & rc) == rc ? 1u << i : 0;
-            double v[128];
-            int nv = 0;
-            auto put = [&](hcplx z) {
-                v[nv++] = z.re;
-                v[nv++] = z.im;
-            };
-            auto record = [&](uint32_t lval) {
-                const size_t body = (sizeof(double) * nv + 15) / 16 * 4, at = out.size();
-                out.resize(at + kHead + body, 0);
-                out[at] = code | uint32_t(kHead + body) << 16;
-                out[at + 1] = lane | lval << 16;
-                out[at + 2] = rmask;
-                out[at + 3] = blk;
-                if (nv) std::memcpy(&out[at + kHead], v, sizeof(double) * nv);
-                nv = 0;
-            };
-            if (o.op == kOpGen1) {
-                code += uint32_t(regbit(o.tq[0]));
-                for (uint32_t r = 0; r < 2; ++r)
-                    for (uint32_t c = 0; c < 2; ++c) put(entry(o, r, c));
-            } else if (o.op == kOpReal || o.op == kOpImag) {
-                code += uint32_t(regbit(o.tq[0]));
-                const bool im = o.op == kOpImag;
-                put(hcplx{entry(o, 0, 0).re, im ? entry(o, 0, 1).im : entry(o, 0, 1).re});
-                put(hcplx{im ? entry(o, 1, 0).im : entry(o, 1, 0).re, entry(o, 1, 1).re});
-            } else if (o.op == kOpX || o.op == kOpAnti) {
-                code += uint32_t(regbit(o.tq[0]));
-                if (o.op == kOpAnti) {
-                    put(entry(o, 0, 1));
-                    put(entry(o, 1, 0));
-                }
-            } else if (o.op == kOpZ) {
-                uint32_t zr = 0, zl = 0, zt = 0;
-                for (uint64_t x = o.D; x; x &= x - 1) {
-                    const uint32_t q = uint32_t(__builtin_ctzll(x));
-                    if (!(tile >> q & 1))
-                        zt |= 1u << blkbit[q];
-                    else if (regbit(q) >= 0)
-                        zr |= 1u << regbit(q);
-                    else
-                        zl |= 1u << lanebit(q);
-                }
-                code += zr;
-                rmask = zl << 8;
-                put(entry(o, 1, 1));
-                const uint64_t bits = zt;
-                std::memcpy(&v[nv], &bits, sizeof bits);
-                nv += 2;
-                v[3] = 0;
-            } else if (o.op == kOpDiagR) {
-                const uint32_t q = o.tq[0];
-                put(entry(o, 0, 0));
-                if ((tile >> q & 1) && regbit(q) < 0) {  // a thread bit: one record per value
-                    const uint32_t l0 = lane;
-                    code = kOpScale;
-                    lane |= 1u << lanebit(q);
-                    record(l0);
-                    put(entry(o, 1, 1));
-                } else {
-                    put(entry(o, 1, 1));
-                    if (tile >> q & 1) {
-                        code += uint32_t(regbit(q));
-                    } else {
-                        code = kOpScale;
-                        rmask |= kPickBit | uint32_t(blkbit[q]) << 16;
-                    }
-                }
-            } else if (o.op == kOpScale) {
-                put(entry(o, 1, 1));
-            } else if (o.op == kOpSwap || o.op == kOpSwapP || o.op == kOpGen2) {
-                int a = regbit(o.tq[0]), b = regbit(o.tq[1]);
-                const bool flip = a > b;  // matrix bit 0 on the higher register bit
-                if (flip) std::swap(a, b);
-                code += uint32_t(a == 0 ? b - 1 : 2);
-                if (o.op == kOpSwapP) put(hcplx{0, o.b0 ? 1.0 : -1.0});
-                if (o.op == kOpGen2)
-                    for (uint32_t r = 0; r < 4; ++r)
-                        for (uint32_t c = 0; c < 4; ++c) {
-                            auto sw = [&](uint32_t x) { return flip ? (x >> 1 | (x & 1) << 1) : x; };
-                            put(entry(o, sw(r), sw(c)));
-                        }
-            } else if (o.op == kOpGen3) {
-                int at[3];  // register bit of matrix bit i
-                for (int i = 0; i < 3; ++i) at[i] = regbit(o.tq[i]);
-                auto perm = [&](uint32_t x) {
-                    uint32_t y = 0;
-                    for (int i = 0; i < 3; ++i) y |= (x >> at[i] & 1) << i;
-                    return y;
-                };
-                for (uint32_t r = 0; r < 8; ++r)
-                    for (uint32_t c = 0; c < 8; ++c) put(entry(o, perm(r), perm(c)));
-            }
-            record(lane);
-        }
-    }
-    out.insert(out.end(), {kOpEnd, 0, 0, 0});
-    out.resize(out.size() + kTail, 0);
-}
-
-// Tile width for an n-qubit register: the whole register while one tile
-// holds it, then as wide as leaves 2^8 tiles (one per CU).
-static uint32_t tile_width(uint32_t n) {
-    return n <= 10 ? n : std::min<uint32_t>(kTileMax, std::max<uint32_t>(10, n - 8));
-}
+// Host side.
 
 template <typename T>
-static int tile_launch(qcs_register* r, const TileGeo& geo, const uint32_t* stream, uint32_t words, bool nt) {
+static int tile_launch(qcs_register* r, const TileGeo& geo, const uint32_t* stream, bool nt) {
     const uint64_t tiles = r->A >> geo.t;
     const unsigned threads = std::max(64u, 1u << (geo.t - kTileReg));
     const size_t shm = std::max<size_t>(sizeof(Amp) << geo.t, sizeof(Amp) * threads << kTileReg);
@@ -1028,10 +443,10 @@ static int tile_launch(qcs_register* r, const TileGeo& geo, const uint32_t* stre
         const unsigned grid = unsigned(std::min(kMaxBlocks, tiles - boff));
         if (nt)
             hipLaunchKernelGGL((k_tile<T, kTileReg, true>), dim3(grid), dim3(threads), shm, r->stream,
-                               static_cast<cv<T>*>(r->psi), geo, stream, words, boff);
+                               static_cast<cv<T>*>(r->psi), geo, stream, boff);
         else
             hipLaunchKernelGGL((k_tile<T, kTileReg, false>), dim3(grid), dim3(threads), shm, r->stream,
-                               static_cast<cv<T>*>(r->psi), geo, stream, words, boff);
+                               static_cast<cv<T>*>(r->psi), geo, stream, boff);
     }
     return check_launch(r, "k_tile");
 }
@@ -1062,22 +477,10 @@ size_t gates_param_bound(const qcs_register* r, const qcs_gate& g) {
 
 template <typename T>
 static int run_tiles(qcs_register* r, const qcs_gate* gates, uint32_t n) {
-    TilePlan P;
-    P.n = r->n;
-    P.t = tile_width(r->n);
-    P.all = r->n >= 64 ? ~0ull : (1ull << r->n) - 1;
-    const bool big = r->A * r->amp_bytes() > (size_t(64) << 20);
-    P.low = (1ull << std::min<uint32_t>(r->n, big ? (sizeof(T) == 8 ? 4 : 5) : (sizeof(T) == 8 ? 3 : 4))) - 1;
-    P.max_bytes = r->mat_bytes - 256;
-    P.g = tile_gates(gates, n, r->n);
-    P.next.resize(P.g.size());
-    for (size_t i = 0; i < P.g.size(); ++i) P.next[i] = i + 1 < P.g.size() ? int(i + 1) : -1;
-    P.head = P.g.empty() ? -1 : 0;
-
+    TilePlanner plan(gates, n, r->n, r->amp_bytes(), r->mat_bytes - 256);
     struct Pass {
         TileGeo geo;
-        size_t at;       // first word of its stream
-        uint32_t words;  // its length
+        size_t at;  // first word of its stream
     };
     std::vector<Pass> passes;
     std::vector<uint32_t> words, one;
@@ -1087,54 +490,23 @@ static int run_tiles(qcs_register* r, const qcs_gate* gates, uint32_t n) {
         const void* dev = nullptr;
         if (const int e = stage_upload(r, words.data(), words.size() * 4, &dev)) return e;
         for (const Pass& p : passes)
-            if (const int e = tile_launch<T>(r, p.geo, static_cast<const uint32_t*>(dev) + p.at, p.words, big))
-                return e;
+            if (const int e = tile_launch<T>(r, p.geo, static_cast<const uint32_t*>(dev) + p.at, plan.big())) return e;
         passes.clear();
         words.clear();
         batch *= 2;
         return QCS_OK;
     };
-    std::vector<int> take;
-    std::vector<const TileGate*> local;
-    while (P.head >= 0) {
-        const uint64_t S = tile_choose(P);
-        take.clear();
-        const double worth = tile_scan(P, S, &take);
-        // A pass moves the whole state once: it has to replace launches that
-        // move more. Where launches cost more than bytes it has to replace
-        // three (us for 2 / 3 / 5 gates on 16 qubits, launches against passes:
-        // 10 / 14 / 23 against 12 / 13 / 14; on 20 qubits 15 / 18 / 37 against
-        // 18 / 18 / 23; on 25 qubits, by worth, 208 / 382 / 602 against
-        // 177 / 211 / 225).
-        const bool pass = P.g[P.head].op != kNoTile && (!P.g[P.head].src || (big ? worth > 1.2 : take.size() > 2));
-        if (!pass) take.assign(1, P.head);
-        int prev = -1;
-        size_t k = 0;
-        for (int i = P.head; i >= 0 && k < take.size(); i = P.next[i]) {
-            if (i == take[k]) {
-                ++k;
-                (prev < 0 ? P.head : P.next[prev]) = P.next[i];
-            } else {
-                prev = i;
-            }
-        }
-        if (!pass) {
+    Pass p{};
+    const qcs_gate* single = nullptr;
+    while (plan.next(p.geo, one, &single)) {
+        if (single) {
             if (const int e = flush()) return e;
-            if (const int e = apply_one(r, *P.g[take[0]].src)) return e;
+            if (const int e = apply_one(r, *single)) return e;
             continue;
         }
-        local.clear();
-        for (const int i : take) local.push_back(&P.g[i]);
-        Pass p{};
-        uint64_t top = S;
-        for (uint64_t x = S; x; x &= x - 1) p.geo.pos[p.geo.t++] = uint8_t(__builtin_ctzll(x));
-        while (popc(top) > kTileReg) top &= top - 1;
-        one.clear();
-        tile_emit(local, tile_rounds(local, S, top), S, r->n, one);
         if ((words.size() + one.size()) * 4 > r->mat_bytes)
             if (const int e = flush()) return e;
         p.at = words.size();
-        p.words = uint32_t(one.size());
         words.insert(words.end(), one.begin(), one.end());
         passes.push_back(p);
         if (passes.size() >= batch)

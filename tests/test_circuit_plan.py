@@ -1,0 +1,101 @@
+"""Tile passes planned and run in host memory: the planner of
+qcsim_amd/csrc/circuit_plan.cpp with tests/cpp/circuit_host.cpp, which states
+in C++ what each operation of a pass does, against the oracle."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from gatecatalog import catalog
+from qcsim_amd import QubitRegister
+from refmath import random_state
+from test_gpu_circuit import circuit, ladder, run_oracle
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+STREAM = 64 * 64 * 8 - 256  # a register's staging slot, less its rounding
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("plan") / "libcircuit_host.so")
+    src = [os.path.join(ROOT, p) for p in ("tests/cpp/circuit_host.cpp", "qcsim_amd/csrc/circuit_plan.cpp")]
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", "-I", os.path.join(ROOT, "include"),
+                    *src, "-o", lib], check=True)
+    L = C.CDLL(lib)
+    L.plan_new.restype, L.plan_new.argtypes = C.c_void_p, [C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint64, C.c_uint64]
+    L.plan_free.restype, L.plan_free.argtypes = None, [C.c_void_p]
+    L.plan_step.restype = C.c_int64
+    L.plan_step.argtypes = [C.c_void_p, C.c_void_p, C.c_uint32, C.c_void_p, C.POINTER(C.c_uint64)]
+    return L
+
+
+def steps(host, arr, count, nq, amp_bytes=16, stream=STREAM, psi=None, single=None):
+    """(passes, gates by themselves, the longest stream); psi is updated in place."""
+    plan = host.plan_new(arr, count, nq, amp_bytes, stream)
+    passes, alone, longest = 0, 0, 0
+    nbytes = C.c_uint64()
+    while True:
+        k = host.plan_step(plan, arr, nq, None if psi is None else psi.ctypes.data, C.byref(nbytes))
+        if k == -1:
+            break
+        if k == -2:
+            passes += 1
+            longest = max(longest, nbytes.value)
+        else:
+            alone += 1
+            if single:
+                single(int(k))
+    host.plan_free(plan)
+    return passes, alone, longest
+
+
+def run_planned(host, psi, n, seq, **kw):
+    out = np.ascontiguousarray(psi, dtype=np.complex128).copy()
+
+    def single(k):
+        out[:] = run_oracle(out, n, [seq[k]])
+
+    return out, steps(host, QubitRegister._gate_array(seq), len(seq), n, psi=out, single=single, **kw)
+
+
+# amp_bytes 8192: as for a register above 64 MiB, whose few gates launch by themselves
+@pytest.mark.parametrize("amp_bytes", [16, 8, 8192])
+@pytest.mark.parametrize("n,blocks", [(3, False), (4, True), (5, False), (9, False), (10, True), (11, False), (13, True),
+                                      (14, False)])
+def test_passes_equal_oracle(host, n, blocks, amp_bytes):
+    rng = np.random.default_rng(1000 * n + amp_bytes)
+    psi = random_state(rng, n)
+    seq = circuit(rng, n, blocks)
+    got, (passes, alone, longest) = run_planned(host, psi, n, seq, amp_bytes=amp_bytes)
+    assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12
+    assert passes and longest <= STREAM + 256 and alone >= 2 * blocks * (n >= 5)
+
+
+@pytest.mark.parametrize("stream", [2048, 4096])
+def test_passes_keep_to_the_stream(host, stream):
+    """A short staging slot makes more passes, none longer than it."""
+    n = 7
+    rng = np.random.default_rng(stream)
+    psi = random_state(rng, n)
+    seq = circuit(rng, n, False)
+    got, (passes, _, longest) = run_planned(host, psi, n, seq, stream=stream)
+    assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12
+    assert passes > 2 and longest <= stream + 256
+
+
+@pytest.mark.parametrize("n", [4, 12])
+def test_long_lists(host, n):
+    """Thousands of gates, with ladders among them."""
+    rng = np.random.default_rng(n)
+    one, two, three = catalog(n)
+    fams = one + two + three
+    seq = []
+    while len(seq) < 5000:
+        seq += ladder(rng, n)
+        _, gate = fams[int(rng.integers(len(fams)))]
+        seq.append((gate, [int(x) for x in rng.choice(n, size=gate.getQubitsNumber(), replace=False)]))
+    psi = random_state(rng, n)
+    got, _ = run_planned(host, psi, n, seq)
+    assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12
