@@ -102,7 +102,10 @@ static TileGate tile_gate(const qcs_gate& g) {
 
 static int popc(uint64_t x) { return __builtin_popcountll(x); }
 
-// Gates in order, doubly linked, those not placed yet.
+// Gates in order, doubly linked, those not placed yet. They are taken in as the
+// passes need them: a pass looks no further ahead than its stream has room for
+// plus what it may leave out, so that the first pass of a long list goes out as
+// soon as that of a short one.
 struct TilePlanner::Plan {
     const qcs_gate* gates = nullptr;
     uint32_t count = 0, at = 0;  // of the caller's list; the next one to take in
@@ -132,7 +135,8 @@ struct TilePlanner::Plan {
 };
 typedef TilePlanner::Plan TilePlan;
 
-constexpr uint32_t kAhead = ~0u;  // the whole list at once
+// Gates that a pass can see: 48 B of stream each at least, and 6 n + 16 left out.
+constexpr uint32_t kAhead = 2048;
 
 // CNOT(c, t) Z CNOT(c, t), with Z = exp(i phi) or its conjugate by the parity
 // of qubits that include t, is such a gate too, in the parity that c joins or
@@ -151,13 +155,14 @@ void TilePlan::add(const qcs_gate& gate) {
             TileGate& D = g[d];
             const bool has = D.D >> c & 1;
             if (D.op == kOpZ && (has ? oc.size() > 1 && oc.back() == d && oc[oc.size() - 2] == x : oc.back() == x)) {
-                ot.erase(std::find(ot.begin(), ot.end(), x));
-                oc.erase(std::find(oc.begin(), oc.end(), x));
+                // of the two qubits' lists these are the last two entries
+                ot.erase(ot.end() - 2);
+                oc.erase(oc.end() - (has ? 2 : 1));
                 remove(x);
                 D.src = nullptr;
                 D.D ^= 1ull << c;
                 if (has)
-                    oc.erase(std::find(oc.begin(), oc.end(), d));
+                    oc.pop_back();
                 else
                     oc.push_back(d);
                 return;

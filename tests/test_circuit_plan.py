@@ -4,12 +4,15 @@ in C++ what each operation of a pass does, against the oracle."""
 import ctypes as C
 import os
 import subprocess
+import time
 
 import numpy as np
 import pytest
 
 from gatecatalog import catalog
 from qcsim_amd import QubitRegister
+from qcsim_amd import gates as G
+from qcsim_amd._lib import QcsGate
 from refmath import random_state
 from test_gpu_circuit import circuit, ladder, run_oracle
 
@@ -87,7 +90,8 @@ def test_passes_keep_to_the_stream(host, stream):
 
 @pytest.mark.parametrize("n", [4, 12])
 def test_long_lists(host, n):
-    """Thousands of gates, with ladders among them."""
+    """More gates than the planner takes in at once, with ladders across the
+    places where it goes on."""
     rng = np.random.default_rng(n)
     one, two, three = catalog(n)
     fams = one + two + three
@@ -99,3 +103,38 @@ def test_long_lists(host, n):
     psi = random_state(rng, n)
     got, _ = run_planned(host, psi, n, seq)
     assert np.max(np.abs(got - run_oracle(psi, n, seq))) < 1e-12
+
+
+def test_planning_grows_with_the_list(host):
+    """Ising steps on few qubits, each CNOT, Rz, CNOT one gate to the planner.
+    The time of the whole plan is proportional to the list, and that of its
+    first pass does not depend on it (a factor of five left for the clock)."""
+    n, rng = 4, np.random.default_rng(1)
+    seq = []
+    while len(seq) < 2000:
+        q = int(rng.integers(n - 1))
+        seq += [(G.CNOTGate(), [q + 1, q]), (G.RzGate(0.1), [q + 1]), (G.CNOTGate(), [q + 1, q])]
+        seq.append((G.RxGate(0.2), [int(rng.integers(n))]))
+    long = 32
+    arr = (QcsGate * (long * len(seq)))()
+    one = QubitRegister._gate_array(seq)
+    head = 32 + 2 * 16 * 8  # header and a 4 x 4 matrix; the rest of a gate stays untouched
+    for r in range(long):
+        for i in range(len(seq)):
+            C.memmove(C.byref(arr[r * len(seq) + i]), C.byref(one[i]), head)
+
+    def best(count, first):
+        times = []
+        for _ in range(5):
+            t = time.perf_counter()
+            if first:
+                plan = host.plan_new(arr, count, n, 16, STREAM)
+                assert host.plan_step(plan, arr, n, None, C.byref(C.c_uint64())) == -2
+                host.plan_free(plan)
+            else:
+                steps(host, arr, count, n)
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    assert best(long * len(seq), False) < 5 * long * best(len(seq), False)
+    assert best(long * len(seq), True) < 5 * best(len(seq), True)
