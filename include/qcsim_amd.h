@@ -114,15 +114,15 @@ int qcs_apply_dense(qcs_register* r, uint32_t k, const uint32_t* qubits,
  * whatever the width. fuse_width 0/1 takes the gates as they come (a refused
  * gate ends the batch after those before it); with 2..5 a list that the
  * fusion pass (qcs_fuse) refuses at that width is refused whole, and
- * QCS_FUSE_AUTO also reports the width (0 or 2..5) whose blocks would cost
- * least under the fusion cost table (qcs_autotune_fusion, measured on first
- * use for this precision and qubit count). No counterpart in the reference,
- * which applies gates one by one (QubitRegister.h:488-492). */
+ * QCS_FUSE_AUTO leaves the width to the library. No counterpart in the
+ * reference, which applies gates one by one (QubitRegister.h:488-492). */
 #define QCS_FUSE_AUTO 0xFFFFFFFFu
 int qcs_apply_circuit(qcs_register* r, const qcs_gate* gates, uint32_t n,
                       uint32_t fuse_width);
-/* The width of the last qcs_apply_circuit on r (0: none; QCS_FUSE_AUTO's
- * choice). */
+/* The width of the last qcs_apply_circuit on r. With QCS_FUSE_AUTO that of the
+ * dense blocks it ran in; where it ran in passes, the one whose blocks would
+ * cost least under the cost table of this precision and qubit count
+ * (qcs_autotune_fusion, qcs_set_fusion_costs), or 0 without a table. */
 uint32_t qcs_last_fuse_width(const qcs_register* r);
 
 /* The fusion pass alone (host only, no device): rewrites `gates` into at

@@ -18,7 +18,6 @@
 #include <atomic>
 #include <functional>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "common.h"
@@ -120,20 +119,17 @@ extern "C" int qcs_get_tuned_variant(int precision, uint32_t n, uint32_t q) {
 }
 
 // ---------------------------------------------------------------------------
-// Fusion width. A circuit runs fastest at the fusion width whose blocks cost
-// least in total: wider blocks mean fewer passes over the state, but a dense
-// k-qubit pass costs more than a plain gate once its 8 * 2^k FLOP per
-// amplitude approach the matrix cores' rate. The cost of each pass kind is
-// measured on the register's own buffer (identity matrices: the state keeps
-// its values) and kept per (precision, n): t[0] for a generic 1-qubit gate,
-// t[k] for a dense k-qubit block (k = 2..5). A gate that changes a fraction
-// f of the amplitudes is priced at f * t[0] (2- and 3-qubit gates without
-// control structure at t[k]); the width with the lowest predicted total is
-// used.
+// Fusion width. The cost of each kind of launch is measured on the register's
+// own buffer (identity matrices: the state keeps its values) and kept per
+// (precision, n): t[0] for a generic 1-qubit gate, t[k] for a dense k-qubit
+// block (k = 2..5). A gate that changes a fraction f of the amplitudes is priced
+// at f * t[0] (2- and 3-qubit gates without control structure at t[k]). The
+// width that QCS_FUSE_AUTO reports where a list runs in tile passes is the one
+// with the lowest total; how a list runs does not depend on the table.
 
 namespace qcs {
 int kdense(qcs_register* r, uint32_t k, const uint32_t* qubits, const double* mat_host);
-int fuse(const qcs_gate* gates, uint32_t n, uint32_t width, std::vector<qcs_gate>& out);
+double fuse_estimate(const qcs_gate* gates, uint32_t n, uint32_t width);
 
 static std::mutex g_fuse_mu;
 static double g_fuse_cost[2][kMaxN + 1][6];  // ms; 0 = not measured
@@ -226,45 +222,24 @@ int autotune_fusion(qcs_register* r, uint32_t reps, double* out6) {
     return QCS_OK;
 }
 
-// The fused sequence of the cheapest width (0 = unfused, else 2..5) under
-// the measured costs; measures them first when this (precision, n) has none.
-int pick_fusion(qcs_register* r, const qcs_gate* gates, uint32_t n, std::vector<qcs_gate>& out, uint32_t* width) {
+uint32_t priced_width(const qcs_register* r, const qcs_gate* gates, uint32_t n) {
     double t[6];
-    bool have = false;
     {
         std::lock_guard<std::mutex> lock(g_fuse_mu);
-        if (r->n <= kMaxN && g_fuse_cost[r->prec][r->n][0] > 0) {
-            for (int i = 0; i < 6; ++i) t[i] = g_fuse_cost[r->prec][r->n][i];
-            have = true;
-        }
+        if (r->n > kMaxN || !(g_fuse_cost[r->prec][r->n][0] > 0)) return 0;
+        for (int i = 0; i < 6; ++i) t[i] = g_fuse_cost[r->prec][r->n][i];
     }
-    if (!have)
-        if (const int e = autotune_fusion(r, 2, t)) return e;
     double best = 0;
     for (uint32_t i = 0; i < n; ++i) best += block_cost(gates[i], t);
-    out.assign(gates, gates + n);
-    *width = 0;
-    // the widths are fused on host threads of their own (the pass is host
-    // code and shares no state between calls), then priced in order
-    const uint32_t wmax = std::min<uint32_t>(5, r->n);
-    std::vector<std::vector<qcs_gate>> f(6);
-    int err[6] = {0, 0, 0, 0, 0, 0};
-    {
-        std::vector<std::thread> pool;
-        for (uint32_t w = 2; w <= wmax; ++w) pool.emplace_back([&, w] { err[w] = fuse(gates, n, w, f[w]); });
-        for (auto& th : pool) th.join();
-    }
-    for (uint32_t w = 2; w <= wmax; ++w) {
-        if (err[w]) return fuse(gates, n, w, f[w]);  // again on this thread, for its error message
-        double c = 0;
-        for (const qcs_gate& g : f[w]) c += block_cost(g, t);
+    uint32_t width = 0;
+    for (uint32_t w = 2; w <= std::min<uint32_t>(5, r->n); ++w) {
+        const double c = fuse_estimate(gates, n, w) * t[w];
         if (c < best) {
             best = c;
-            *width = w;
-            out.swap(f[w]);
+            width = w;
         }
     }
-    return QCS_OK;
+    return width;
 }
 
 }  // namespace qcs

@@ -369,23 +369,15 @@ int qcs_apply_circuit(qcs_register* r, const qcs_gate* gates, uint32_t n, uint32
     for (uint32_t i = 0; i < n; ++i)
         for (uint32_t j = 0; j < gates[i].k && j < 5; ++j)
             QCS_REQUIRE(gates[i].qubits[j] < r->n, "gate %u: qubit out of range", i);
-    // The list runs in passes of many gates (circuit.hip) at every width, which
-    // beat dense blocks of the width: 25 qubits complex128, 592 gates, width 5
-    // 20.0 ms in dense blocks, 8.5 ms in passes; 28 qubits, 252 gates 37.0
-    // against 25.5 ms at most; 27 qubits complex64, 867 gates 19.2 against 13.4 ms
-    // (host fusion, launches and waits included). The width stays what the
-    // caller gets told, and what is refused. Where dense blocks still win
-    // (fused_blocks), each is launched as soon as it is built.
-    if (fuse_width == QCS_FUSE_AUTO) {
-        std::vector<qcs_gate> fused;
-        if (const int e = pick_fusion(r, gates, n, fused, &fuse_width)) return e;
-        r->last_fuse_width = fuse_width;
-        if (fused_blocks(r, fuse_width)) return run_gates(r, fused.data(), uint32_t(fused.size()));
-    } else if (fused_blocks(r, fuse_width)) {
-        return fuse_stream(gates, n, fuse_width, [&](const qcs_gate& g) { return run_gates(r, &g, 1); });
-    } else if (const int e = fuse_check(gates, n, fuse_width)) {
-        return e;
-    }
+    // In passes of many gates (circuit.hip) whatever the width, which stays what
+    // the caller gets told, and what is refused; or in dense blocks where those
+    // win, each launched as soon as it is built.
+    const bool any = fuse_width == QCS_FUSE_AUTO;
+    if (!any || r->n > 1)
+        if (const int e = fuse_check(gates, n, any ? 5 : fuse_width)) return e;
+    const uint32_t width = fused_blocks(r, any ? 5 : fuse_width) ? (any ? 5 : fuse_width) : 0;
+    if (any) r->last_fuse_width = width ? width : priced_width(r, gates, n);
+    if (width) return fuse_stream(gates, n, width, [&](const qcs_gate& g) { return run_gates(r, &g, 1); });
     return run_gates(r, gates, n);
 }
 

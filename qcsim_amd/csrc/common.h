@@ -302,8 +302,9 @@ int run_gates(qcs_register* r, const qcs_gate* gates, uint32_t n);
 // Upper bound of the parameter bytes run_gates stages for one gate.
 size_t gates_param_bound(const qcs_register* r, const qcs_gate& g);
 
-// autotune.hip: the fused sequence of the cheapest fusion width
-int pick_fusion(qcs_register* r, const qcs_gate* gates, uint32_t n, std::vector<qcs_gate>& out, uint32_t* width);
+// autotune.hip: the fusion width whose blocks cost least under the cost table
+// of the register's precision and size (0: single gates do, or there is none).
+uint32_t priced_width(const qcs_register* r, const qcs_gate* gates, uint32_t n);
 
 // expect_kernels.hip
 // Makes r->xfer at least `bytes` long (at most kXferBytes).

@@ -123,17 +123,17 @@ int qcs_program_create(qcs_register* r, const qcs_gate* gates, uint32_t n, uint3
     auto* p = new qcs_program;
     p->r = r;
     if (fuse_width >= 2) {
-        std::vector<qcs_gate> fused;
-        uint32_t picked = fuse_width;
+        const bool any = fuse_width == QCS_FUSE_AUTO;
         const uint32_t m = uint32_t(seq.size());
-        const int e = fuse_width == QCS_FUSE_AUTO   ? pick_fusion(r, seq.data(), m, fused, &picked)
-                      : fused_blocks(r, fuse_width) ? fuse(seq.data(), m, fuse_width, fused)
-                                                    : fuse_check(seq.data(), m, fuse_width);
+        int e = !any || r->n > 1 ? fuse_check(seq.data(), m, any ? 5 : fuse_width) : QCS_OK;
+        const uint32_t width = !e && fused_blocks(r, any ? 5 : fuse_width) ? (any ? 5 : fuse_width) : 0;
+        std::vector<qcs_gate> fused;
+        if (width) e = fuse(seq.data(), m, width, fused);
         if (e) {
             delete p;
             return e;
         }
-        if (fused_blocks(r, picked)) seq.swap(fused);
+        if (width) seq.swap(fused);
     }
     p->gates.swap(seq);
     for (const auto& g : p->gates) p->param_bytes += gates_param_bound(r, g);

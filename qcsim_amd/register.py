@@ -271,8 +271,8 @@ class QubitRegister:
         return (QcsGate * n).from_buffer(a)
 
     def apply_circuit(self, gates, fuse_width=0):
-        """The gates in order; fuse_width 0 (none), 2..5 or "auto" (the width
-        with the lowest cost under the measured fusion cost table)."""
+        """The gates in order; fuse_width 0 (none), 2..5 or "auto" (left to the
+        library)."""
         arr = self._gate_array(gates)
         w = QCS_FUSE_AUTO if fuse_width == "auto" else int(fuse_width)
         check(lib().qcs_apply_circuit(self._h, arr, len(gates), w))
