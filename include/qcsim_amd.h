@@ -110,10 +110,13 @@ int qcs_apply_gate(qcs_register* r, uint32_t k, uint32_t traits,
 int qcs_apply_dense(qcs_register* r, uint32_t k, const uint32_t* qubits,
                     const double* mat);
 
-/* A batch of gates in order, run in passes of many gates over the state
- * whatever the width. fuse_width 0/1 takes the gates as they come (a refused
+/* A batch of gates in order, run in passes of many gates over the state.
+ * fuse_width 0/1 takes the gates as they come (a refused
  * gate ends the batch after those before it); with 2..5 a list that the
- * fusion pass (qcs_fuse) refuses at that width is refused whole, and
+ * fusion pass (qcs_fuse) refuses at that width is refused whole, and at 4
+ * and 5 a large register applies a list whose gates keep to neighbourhoods in
+ * that pass's dense blocks, where those take less time (complex128 from 25
+ * qubits on; complex64, in FP32 then, from 28 on).
  * QCS_FUSE_AUTO leaves the width to the library. No counterpart in the
  * reference, which applies gates one by one (QubitRegister.h:488-492). */
 #define QCS_FUSE_AUTO 0xFFFFFFFFu

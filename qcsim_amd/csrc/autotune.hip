@@ -125,7 +125,8 @@ extern "C" int qcs_get_tuned_variant(int precision, uint32_t n, uint32_t q) {
 // block (k = 2..5). A gate that changes a fraction f of the amplitudes is priced
 // at f * t[0] (2- and 3-qubit gates without control structure at t[k]). The
 // width that QCS_FUSE_AUTO reports where a list runs in tile passes is the one
-// with the lowest total; how a list runs does not depend on the table.
+// with the lowest total; how a list runs does not depend on the table
+// (blocks_width).
 
 namespace qcs {
 int kdense(qcs_register* r, uint32_t k, const uint32_t* qubits, const double* mat_host);

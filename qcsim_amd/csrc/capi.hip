@@ -375,7 +375,7 @@ int qcs_apply_circuit(qcs_register* r, const qcs_gate* gates, uint32_t n, uint32
     const bool any = fuse_width == QCS_FUSE_AUTO;
     if (!any || r->n > 1)
         if (const int e = fuse_check(gates, n, any ? 5 : fuse_width)) return e;
-    const uint32_t width = fused_blocks(r, any ? 5 : fuse_width) ? (any ? 5 : fuse_width) : 0;
+    const uint32_t width = fused_blocks(r, gates, n, any ? 2 : fuse_width, any ? 5 : fuse_width);
     if (any) r->last_fuse_width = width ? width : priced_width(r, gates, n);
     if (width) return fuse_stream(gates, n, width, [&](const qcs_gate& g) { return run_gates(r, &g, 1); });
     return run_gates(r, gates, n);

@@ -475,9 +475,12 @@ size_t gates_param_bound(const qcs_register* r, const qcs_gate& g) {
     return 2 * D * D * sizeof(double) + (6 * kHead + kTail) * 4 + 256;
 }
 
+// What a pass's stream may take: a staging slot, less its rounding.
+static size_t stream_bytes(const qcs_register* r) { return r->mat_bytes - 256; }
+
 template <typename T>
 static int run_tiles(qcs_register* r, const qcs_gate* gates, uint32_t n) {
-    TilePlanner plan(gates, n, r->n, r->amp_bytes(), r->mat_bytes - 256);
+    TilePlanner plan(gates, n, r->n, r->amp_bytes(), stream_bytes(r));
     struct Pass {
         TileGeo geo;
         size_t at;  // first word of its stream
@@ -513,6 +516,10 @@ static int run_tiles(qcs_register* r, const qcs_gate* gates, uint32_t n) {
             if (const int e = flush()) return e;
     }
     return flush();
+}
+
+uint32_t fused_blocks(const qcs_register* r, const qcs_gate* gates, uint32_t n, uint32_t lo, uint32_t hi) {
+    return blocks_width(gates, n, r->n, r->amp_bytes(), stream_bytes(r), lo, hi);
 }
 
 // The gates in order: in tile passes, or one launch each where a pass does

@@ -13,6 +13,8 @@
 
 namespace qcs {
 
+double fuse_estimate(const qcs_gate* gates, uint32_t n, uint32_t width);
+
 struct hcplx {
     double re, im;
 };
@@ -565,6 +567,114 @@ bool TilePlanner::next(TileGeo& geo, std::vector<uint32_t>& words, const qcs_gat
     words.clear();
     tile_emit(P.local, tile_rounds(P.local, S, top), S, P.n, words);
     return true;
+}
+
+// ---------------------------------------------------------------------------
+// Passes or dense blocks.
+//
+// Times are in ps per amplitude of a state that HBM bounds. Those of the steps
+// of a plan were fitted to 135 runs of 16 kinds of list on 25 to 30 qubits, which
+// they give to 10 % each; a pass is not below the time of its bytes. A dense
+// block's are its kernel's rate on 30 qubits, and ms for its matrix's way there.
+struct BlockTime {
+    double ps, ms;
+};
+
+static BlockTime block_time(uint32_t k, bool c64) {
+    if (k == 5) return c64 ? BlockTime{3.42, 0.14} : BlockTime{6.4, 0.14};
+    return c64 ? BlockTime{2.88, 0.045} : BlockTime{5.6, 0.04};
+}
+
+static double pass_time(const std::vector<uint32_t>& words, bool c64) {
+    double ps = 2.5;
+    for (size_t i = 0; (words[i] & 0xffff) != kOpEnd; i += words[i] >> 16) {
+        const uint32_t code = words[i] & 0xffff;
+        if (code == kOpRound) {
+            ps += 0.29;
+            continue;
+        }
+        if (code >= kOpZ && code < kOpGen2) {
+            ps += 0.16;
+            continue;
+        }
+        // of the amplitudes, or the tiles, those with every control set
+        const double part = popc(words[i + 2] & 255) / 8.0 / double(1 << popc(words[i + 3]));
+        ps += part * (code < kOpReal                       ? 0.26
+                      : code < kOpX                        ? 0.18
+                      : code < kOpDiagR                    ? 0.20
+                      : code < kOpSwap                     ? 0.16
+                      : code < kOpZ                        ? 0.20
+                      : code < kOpGen3                     ? 0.97
+                                                           : 1.5);
+    }
+    return std::max(ps, c64 ? 4.4 : 7.1);
+}
+
+// Mostly above the time a gate takes in a pass with its share of the rounds,
+// and without a plan.
+static double gate_time(const qcs_gate& g, bool c64) {
+    if (g.k > 3) return block_time(g.k, c64).ps;
+    const uint32_t t = (g.flags & QCS_GATE_DENSE) ? 0 : g.traits;
+    if (g.k == 1) return 0.3;
+    if (t & (QCS_TRAIT_SWAP | QCS_TRAIT_ISWAP | QCS_TRAIT_ISWAPDAG)) return 0.7;
+    const uint32_t targets = !(t & QCS_TRAIT_CONTROLLED) ? g.k : g.k == 3 && !(t & QCS_TRAIT_CTRL_Q1) ? 2 : 1;
+    return targets == 1 ? 0.6 : targets == 2 ? 1.5 : 2.7;
+}
+
+// Blocks multiply on the matrix cores, at nearly the rate of their bytes for
+// as many gates as meet on four or five qubits; a pass computes each gate by
+// itself, on any qubits, and a phase over many for the price of one. So lists
+// that keep to neighbourhoods are faster in blocks, and others in passes (ms at
+// width 5, blocks and passes; 28 qubits complex128: Heisenberg steps, 1377
+// gates, 29.4 and 54.9; layers of U(2) and CNOT, 504 gates, 72.3 and 46.7; Ising
+// steps, 654 gates, 47.2 and 23.0. Complex64: 17.2 and 55.6, 41.6 and 43.9, 26.8
+// and 23.9. 26 qubits complex128: 8.7 and 12.8, 21.9 and 10.8, 14.3 and 5.4).
+//
+// complex128, from 25 qubits on (below, the host's fusion takes longer than the
+// passes): blocks where they take less than 0.85 of the passes' time, and
+// where a quarter of the gates or more join qubits, as for others the fusion
+// itself takes longest. Both compute in FP64; of a normalised state of 13 qubits
+// after 612 gates the passes err by 1.1e-15, the blocks by 1.5e-15. complex64, where blocks are in FP32 and passes in FP64:
+// from 28 qubits on blocks, unless the passes take less than 0.9 of their time;
+// below always passes, which are 20 times as exact (27 qubits, the lists above:
+// 9.9 and 27.5, 22.9 and 20.5, 14.3 and 11.2 ms).
+uint32_t blocks_width(const qcs_gate* gates, uint32_t n, uint32_t nq, size_t amp_bytes, size_t stream_bytes, uint32_t lo,
+                      uint32_t hi) {
+    constexpr uint32_t kSample = 4096;  // of a long list, its beginning tells
+    const bool c64 = amp_bytes == 8;
+    if (hi < 4 || nq < (c64 ? 28u : 25u)) return 0;
+    n = std::min(n, kSample);
+    uint32_t joined = 0;
+    double quick = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        joined += gates[i].k > 1;
+        quick += gate_time(gates[i], c64);
+    }
+    if (!c64 && 4 * joined < n) return 0;
+    const double ms = double(1ull << nq) * 1e-9;  // a ps per amplitude
+    double blocks = 0;
+    uint32_t width = 0;
+    for (uint32_t w = std::max(lo, 4u); w <= hi; ++w) {
+        const BlockTime t = block_time(w, c64);
+        const double b = fuse_estimate(gates, n, w) * (t.ps * ms + t.ms);
+        if (!width || b < blocks) {
+            blocks = b;
+            width = w;
+        }
+    }
+    // plainly the one or the other, by the gates alone
+    quick *= ms;
+    if (c64 ? quick < 0.9 * blocks : blocks > 0.85 * quick) return 0;
+    if (blocks < 0.3 * quick) return width;
+    TilePlanner plan(gates, n, nq, amp_bytes, stream_bytes);
+    TileGeo geo;
+    std::vector<uint32_t> words;
+    const qcs_gate* single = nullptr;
+    double passes = 0;
+    while (plan.next(geo, words, &single))
+        passes += !single ? pass_time(words, c64) : single->k > 3 ? block_time(single->k, c64).ps : c64 ? 3.8 : 5.2;
+    passes *= ms;
+    return (c64 ? passes < 0.9 * blocks : blocks > 0.85 * passes) ? 0 : width;
 }
 
 }  // namespace qcs

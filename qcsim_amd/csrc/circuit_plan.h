@@ -75,4 +75,9 @@ class TilePlanner {
     Plan* p_;
 };
 
+// The width, of those from lo to hi (2..5), at whose dense blocks a list that
+// the fusion pass takes runs rather than in passes; 0 if passes.
+uint32_t blocks_width(const qcs_gate* gates, uint32_t n, uint32_t nq, size_t amp_bytes, size_t stream_bytes, uint32_t lo,
+                      uint32_t hi);
+
 }  // namespace qcs

@@ -286,16 +286,9 @@ int rising(qcs_register* r, uint32_t ne, const uint32_t* ei, const uint32_t* ej,
 // qft.hip
 int qft(qcs_register* r, uint32_t sq, uint32_t eq, int do_swap, int inverse);
 
-// Whether a circuit fused to `width` runs in dense blocks instead of tile
-// passes: complex64 from 28 qubits on, where four- and five-qubit blocks
-// multiply in FP32 on the matrix cores at nearly the rate of their bytes while
-// the passes compute in FP64 (layers of U(2) and CNOT, width 5: 28 qubits, 672
-// gates 50.5 ms in blocks and 59.4 in passes; 30 qubits, 540 gates 149 and
-// 191; but 26 qubits, 624 gates 20.9 and 14.4).
-inline bool fused_blocks(const qcs_register* r, uint32_t width) {
-    return r->prec != QCS_COMPLEX128 && r->n >= 28 && width >= 4 && width <= 5;
-}
-
+// circuit.hip: whether and at what width, of those from lo to hi, a list that
+// the fusion pass takes runs in dense blocks instead of tile passes (0: passes).
+uint32_t fused_blocks(const qcs_register* r, const qcs_gate* gates, uint32_t n, uint32_t lo, uint32_t hi);
 // circuit.hip: a gate list in passes of many gates; the first gate its entry
 // point refuses ends it with that error.
 int run_gates(qcs_register* r, const qcs_gate* gates, uint32_t n);

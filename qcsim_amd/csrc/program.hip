@@ -126,7 +126,7 @@ int qcs_program_create(qcs_register* r, const qcs_gate* gates, uint32_t n, uint3
         const bool any = fuse_width == QCS_FUSE_AUTO;
         const uint32_t m = uint32_t(seq.size());
         int e = !any || r->n > 1 ? fuse_check(seq.data(), m, any ? 5 : fuse_width) : QCS_OK;
-        const uint32_t width = !e && fused_blocks(r, any ? 5 : fuse_width) ? (any ? 5 : fuse_width) : 0;
+        const uint32_t width = e ? 0 : fused_blocks(r, seq.data(), m, any ? 2 : fuse_width, any ? 5 : fuse_width);
         std::vector<qcs_gate> fused;
         if (width) e = fuse(seq.data(), m, width, fused);
         if (e) {

@@ -8,6 +8,9 @@
 
 #include "../../qcsim_amd/csrc/circuit_plan.h"
 
+namespace qcs {
+int set_error(int code, const char*, ...) { return code; }  // fusion.cpp's
+}  // namespace qcs
 using namespace qcs;
 typedef std::complex<double> Amp;
 
@@ -89,6 +92,11 @@ extern "C" {
 
 void* plan_new(const qcs_gate* gates, uint32_t n, uint32_t nq, uint64_t amp_bytes, uint64_t stream_bytes) {
     return new TilePlanner(gates, n, nq, amp_bytes, stream_bytes);
+}
+
+uint32_t plan_width(const qcs_gate* gates, uint32_t n, uint32_t nq, uint64_t amp_bytes, uint64_t stream_bytes, uint32_t lo,
+                    uint32_t hi) {
+    return blocks_width(gates, n, nq, amp_bytes, stream_bytes, lo, hi);
 }
 
 void plan_free(void* p) { delete static_cast<TilePlanner*>(p); }

@@ -23,12 +23,15 @@ STREAM = 64 * 64 * 8 - 256  # a register's staging slot, less its rounding
 @pytest.fixture(scope="module")
 def host(tmp_path_factory):
     lib = str(tmp_path_factory.mktemp("plan") / "libcircuit_host.so")
-    src = [os.path.join(ROOT, p) for p in ("tests/cpp/circuit_host.cpp", "qcsim_amd/csrc/circuit_plan.cpp")]
+    src = [os.path.join(ROOT, p) for p in ("tests/cpp/circuit_host.cpp", "qcsim_amd/csrc/circuit_plan.cpp",
+                                          "qcsim_amd/csrc/fusion.cpp")]
     subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", "-I", os.path.join(ROOT, "include"),
                     *src, "-o", lib], check=True)
     L = C.CDLL(lib)
     L.plan_new.restype, L.plan_new.argtypes = C.c_void_p, [C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint64, C.c_uint64]
     L.plan_free.restype, L.plan_free.argtypes = None, [C.c_void_p]
+    L.plan_width.restype, L.plan_width.argtypes = C.c_uint32, [C.c_void_p, *[C.c_uint32] * 2, *[C.c_uint64] * 2,
+                                                               *[C.c_uint32] * 2]
     L.plan_step.restype = C.c_int64
     L.plan_step.argtypes = [C.c_void_p, C.c_void_p, C.c_uint32, C.c_void_p, C.POINTER(C.c_uint64)]
     return L
@@ -138,3 +141,49 @@ def test_planning_grows_with_the_list(host):
 
     assert best(long * len(seq), False) < 5 * long * best(len(seq), False)
     assert best(long * len(seq), True) < 5 * best(len(seq), True)
+
+
+def layers(n, rng):
+    seq = []
+    for _ in range(10):
+        seq += [(G.SingleQubitGate(G.haar_u2(rng)), [q]) for q in range(n)]
+        perm = [int(q) for q in rng.permutation(n)]
+        seq += [(G.CNOTGate(), [a, b]) for a, b in zip(perm[0::2], perm[1::2])]
+    return seq
+
+
+def ising_steps(n):
+    seq = []
+    for _ in range(5):
+        for q in range(n - 1):
+            seq += [(G.CNOTGate(), [q + 1, q]), (G.RzGate(0.2), [q + 1]), (G.CNOTGate(), [q + 1, q])]
+        seq += [(G.RxGate(0.3), [q]) for q in range(n)]
+    return seq
+
+
+def heisenberg_steps(n):
+    seq = []
+    for _ in range(3):
+        for q in [*range(0, n - 1, 2), *range(1, n - 1, 2)]:
+            for before, after in ((G.HadamardGate(), G.HadamardGate()), (G.RxGate(1.5), G.RxGate(-1.5)), (None, None)):
+                seq += [(before, [q]), (before, [q + 1])] if before else []
+                seq += [(G.CNOTGate(), [q + 1, q]), (G.RzGate(0.2), [q + 1]), (G.CNOTGate(), [q + 1, q])]
+                seq += [(after, [q]), (after, [q + 1])] if after else []
+    return seq
+
+
+# what the rule says where both ways were timed, and next to where it begins
+@pytest.mark.parametrize("amp_bytes,n,kind,width,blocks", [
+    (16, 24, "heisenberg", 5, False), (16, 26, "heisenberg", 5, True), (16, 27, "heisenberg", 4, True),
+    (16, 28, "heisenberg", 5, True), (16, 26, "layers", 4, False), (16, 28, "layers", 5, False),
+    (16, 28, "ising", 5, False), (16, 28, "heisenberg", 3, False), (8, 27, "heisenberg", 5, False),
+    (8, 28, "heisenberg", 5, True), (8, 28, "heisenberg", 4, True), (8, 28, "layers", 5, True), (8, 30, "layers", 4, True),
+    (8, 28, "ising", 4, False), (8, 30, "ising", 4, False), (8, 28, "ising", 3, False)])
+def test_blocks_or_passes(host, amp_bytes, n, kind, width, blocks):
+    seq = {"layers": lambda: layers(n, np.random.default_rng(n)), "ising": lambda: ising_steps(n),
+           "heisenberg": lambda: heisenberg_steps(n)}[kind]()
+    arr = QubitRegister._gate_array(seq)
+    assert host.plan_width(arr, len(seq), n, amp_bytes, STREAM, width, width) == (width if blocks else 0)
+    picked = host.plan_width(arr, len(seq), n, amp_bytes, STREAM, 2, 5)
+    assert picked in (4, 5) if blocks else width < 4 or picked == 0
+    assert host.plan_width(arr, 0, n, amp_bytes, STREAM, 2, 5) in (0, 4, 5)  # an empty list
