@@ -1,16 +1,54 @@
-"""Gate lists at a fusion width on the device: those that run in dense blocks
-against the same lists in tile passes, where registers are large enough for
+"""The blocks of the fusion pass on the device: every width's blocks one by one
+against the oracle on small registers, and gate lists that run in blocks
+against the same lists in tile passes where registers are large enough for
 it."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
+from oracle.oracle import OracleRegister
 from qcsim_amd import QubitRegister, _lib
+from refmath import random_state
 from test_circuit_plan import heisenberg_steps, ising_steps, layers
-from test_fusion import to_struct
+from test_fusion import fuse, random_circuit, to_struct
 
 pytestmark = pytest.mark.gpu
+
+
+def apply_block(reg, g):
+    m = np.frombuffer(bytes(g.mat), dtype=np.float64)[: 2 * 4**g.k].view(np.complex128).reshape(1 << g.k, 1 << g.k)
+    if (g.flags & _lib.QCS_GATE_DENSE) or g.k > 3:
+        reg.apply_dense([g.qubits[j] for j in range(g.k)], m)
+    else:
+        _lib.check(_lib.lib().qcs_apply_gate(reg._h, g.k, g.traits, *g.qubits[:3], m.tobytes()))
+
+
+@pytest.mark.parametrize("precision", ["c128", "c64"])
+@pytest.mark.parametrize("width", [2, 3, 4, 5])
+@pytest.mark.parametrize("n", [5, 7, 9, 13])
+def test_blocks_equal_oracle(n, width, precision):
+    """n = 5, 7: states below one tile of the matrix-core kernel. In complex64 a
+    row of a block errs by at most (2^k + 2) 2^-24 of its vector's norm."""
+    rng = np.random.default_rng(10 * n + width)
+    seq = random_circuit(rng, n, 80)
+    psi = random_state(rng, n)
+    ref = OracleRegister(n)
+    ref.set_state(psi)
+    for gate, qs in seq:
+        ref.apply_gate(gate, *qs)
+    out, count = fuse(to_struct(seq), width)
+    assert any(out[i].flags & _lib.QCS_GATE_DENSE for i in range(count))
+    reg = QubitRegister(n, precision=precision)
+    reg.setRegisterStorageFastNoNormalize(psi.copy())
+    for i in range(count):
+        apply_block(reg, out[i])
+    err = np.asarray(reg.getRegisterStorage()) - ref.state()
+    reg.close()
+    if precision == "c128":
+        assert np.max(np.abs(err)) < 1e-12
+    else:
+        assert np.linalg.norm(err) < count * (2**width + 2) * 2 * 2.0**-24
 
 
 @pytest.mark.parametrize("n,precision,kind,width,blocks", [
@@ -20,8 +58,7 @@ pytestmark = pytest.mark.gpu
 def test_list_in_blocks_equals_passes(n, precision, kind, width, blocks):
     """The whole state of a list at a fusion width against width 0, which is
     always tile passes, and how many launches it took. In complex64 the two
-    differ by what FP32 blocks of 2^5 rows may err, a row
-    34 2^-24 of its vector's norm."""
+    differ by what FP32 blocks of 2^5 rows may err, as above."""
     seq = {"layers": lambda: layers(n, np.random.default_rng(n)), "ising": lambda: ising_steps(n),
            "heisenberg": lambda: heisenberg_steps(n)}[kind]()
     a, b = QubitRegister(n, precision=precision), QubitRegister(n, precision=precision)
