@@ -20,12 +20,10 @@
 // mask too wide for a tile has one of its own (k_pauli). All sums are FP64
 // with a fixed grid and a fixed combination order.
 #include <algorithm>
-#include <map>
-#include <set>
-#include <unordered_map>
 #include <vector>
 
 #include "common.h"
+#include "pauli_plan.h"
 
 namespace qcs {
 
@@ -150,23 +148,7 @@ __global__ __launch_bounds__(kExThreads) void k_pauli(const cv<T>* __restrict__ 
 // costs each wave a trip to LDS. One block of 1024 threads a CU holds two
 // tiles in LDS (one barrier a tile) and prefetches the next into registers.
 // 27 terms on 27 qubits complex64: 0.51 ms in two passes, now 0.26 ms in one.
-constexpr int kPtMax = 12;       // tile qubits
 constexpr int kPtThreads = 1024;  // of a full tile
-constexpr int kPtSlots = 12;
-constexpr int kPtTerms = 64;     // terms of a pass
-constexpr int kPtBlocks = 256;
-
-struct PauliTile {  // words throughout: the scalar unit loads nothing smaller
-    uint32_t t, ns, nt;
-    uint32_t im;                   // slots of imaginary parts
-    uint32_t pos[kPtMax];          // tile qubits, ascending
-    uint64_t tile_bits, step;      // the tile qubits; the grid's size on the qubits outside
-    uint32_t x[kPtSlots];          // x mask within the tile
-    uint32_t zt[2 * kPtSlots];     // z bits on the tile index; without pairs: from bit 30 on those on the register
-                                   // qubits. With pairs one word a slot
-    uint32_t first[kPtSlots + 1];  // terms first[j]..first[j+1] are slot j's, from first[ns] on those of x = 0
-    uint32_t z[kPtTerms];          // z mask within the tile; without pairs: bit 15 for the slot's second sum
-};
 
 template <typename T, bool PAIRS>
 __global__ __launch_bounds__(kPtThreads) void k_pauli_tile(const cv<T>* __restrict__ psi, uint64_t amps, uint32_t ntiles,
@@ -481,77 +463,15 @@ static int pauli_wide(qcs_register* r, const std::vector<uint32_t>& terms, uint6
     return QCS_OK;
 }
 
-// The qubits of the next tile: the lowest ones, for whole memory lines, then
-// the x masks that need the fewest more, in order of first appearance.
-static uint64_t pauli_tile_qubits(const std::vector<uint64_t>& xs, uint64_t low, uint32_t n, uint32_t t) {
-    uint64_t S = low;
-    for (;;) {
-        uint64_t best = 0;
-        int need = 64;
-        for (const uint64_t x : xs) {
-            const int more = __builtin_popcountll(x & ~S);
-            if (more && more < need && more + __builtin_popcountll(S) <= int(t)) {
-                need = more;
-                best = x;
-            }
-        }
-        if (!best) break;
-        S |= best;
-    }
-    for (uint32_t q = 0; q < n && __builtin_popcountll(S) < int(t); ++q) S |= 1ull << q;
-    return S;
-}
-
-// bits of m at the set bits of S, packed
-static uint32_t pack_bits(uint64_t m, uint64_t S) {
-    uint32_t v = 0, i = 0;
-    for (; S; S &= S - 1, ++i) v |= uint32_t(m >> __builtin_ctzll(S) & 1) << i;
-    return v;
-}
-
 template <typename T>
 static int pauli_t(qcs_register* r, uint32_t nterms, const uint64_t* xmask, const uint64_t* zmask, double* out) {
     const uint64_t full = r->A - 1;
     for (uint32_t t = 0; t < nterms; ++t)
         if ((xmask[t] | zmask[t]) & ~full) return set_error(QCS_EINVAL, "term %u: mask beyond the register", t);
-    const uint32_t n = r->n, t = std::max<uint32_t>(2, std::min<uint32_t>(n, kPtMax));
-    const uint64_t low = (1ull << std::min<uint32_t>(n, sizeof(T) == 8 ? 3 : 4)) - 1;
-    const uint32_t ntiles = n > t ? 1u << (n - t) : 1, nb = std::min<uint32_t>(ntiles, kPtBlocks);
-    // In units of one read of the state, a slot of a tile pass costs a twelfth
-    // of the pass and 0.05 for its trips to LDS, and a pass of k_pauli 1.25 for
-    // 16 terms of one x mask. So an x mask whose terms share few slots (z masks
-    // all over the register) is faster apart, where reading counts (30 qubits,
-    // 32 random z masks with one x mask: 10.5 ms in tile passes, 5.9 apart).
-    constexpr uint32_t kApart = 10;  // slots that cost more than a pass of k_pauli
-    std::unordered_map<uint64_t, uint32_t> sharing;
-    const bool big = r->A * r->amp_bytes() > size_t(256) << 20;
-    for (uint32_t i = 0; big && i < nterms; ++i) ++sharing[xmask[i]];
-    std::map<uint64_t, bool> decided;
-    auto apart = [&](uint64_t x) {
-        const uint32_t terms = big ? sharing[x] : 0;
-        if (terms < kApart) return false;
-        const auto it = decided.find(x);
-        if (it != decided.end()) return it->second;
-        const uint64_t S = pauli_tile_qubits({x}, low, n, t);
-        std::set<std::pair<uint64_t, int>> slots;
-        for (uint32_t i = 0; i < nterms; ++i)
-            if (xmask[i] == x) slots.insert({zmask[i] & full & ~S, __builtin_popcountll(x & zmask[i]) & 1});
-        return decided[x] = (1.0 / kPtSlots + 0.05) * double(slots.size()) > 1.25 * ((terms + 15) / 16);
-    };
-    std::vector<uint32_t> rest;
-    std::vector<uint64_t> wide, xs;
-    std::map<uint64_t, std::vector<uint32_t>> wides;
-    for (uint32_t i = 0; i < nterms; ++i) {
-        const uint64_t x = xmask[i];
-        if (__builtin_popcountll(x | low) <= int(t) && !(x && apart(x))) {
-            rest.push_back(i);
-        } else {
-            if (!wides.count(x)) wide.push_back(x);
-            wides[x].push_back(i);
-        }
-    }
+    PauliPlanner plan(r->n, r->amp_bytes(), nterms, xmask, zmask);
+    const uint32_t nb = plan.blocks;
     // the terms whose sums are on their way
-    std::vector<uint32_t> batch;
+    std::vector<uint32_t> batch, terms;
     double* res = r->red + kRedResult;
     auto flush = [&]() -> int {
         if (batch.empty()) return QCS_OK;
@@ -563,101 +483,25 @@ static int pauli_t(qcs_register* r, uint32_t nterms, const uint64_t* xmask, cons
         batch.clear();
         return QCS_OK;
     };
-    while (!rest.empty()) {
-        xs.clear();
-        for (const uint32_t i : rest)
-            if (xmask[i] && std::find(xs.begin(), xs.end(), xmask[i]) == xs.end()) xs.push_back(xmask[i]);
-        const uint64_t S = n < t ? 3 : pauli_tile_qubits(xs, low, n, t);
-        PauliTile P{};
-        P.t = t;
-        P.tile_bits = S;
-        P.step = nb;
-        for (uint64_t m = S, i = 0; m; m &= m - 1) P.pos[i++] = uint32_t(__builtin_ctzll(m));
-        for (uint32_t i = 0; i < t; ++i) {
-            const uint64_t below = (1ull << P.pos[i]) - 1;
-            P.step = ((P.step & ~below) << 1) | (P.step & below);
-        }
-        struct Slot {
-            uint64_t x;
-            bool im;
-            uint32_t zt, halves;
-            std::vector<uint32_t> terms;
-            std::vector<uint32_t> z;
-        };
-        std::vector<Slot> slots;
-        std::vector<uint32_t> inner, left;
-        const uint32_t top = t - 2;
-        uint32_t taken = 0;
-        const uint32_t most = std::min<uint32_t>(kPtTerms, kPauliResults - uint32_t(batch.size()));
-        for (const uint32_t i : rest) {
-            const uint64_t x = xmask[i], z = zmask[i];
-            const uint32_t zt = pack_bits(z, full & ~S), zl = pack_bits(z, S);
-            bool ok = taken < most && !(x & ~S);
-            if (ok && x) {
-                const bool im = __builtin_popcountll(x & z) & 1;
-                size_t j = 0;
-                while (j < slots.size() && !(slots[j].x == x && slots[j].im == im && slots[j].zt == zt)) ++j;
-                ok = j < slots.size() || j < kPtSlots;
-                if (ok) {
-                    if (j == slots.size()) {
-                        slots.push_back(Slot{x, im, zt, 2, {}, {}});
-                        P.zt[j] = zt;
-                    }
-                    slots[j].terms.push_back(i);
-                    slots[j].z.push_back(zl);
-                }
-            } else if (ok && !zt) {
-                inner.push_back(i);
-            } else if (ok) {
-                // with a later x mask's tile around it it costs nothing
-                size_t j = slots.size();
-                const bool half = j && slots[j - 1].halves == 1;
-                ok = xs.empty() && (half || j < kPtSlots);
-                if (ok) {
-                    if (!half) slots.push_back(Slot{0, false, 0, 0, {}, {}});
-                    j = slots.size() - 1;
-                    const uint32_t h = slots[j].halves++;
-                    P.zt[2 * j + h] = zt | (zl >> top) << 30;
-                    slots[j].terms.push_back(i);
-                    slots[j].z.push_back(zl | h << 15);
-                }
-            }
-            if (ok)
-                ++taken;
-            else
-                left.push_back(i);
-        }
-        if (!taken) {  // no result slot free
+    PauliTile P;
+    bool pairs = false;
+    while (plan.next(P, pairs, terms)) {
+        if (batch.size() + terms.size() > size_t(kPauliResults))
             if (const int e = flush()) return e;
-            continue;
-        }
-        bool pairs = false;
-        P.ns = uint32_t(slots.size());
-        for (size_t j = 0; j < slots.size(); ++j) {
-            P.im |= uint32_t(slots[j].im) << j;
-            P.x[j] = pack_bits(slots[j].x, S);
-            pairs = pairs || slots[j].x;
-            P.first[j] = P.nt;
-            for (size_t k = 0; k < slots[j].terms.size(); ++k) P.z[P.nt++] = slots[j].z[k];
-        }
-        P.first[P.ns] = P.nt;
-        for (const uint32_t i : inner) P.z[P.nt++] = pack_bits(zmask[i], S);
-        const unsigned threads = std::max(64u, 1u << top);
+        const unsigned threads = std::max(64u, 1u << (P.t - 2));
         double* partial = r->red + batch.size() * nb;
         if (pairs)
             hipLaunchKernelGGL((k_pauli_tile<T, true>), dim3(nb), dim3(threads), 0, r->stream,
-                               static_cast<const cv<T>*>(r->psi), r->A, ntiles, P, partial);
+                               static_cast<const cv<T>*>(r->psi), r->A, plan.ntiles, P, partial);
         else
             hipLaunchKernelGGL((k_pauli_tile<T, false>), dim3(nb), dim3(threads), 0, r->stream,
-                               static_cast<const cv<T>*>(r->psi), r->A, ntiles, P, partial);
+                               static_cast<const cv<T>*>(r->psi), r->A, plan.ntiles, P, partial);
         if (const int e = check_launch(r, "k_pauli_tile")) return e;
-        for (const Slot& sl : slots) batch.insert(batch.end(), sl.terms.begin(), sl.terms.end());
-        batch.insert(batch.end(), inner.begin(), inner.end());
-        rest.swap(left);
+        batch.insert(batch.end(), terms.begin(), terms.end());
     }
     if (const int e = flush()) return e;
-    for (const uint64_t x : wide)
-        if (const int e = pauli_wide<T>(r, wides[x], x, zmask, out)) return e;
+    for (const PauliPlanner::Group& g : plan.wide)
+        if (const int e = pauli_wide<T>(r, g.terms, g.x, zmask, out)) return e;
     return QCS_OK;
 }
 
