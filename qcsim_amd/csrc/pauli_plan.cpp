@@ -108,9 +108,12 @@ void PauliPlanner::choose() {
     for (size_t k = 0; k < live_.size() && k < kLook; ++k) xs.push_back(groups_[live_[k]].x);
     S_ = n_ < t ? 3 : pauli_tile_qubits(xs, low_, n_, t);
     if (live_.empty()) {
+        // Passes of even size: a sum takes its time, of which the reads hide a part
         for (const uint32_t i : diag_) (z_[i] & full_ & ~S_ ? outer_ : inner_).push_back(i);
         diag_.clear();
-        sums_ = 2 * kPtSlots;
+        const size_t k = outer_.size(), all = k + inner_.size();
+        const size_t passes = std::max((k + 2 * kPtSlots - 1) / (2 * kPtSlots), (all + kPtTerms - 1) / kPtTerms);
+        sums_ = passes ? (k + passes - 1) / passes : 0;
         return;
     }
     std::unordered_map<uint64_t, size_t> slot;

@@ -122,10 +122,13 @@ def test_every_term_once(host, n):
 
 def test_passes_are_few(host):
     """A Heisenberg chain's pairs in three tiles, its fields and bonds with
-    them; and of terms on few qubits nearly as many in a pass as it holds."""
+    them; and terms that differ in z alone in as many passes as they need."""
     x, z = chain(26)
     assert len(plan(host, 26, x, z)[0]) == 3
     rng = np.random.default_rng(1)
+    z = [int(v) | 1 << 25 for v in rng.integers(0, 1 << 26, 32)]
+    passes, _ = plan(host, 26, [0] * 32, z)
+    assert [p[0].nt for p in passes] == [16, 16]  # 24 and 8 sums take longer
     x, z = random_terms(rng, 12, 100, 1280)
     assert len(plan(host, 12, x, z)[0]) <= 25  # 20 hold as many terms
 
