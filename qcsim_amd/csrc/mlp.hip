@@ -139,15 +139,12 @@ typedef float fx4 __attribute__((ext_vector_type(4)));
 template <int J> struct bvec;
 template <> struct bvec<1> { using type = uint16_t; };
 template <> struct bvec<2> { using type = uint32_t; };
-template <> struct bvec<4> { using type = uint2; };
 __device__ __forceinline__ float bv_get(uint16_t v, int) { return bf16_to(v); }
 __device__ __forceinline__ float bv_get(uint32_t v, int j) {
     return __builtin_bit_cast(float, j ? (v & 0xffff0000u) : (v << 16));
 }
-__device__ __forceinline__ float bv_get(uint2 v, int j) { return bv_get(j < 2 ? v.x : v.y, j & 1); }
 __device__ __forceinline__ void bv_set(uint16_t& v, int, bf16 b) { v = b; }
 __device__ __forceinline__ void bv_set(uint32_t& v, int j, bf16 b) { v |= uint32_t(b) << (16 * j); }
-__device__ __forceinline__ void bv_set(uint2& v, int j, bf16 b) { bv_set(j < 2 ? v.x : v.y, j & 1, b); }
 
 constexpr int kMlpMaxLayers = 9;   // weight layers: at most 8 hidden ones and the output
 constexpr int kMlpPad = 256;       // rows of a packed weight matrix are a multiple of this

@@ -3,7 +3,8 @@
 // The reference builds QFT/IQFT from Hadamards, controlled phase shifts and a
 // SWAP network (QuantumFourierTransform.h:35-87, QubitsSwapper.h:23-33): at
 // n = 30 that is 480 full passes over the state. Here the same operator is
-// applied in about (n - 12)/9 + 2 passes (4 at n = 22 to 30):
+// applied in about (n - 12)/9 + 2 passes in complex128 (4 at n = 22 to 30) and
+// (n - 12)/8 + 2 in complex64 (4 at n = 21 to 28, 5 at 29 to 34):
 //
 //   The controlled phase shifts between target `cur` and every control below
 //   it (phase pi/2, pi/4, ... for distance 1, 2, ...) multiply to one
@@ -527,7 +528,7 @@ __device__ void lds_round_g(cv<T>* s, uint64_t base, const QftTile& t, uint32_t 
 // of at most kMaxBlocks blocks from tile boff).
 //
 // The lowest targets come in contiguous chunks of 2^12 amplitudes, the others
-// five to nine a tile (complex64: to eight) with the lowest qubits, whole
+// four to nine a tile (complex64: to eight) with the lowest qubits, whole
 // memory lines. Two such passes took the place of three in registers at 25 to
 // 29 qubits: a transform of 29 qubits complex128 16.9 ms, now 13.8 ms, of 20
 // qubits (one for two) 49 us, now 35 us. A pass is bound by HBM: 3.3 ms for

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(1024) void k_scan_chunks(double* __restrict__ chunk
 // leaves the chunk's last value short of it, the last element.
 template <typename T>
 __device__ __forceinline__ uint64_t chunk_find(const double* nrm, uint64_t cbase, ChunkGeom g, double before, double pre,
-                                               double prob, int strict, unsigned long long* found) {
+                                               double prob, bool strict, unsigned long long* found) {
     const double acc = before + pre;
     const uint64_t beg = uint64_t(threadIdx.x) * g.per;
     double run = 0;
@@ -293,29 +293,26 @@ __device__ __forceinline__ uint64_t chunk_find(const double* nrm, uint64_t cbase
     return f == ~0ull ? cbase + g.clen - 1 : uint64_t(f);
 }
 
-// One block per shot. out[s] = first index i with prob <= cdf(i) (strict:
-// prob < cdf(i)), or `dflt` when the total stays below prob; the probabilities
-// are probs[s] (one_minus: 1 - probs[s]), or without probs prob1. With tout
-// the last block looks for prob1 strictly and writes there. Without chunk the
+// One block per shot. out[s] = first index i with prob <= cdf(i), or `dflt`
+// when the total stays below prob; prob is 1 - probs[s], or without probs
+// prob1. With tout the last block looks for prob1 < cdf(i) and writes there. Without chunk the
 // state is one chunk, whose total the block adds up itself.
 template <typename T>
 __global__ __launch_bounds__(kScanThreads) void k_search(const cv<T>* __restrict__ psi, ChunkGeom g,
                                                          const double* __restrict__ chunk, uint64_t nchunks,
-                                                         const double* __restrict__ probs, double prob1, int one_minus,
-                                                         int strict, uint64_t dflt, uint64_t* __restrict__ out,
-                                                         uint64_t* __restrict__ tout) {
+                                                         const double* __restrict__ probs, double prob1, uint64_t dflt,
+                                                         uint64_t* __restrict__ out, uint64_t* __restrict__ tout) {
     __shared__ double lds[4];
     __shared__ double nrm[kNrmLds];
     __shared__ uint64_t sc;
     __shared__ unsigned long long found;
     double prob = prob1;
     uint64_t* o = out + blockIdx.x;
-    if (tout && blockIdx.x == gridDim.x - 1) {
-        strict = 1;
+    const bool strict = tout && blockIdx.x == gridDim.x - 1;
+    if (strict)
         o = tout;
-    } else if (probs) {
-        prob = one_minus ? 1.0 - probs[blockIdx.x] : probs[blockIdx.x];
-    }
+    else if (probs)
+        prob = 1.0 - probs[blockIdx.x];
     auto reaches = [&](double v) { return strict ? v > prob : v >= prob; };
     if (threadIdx.x == 0) {
         // first c with chunk[c] >= prob (strict: > prob)
@@ -381,7 +378,7 @@ __global__ __launch_bounds__(kScanThreads) void k_measure_one(cv<T>* __restrict_
     if (threadIdx.x == 0) found = ~0ull;
     double total;
     const double pre = chunk_thread_prefix<T>(psi, 0, g, lds, nrm, &total);
-    const uint64_t f = total >= prob ? chunk_find<T>(nrm, 0, g, 0.0, pre, prob, 0, &found) : dflt;
+    const uint64_t f = total >= prob ? chunk_find<T>(nrm, 0, g, 0.0, pre, prob, false, &found) : dflt;
     const uint64_t mask = ((1ull << len) - 1) << first, val = f & mask;
     double acc = 0;
     for (uint64_t o = threadIdx.x; o < g.clen >> len; o += kScanThreads) acc += nrm[nrm_slot(insert_run(o, first, len) | val)];
@@ -559,8 +556,8 @@ static int search_launch(qcs_register* r, const ChunkGeom& g, uint64_t cnt, cons
                          uint64_t dflt, uint64_t* out, uint64_t* tout) {
     const uint64_t nchunks = r->A / g.clen;
     hipLaunchKernelGGL((k_search<T>), dim3(unsigned(cnt + (tout ? 1 : 0))), dim3(kScanThreads), 0, r->stream,
-                       static_cast<const cv<T>*>(r->psi), g, nchunks > 1 ? r->chunk : nullptr, nchunks, probs, prob1, 1, 0,
-                       dflt, out, tout);
+                       static_cast<const cv<T>*>(r->psi), g, nchunks > 1 ? r->chunk : nullptr, nchunks, probs, prob1, dflt,
+                       out, tout);
     return check_launch(r, "k_search");
 }
 
