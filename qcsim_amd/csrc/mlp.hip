@@ -112,12 +112,12 @@ __global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const TA* __r
 }
 
 // Output layer gradient for MSE: dY = 2 (y - t) / B; per-sample loss terms.
-__global__ void k_mse(int Bn, const float* __restrict__ y, const float* __restrict__ t, float4* __restrict__ dy,
-                      float* __restrict__ lossv) {
+__global__ void k_mse(int Bn, int batch, const float* __restrict__ y, const float* __restrict__ t,
+                      float4* __restrict__ dy, float* __restrict__ lossv) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= Bn) return;
     const float d = y[i] - t[i];
-    dy[i] = float4{2.f * d / float(Bn), 0.f, 0.f, 0.f};
+    dy[i] = float4{2.f * d / float(batch), 0.f, 0.f, 0.f};
     lossv[i] = d * d;
 }
 
@@ -152,6 +152,7 @@ constexpr int kMlpWide = 256;      // k_mlp_rows: widest layer
 
 struct MlpRows {
     int B, in, L, H;
+    int batch;                          // rows of the batch these are of: what its mean is over
     int ldx;                            // LDS rows and stride of the BF16 inputs (multiple of 32)
     int groups;                         // LDS size: groups of 16 columns per row tile
     const float* X;                     // inputs, rows of `in`
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(64 * NW) void k_mlp_rows(MlpRows a) {
                     a.y[row] = y;
                     if (TRAIN) {
                         const float d = y - target[r];
-                        dy = 2.f * d / float(a.B);
+                        dy = 2.f * d / float(a.batch);
                         a.dy[row] = float4{dy, 0.f, 0.f, 0.f};
                         a.lossv[row] = d * d;
                     }
@@ -421,10 +422,14 @@ struct DwLayer {
     uint32_t block0, nblk;    // first block, column blocks
 };
 
+constexpr int kDwRows = 192;  // rows of a slab
+
 struct DwArgs {
     int B, nl;
     uint32_t blocks;          // blocks of the layers; one more sums the loss
     int adam;                 // update the weights, else store the gradients
+    int more;                 // go on from the stored gradients: those of the batch's rows before these
+    int lossn;                // loss terms to add up
     float *g, *w, *m, *v;
     float lr, b1, b2, eps, c1, c2;
     const float* lossv;
@@ -446,15 +451,15 @@ struct DwArgs {
 // them 36 us; with the multiplying waves bringing the slabs themselves between
 // two barriers each 46 us; with branches around the loads 75 us.
 __global__ __launch_bounds__(512) void k_mlp_dw(DwArgs a) {
-    constexpr int KS = 192, NG = KS / 32, L = 32, NB = 4;  // rows of a slab, in groups of 32; columns; slabs in LDS
+    constexpr int KS = kDwRows, NG = KS / 32, L = 32, NB = 4;  // rows of a slab, in groups of 32; columns; slabs in LDS
     __shared__ __attribute__((aligned(16))) float Zs[NB][KS * L];
     __shared__ __attribute__((aligned(16))) bf16 As[NB][KS * L];
     const int tid = threadIdx.x & 255;
     const bool stager = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // the same in a whole wave
-    if (blockIdx.x == a.blocks) {
+    if (blockIdx.x == a.blocks) {  // not launched without loss terms
         float s = 0.f;
         if (!stager) {
-            for (int i = tid; i < a.B; i += 256) s += a.lossv[i];
+            for (int i = tid; i < a.lossn; i += 256) s += a.lossv[i];
             Zs[0][tid] = s;
         }
         __syncthreads();
@@ -542,6 +547,7 @@ __global__ __launch_bounds__(512) void k_mlp_dw(DwArgs a) {
         const int m = m0 + wm + 4 * kk + r;
         mine[r] = active && n < N && m <= M;
         at[r] = !mine[r] ? 0 : m < M ? y.woff + size_t(m) * N + n : y.boff + size_t(n);
+        if (a.more) acc[r] = a.g[at[r]];
         if (a.adam) {
             aw[r] = a.w[at[r]];
             am[r] = a.m[at[r]];
@@ -653,8 +659,10 @@ struct qcs_mlp {
     std::vector<size_t> poff, toff;
     int ldw = 0, ldx = 0;              // strides of hidden-wide and input rows
     bool rows_kernel = false;          // k_mlp_rows holds the network
-    // activations for the current batch
-    int cap = 0;
+    // activations and gradients of the rows in work: a batch's, or of a large
+    // batch as many as slice says, one slice after the other
+    int slice = 0;
+    int cap = 0, rows_cap = 0;  // rows of outputs and loss terms; of the others
     bf16* x0 = nullptr;
     std::vector<bf16*> act;   // outputs of hidden layers (bf16)
     std::vector<float*> dz;   // gradients before their ReLU
@@ -689,10 +697,12 @@ template <typename T> static bool grow(T*& p, size_t& cap, size_t n) {
     return true;
 }
 
-// Buffers for batches of B rows; `train`: those of the backward pass too.
-static int mlp_reserve(qcs_mlp* n, int B, bool train) {
-    if (B <= n->cap && (n->train_bufs || !train)) return QCS_OK;
-    const size_t rows = size_t(std::max(B, n->cap));
+// Buffers for batches of B rows, R of them in work at a time; `train`: those of
+// the backward pass too.
+static int mlp_reserve(qcs_mlp* n, int B, int R, bool train) {
+    if (B < 0) return set_error(QCS_ENOMEM, "mlp activations");  // a batch past 2^31
+    if (B <= n->cap && R <= n->rows_cap && (n->train_bufs || !train)) return QCS_OK;
+    const size_t all = size_t(std::max(B, n->cap)), rows = size_t(std::max(R, n->rows_cap));
     if (hipStreamSynchronize(n->stream) != hipSuccess) return set_error(QCS_EDEVICE, "sync failed");
     auto fr = [](auto*& p) {
         if (p) (void)hipFree(p);
@@ -705,24 +715,25 @@ static int mlp_reserve(qcs_mlp* n, int B, bool train) {
     fr(n->dy);
     fr(n->yt);
     fr(n->lossv);
-    n->cap = 0;
+    n->cap = n->rows_cap = 0;
     train = train || n->train_bufs;
     n->train_bufs = false;
     auto get = [](auto*& p, size_t k) { return hipMalloc(reinterpret_cast<void**>(&p), sizeof(*p) * k) == hipSuccess; };
-    bool ok = get(n->out, rows);
+    bool ok = get(n->out, all);
     if (train || !n->rows_kernel) {
         ok = ok && get(n->x0, rows * n->ldx);
         for (auto*& a : n->act) ok = ok && get(a, rows * n->ldw);
     }
     if (train) {
         for (auto*& z : n->dz) ok = ok && get(z, rows * n->ldw);
-        ok = ok && get(n->dy, rows) && get(n->yt, rows) && get(n->lossv, rows);
+        ok = ok && get(n->dy, rows) && get(n->yt, rows) && get(n->lossv, all);
     }
     if (!ok) {
         (void)hipGetLastError();
         return set_error(QCS_ENOMEM, "mlp activations");
     }
-    n->cap = int(rows);
+    n->cap = int(all);
+    n->rows_cap = int(rows);
     n->train_bufs = train;
     return QCS_OK;
 }
@@ -746,11 +757,15 @@ template <int J, int NW> static void launch_rows_j(const MlpRows& a, bool train,
 }
 
 // B rows of X (by idx, or in order) through the network into out; with
-// `train` (targets T, indexed like X) also through the loss and back.
-static int mlp_rows(qcs_mlp* n, int B, const float* X, const uint32_t* idx, const float* T, bool train, float* out) {
+// `batch` (targets T, indexed like X) also through the loss, of a batch of that
+// many rows, into lossv, and back.
+static int mlp_rows(qcs_mlp* n, int B, const float* X, const uint32_t* idx, const float* T, int batch, float* out,
+                    float* lossv) {
+    const bool train = batch > 0;
     if (n->rows_kernel) {
         MlpRows a{};
         a.B = B;
+        a.batch = batch;
         a.in = n->in;
         a.L = n->L;
         a.H = n->H;
@@ -771,7 +786,7 @@ static int mlp_rows(qcs_mlp* n, int B, const float* X, const uint32_t* idx, cons
         }
         a.y = out;
         a.dy = n->dy;
-        a.lossv = n->lossv;
+        a.lossv = lossv;
         if (n->ldw == 64)
             launch_rows_j<1, 4>(a, train, n->stream);
         else if (n->ldw == 128)
@@ -794,7 +809,7 @@ static int mlp_rows(qcs_mlp* n, int B, const float* X, const uint32_t* idx, cons
         hipLaunchKernelGGL((k_gemm<bf16, bf16, false, EPI_LINEAR_F32>), ggrid(B, 1), dim3(256), 0, n->stream, B, 1, din,
                            x, ld, n->wpack + n->poff[n->L], 1, out, nullptr, 1, n->w + n->boff[n->L], nullptr, 0);
         if (train) {
-            hipLaunchKernelGGL(k_mse, dim3((B + 255) / 256), dim3(256), 0, n->stream, B, out, n->yt, n->dy, n->lossv);
+            hipLaunchKernelGGL(k_mse, dim3((B + 255) / 256), dim3(256), 0, n->stream, B, batch, out, n->yt, n->dy, lossv);
             // dz_{l} = dz_{l+1} W^T, masked by ReLU' (activation > 0)
             for (int l = n->L - 1; l >= 0; --l) {
                 const bool top = l == n->L - 1;
@@ -809,13 +824,16 @@ static int mlp_rows(qcs_mlp* n, int B, const float* X, const uint32_t* idx, cons
     return e == hipSuccess ? QCS_OK : set_error(QCS_EDEVICE, "mlp rows: %s", hipGetErrorString(e));
 }
 
-// Gradients of the batch whose rows mlp_rows has just taken back, into n->g
-// or (adam) straight into the weights; the sum of the loss terms into *loss.
-static int mlp_dw(qcs_mlp* n, int B, bool adam, float lr, float* loss) {
+// Gradients of the rows that mlp_rows has just taken back, added to n->g if
+// they are not the batch's first (`more`), into n->g or (adam) straight into the
+// weights; with `loss` the sum of the batch's loss terms goes there.
+static int mlp_dw(qcs_mlp* n, int B, bool more, int batch, bool adam, float lr, float* loss) {
     DwArgs a{};
     a.B = B;
     a.nl = n->L + 1;
     a.adam = adam;
+    a.more = more;
+    a.lossn = batch;
     a.g = n->g;
     a.w = n->w;
     a.m = n->m;
@@ -850,9 +868,25 @@ static int mlp_dw(qcs_mlp* n, int B, bool adam, float lr, float* loss) {
         y.block0 = a.blocks;
         a.blocks += y.nblk * uint32_t((y.M + 1 + 31) / 32);
     }
-    hipLaunchKernelGGL(k_mlp_dw, dim3(a.blocks + 1), dim3(512), 0, n->stream, a);
+    hipLaunchKernelGGL(k_mlp_dw, dim3(a.blocks + (loss ? 1 : 0)), dim3(512), 0, n->stream, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? QCS_OK : set_error(QCS_EDEVICE, "mlp gradients: %s", hipGetErrorString(e));
+}
+
+// A batch of B rows through the network and back, in slices; its gradients and
+// loss as mlp_dw leaves them. The sums over the batch go on from slice to slice in
+// the order of its rows, so they do not depend on where it is cut.
+static int mlp_batch(qcs_mlp* n, int B, const float* X, const uint32_t* idx, const float* T, bool adam, float lr,
+                     float* loss) {
+    for (int b0 = 0; b0 < B; b0 += n->slice) {
+        const int P = std::min(n->slice, B - b0);
+        const bool last = b0 + P == B;
+        int e = mlp_rows(n, P, idx ? X : X + size_t(b0) * n->in, idx ? idx + b0 : nullptr, idx ? T : T + b0, B, n->out + b0,
+                         n->lossv + b0);
+        if (!e) e = mlp_dw(n, P, b0 > 0, B, adam && last, lr, last ? loss : nullptr);
+        if (e) return e;
+    }
+    return QCS_OK;
 }
 
 // The packed BF16 copies from the FP32 weights.
@@ -913,6 +947,8 @@ int qcs_mlp_create(uint32_t in_dim, uint32_t hidden, uint32_t layers, uint64_t s
     n->rows_kernel = n->in <= kMlpWide && n->H <= kMlpWide;
     n->ldx = (n->in + 31) / 32 * 32;
     n->ldw = !n->rows_kernel ? (n->H + 31) / 32 * 32 : n->H <= 64 ? 64 : n->H <= 128 ? 128 : 256;
+    // of activations and gradients about 1 GiB at a time, in whole slabs of k_mlp_dw
+    n->slice = std::max(int((size_t(1) << 30) / (size_t(n->L) * n->ldw * 6 + size_t(n->ldx) * 2)) / kDwRows, 1) * kDwRows;
     auto padded = [](int k) { return size_t((k + kMlpPad - 1) / kMlpPad * kMlpPad); };
     size_t packed = 0;
     for (int l = 0; l <= n->L; ++l) {
@@ -990,7 +1026,7 @@ int qcs_mlp_forward(qcs_mlp* n, const float* x, uint32_t batch, float* y) {
     if (!n || !x || !y || batch == 0) return set_error(QCS_EINVAL, "bad argument");
     for (uint32_t b0 = 0; b0 < batch; b0 += kMlpSlice) {
         const uint32_t B = std::min(kMlpSlice, batch - b0);
-        if (const int e = mlp_reserve(n, int(B), false)) return e;
+        if (const int e = mlp_reserve(n, int(B), n->rows_kernel ? 0 : int(B), false)) return e;
         if (!grow(n->xin, n->xin_cap, size_t(B) * n->in)) return set_error(QCS_ENOMEM, "mlp inputs");
         // wide networks keep one batch's activations: one piece
         const uint32_t fit = uint32_t(kMlpPiece / (sizeof(float) * n->in)) / 512 * 512;
@@ -1008,7 +1044,7 @@ int qcs_mlp_forward(qcs_mlp* n, const float* x, uint32_t batch, float* y) {
                 (apart && (hipEventRecord(n->up_ev, n->up) != hipSuccess ||
                            hipStreamWaitEvent(n->stream, n->up_ev, 0) != hipSuccess)))
                 return set_error(QCS_EDEVICE, "input upload failed");
-            if (const int e = mlp_rows(n, int(P), xd, nullptr, nullptr, false, n->out + p0)) return e;
+            if (const int e = mlp_rows(n, int(P), xd, nullptr, nullptr, 0, n->out + p0, nullptr)) return e;
         }
         if (hipMemcpyAsync(y + b0, n->out, sizeof(float) * B, hipMemcpyDeviceToHost, n->stream) != hipSuccess ||
             hipStreamSynchronize(n->stream) != hipSuccess)
@@ -1021,17 +1057,14 @@ int qcs_mlp_forward(qcs_mlp* n, const float* x, uint32_t batch, float* y) {
 int qcs_mlp_gradients(qcs_mlp* n, const float* x, const float* t, uint32_t batch, float* grad, float* loss) {
     if (!n || !x || !t || batch == 0) return set_error(QCS_EINVAL, "bad argument");
     const int B = int(batch);
-    int e = mlp_reserve(n, B, true);
-    if (e) return e;
+    if (const int e = mlp_reserve(n, B, std::min(B, n->slice), true)) return e;
     if (!grow(n->xin, n->xin_cap, size_t(B) * (n->in + 1)) || !grow(n->lsum, n->lsum_cap, size_t(4)))
         return set_error(QCS_ENOMEM, "mlp inputs");
     float* td = n->xin + size_t(B) * n->in;
     if (hipMemcpyAsync(n->xin, x, sizeof(float) * B * n->in, hipMemcpyHostToDevice, n->stream) != hipSuccess ||
         hipMemcpyAsync(td, t, sizeof(float) * B, hipMemcpyHostToDevice, n->stream) != hipSuccess)
         return set_error(QCS_EDEVICE, "input upload failed");
-    e = mlp_rows(n, B, n->xin, nullptr, td, true, n->out);
-    if (!e) e = mlp_dw(n, B, false, 0.f, n->lsum);
-    if (e) return e;
+    if (const int e = mlp_batch(n, B, n->xin, nullptr, td, false, 0.f, n->lsum)) return e;
     float l = 0;
     if ((grad && hipMemcpyAsync(grad, n->g, sizeof(float) * n->nparams, hipMemcpyDeviceToHost, n->stream) != hipSuccess) ||
         hipMemcpyAsync(&l, n->lsum, sizeof(float), hipMemcpyDeviceToHost, n->stream) != hipSuccess ||
@@ -1066,7 +1099,7 @@ int qcs_mlp_train(qcs_mlp* n, const float* X, const float* Y, uint64_t rows, uin
         hipMemcpy(n->dY, Y, sizeof(float) * rows, hipMemcpyHostToDevice) != hipSuccess)
         return set_error(QCS_EDEVICE, "dataset upload failed");
     const uint64_t steps = rows / batch;
-    if (const int e = mlp_reserve(n, int(batch), true)) return e;
+    if (const int e = mlp_reserve(n, int(batch), std::min(int(batch), n->slice), true)) return e;
     if (!grow(n->lsum, n->lsum_cap, size_t(std::max<uint64_t>(steps, 1)))) return set_error(QCS_ENOMEM, "loss buffer");
     std::vector<uint32_t> perm(rows);
     std::vector<float> losses(steps);
@@ -1079,9 +1112,7 @@ int qcs_mlp_train(qcs_mlp* n, const float* X, const float* Y, uint64_t rows, uin
             hipMemcpy(n->didx, perm.data(), sizeof(uint32_t) * rows, hipMemcpyHostToDevice) != hipSuccess)
             return set_error(QCS_EDEVICE, "index upload failed");
         for (uint64_t k = 0; k < steps; ++k) {
-            int e = mlp_rows(n, int(batch), n->dX, n->didx + k * batch, n->dY, true, n->out);
-            if (!e) e = mlp_dw(n, int(batch), true, lr, n->lsum + k);
-            if (e) return e;
+            if (const int e = mlp_batch(n, int(batch), n->dX, n->didx + k * batch, n->dY, true, lr, n->lsum + k)) return e;
         }
         if (loss_per_epoch) {
             if (steps && (hipMemcpyAsync(losses.data(), n->lsum, sizeof(float) * steps, hipMemcpyDeviceToHost,
