@@ -199,9 +199,9 @@ def gate_bytes(gate, n, amp=16):
 
 
 def gpu_circuit(n, layers, widths=(0, 4, 5, "auto")):
-    """The layered random circuit, unfused, fused to 4 and 5 qubits and at the
-    width the fusion autotuner picks; one run each after a warm-up on a
-    smaller circuit of the same kind."""
+    """The layered random circuit at fusion widths 0, 4, 5 and the one left to
+    the library (tile passes or dense blocks, whichever it takes to be faster);
+    one run each after a warm-up on a smaller circuit of the same kind."""
     from qcsim_amd import QubitRegister
 
     from qcsim_amd.tuning import apply_cache
@@ -426,8 +426,9 @@ def random_toffoli_circuit(n, layers, seed=13):
 
 
 def gpu_precision_fused_c64(n, layers, width=5):
-    """complex64 state running the fused circuit (FP32 MFMA blocks) beside an
-    FP64 GPU copy running it unfused; error of the former against the latter."""
+    """complex64 state running the circuit at a fusion width (at 32 qubits and
+    width 5 FP32 MFMA blocks; below 28 qubits tile passes) beside an FP64 GPU
+    copy running it at width 0; error of the former against the latter."""
     from qcsim_amd import QubitRegister
 
     from qcsim_amd.tuning import apply_cache

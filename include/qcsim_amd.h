@@ -111,14 +111,14 @@ int qcs_apply_dense(qcs_register* r, uint32_t k, const uint32_t* qubits,
                     const double* mat);
 
 /* A batch of gates in order, run in passes of many gates over the state.
- * fuse_width 0/1 takes the gates as they come (a refused
- * gate ends the batch after those before it); with 2..5 a list that the
- * fusion pass (qcs_fuse) refuses at that width is refused whole, and at 4
- * and 5 a large register applies a list whose gates keep to neighbourhoods in
- * that pass's dense blocks, where those take less time (complex128 from 25
- * qubits on; complex64, in FP32 then, from 28 on).
- * QCS_FUSE_AUTO leaves the width to the library. No counterpart in the
- * reference, which applies gates one by one (QubitRegister.h:488-492). */
+ * fuse_width 0/1 takes the gates as they come (a refused gate ends the batch
+ * after those before it); with 2..5 a list that the fusion pass (qcs_fuse)
+ * refuses at that width is refused whole, and at 4 and 5 a large register
+ * applies a list whose gates keep to neighbourhoods in that pass's dense
+ * blocks, where those take less time (complex128 from 25 qubits on; complex64,
+ * in FP32 then, from 28 on). QCS_FUSE_AUTO leaves the width to the library. No
+ * counterpart in the reference, which applies gates one by one
+ * (QubitRegister.h:488-492). */
 #define QCS_FUSE_AUTO 0xFFFFFFFFu
 int qcs_apply_circuit(qcs_register* r, const qcs_gate* gates, uint32_t n,
                       uint32_t fuse_width);
@@ -337,7 +337,8 @@ int qcs_mlp_train(qcs_mlp* n, const float* X, const float* Y, uint64_t rows, uin
  * algorithmic GB/s figures. */
 int qcs_autotune(qcs_register* r, uint32_t reps, double* gbps);
 int qcs_autotune_variants(void);
-/* The fusion cost table of QCS_FUSE_AUTO: times a generic 1-qubit gate and
+/* The fusion cost table, by which QCS_FUSE_AUTO reports a width where a list
+ * runs in passes: times a generic 1-qubit gate and
  * dense 2..5-qubit blocks (identity matrices: the state keeps its values)
  * on this register, mean over low, high and spread qubits, and keeps the
  * figures for its precision and qubit count. ms, if not NULL, receives 6

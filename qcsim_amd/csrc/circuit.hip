@@ -17,7 +17,6 @@
 // of two U(2)).
 // How a list is cut is in circuit_plan.cpp.
 #include <algorithm>
-#include <cstring>
 #include <vector>
 
 #include "circuit_plan.h"
