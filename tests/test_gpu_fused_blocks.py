@@ -79,6 +79,12 @@ def test_list_in_blocks_equals_passes(n, precision, kind, width, blocks):
         assert launches < len(seq) / 10
     largest, overlap = a.compare(b)
     na, nb = a.norm2(), b.norm2()
+    if blocks:  # a program of the list takes the same blocks
+        prog = b.compile_program(seq, fuse_width=width)
+        b.setToBasisState(5)
+        prog.run()
+        assert prog.launches() == count.value and a.compare(b)[0] == 0
+        prog.close()
     a.close()
     b.close()
     if precision == "c128":
