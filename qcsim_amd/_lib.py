@@ -134,6 +134,9 @@ def load(path: str = LIB_PATH) -> C.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    # ApplyGate's own, with the matrix as bytes: converted without a Python call
+    lib.apply_gate_bytes = fn = lib["qcs_apply_gate"]
+    fn.restype, fn.argtypes = _I, [*SIGNATURES["qcs_apply_gate"][1][:-1], C.c_char_p]
     return lib
 
 

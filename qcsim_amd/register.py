@@ -40,7 +40,12 @@ def _mat_bytes(m) -> bytes:
     """A matrix, or what converts to one, as the C-ABI reads it. A pointer
     argument takes bytes at a tenth of what numpy's ctypes interface costs (0.1
     against 1 us)."""
-    return m.tobytes() if getattr(m, "dtype", None) is _C128 else _mat_buf(m).tobytes()
+    try:
+        if m.dtype is _C128:
+            return m.tobytes()
+    except AttributeError:  # nested lists
+        pass
+    return _mat_buf(m).tobytes()
 
 
 def _mat_buf(m: np.ndarray) -> np.ndarray:
@@ -206,7 +211,7 @@ class QubitRegister:
             qubit, controllingQubit1, controllingQubit2 = gate.q1, gate.q2, gate.q3
         m = gate.getRawOperatorMatrix()
         check(
-            lib().qcs_apply_gate(
+            lib().apply_gate_bytes(
                 self._h,
                 gate.getQubitsNumber(),
                 gate.traits,
