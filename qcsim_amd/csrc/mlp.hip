@@ -878,10 +878,10 @@ static int mlp_dw(qcs_mlp* n, int B, bool more, int batch, bool adam, float lr, 
 // the order of its rows, so they do not depend on where it is cut.
 static int mlp_batch(qcs_mlp* n, int B, const float* X, const uint32_t* idx, const float* T, bool adam, float lr,
                      float* loss) {
-    for (int b0 = 0; b0 < B; b0 += n->slice) {
-        const int P = std::min(n->slice, B - b0);
-        const bool last = b0 + P == B;
-        int e = mlp_rows(n, P, idx ? X : X + size_t(b0) * n->in, idx ? idx + b0 : nullptr, idx ? T : T + b0, B, n->out + b0,
+    for (size_t b0 = 0; b0 < size_t(B); b0 += n->slice) {
+        const int P = int(std::min(size_t(n->slice), B - b0));
+        const bool last = b0 + P == size_t(B);
+        int e = mlp_rows(n, P, idx ? X : X + b0 * n->in, idx ? idx + b0 : nullptr, idx ? T : T + b0, B, n->out + b0,
                          n->lossv + b0);
         if (!e) e = mlp_dw(n, P, b0 > 0, B, adam && last, lr, last ? loss : nullptr);
         if (e) return e;
